@@ -187,6 +187,79 @@ hipError_t energy_scratch(int device, double** out);
 constexpr int32_t kEnergyMaxEntities = 0x7FFFFFFF - kEnergyMaxBlocks * 256;
 hipError_t launch_energy_f32(const EnergyArgs<float>& a, int nblocks, double* out, hipStream_t s);
 
+// ---------------------------------------------------------------- resident stepping
+// Many steps in one launch (rsg_resident.hip): the mesh is cut into tiles of cells, one
+// workgroup per tile, all of them on the GPU at once.  A tile holds the stresses of its cells
+// and the velocities of its nodes (every vertex of its cells) in LDS for the whole launch, and
+// each step reads from memory only the stresses of its halo: the other tiles' cells at its
+// nodes.
+constexpr int kResidentSlots = 4095;  // 12-bit local links: slot numbers stay at or below this
+
+// One tile: ranges of the plan's arrays.  The exported cells (in some other tile's halo) come
+// first among its cells, and the nodes whose 8 cells are all its own first among its nodes.
+struct ResidentTile {
+  int32_t cell0, ncell, nexp;  // cell records; how many of them are exported
+  int32_t node0, nnode, nown;  // node records; how many of them touch no halo cell
+  int32_t halo0, nhalo;        // halo entries
+  int32_t exp0;                // exchange slot of the tile's first exported cell
+  int32_t pad;
+};
+constexpr uint32_t kResidentOwner = 0x80000000u;  // node record: this tile writes the node's results
+
+constexpr int kFlagStride = 32;                   // a flag per 128-byte line
+// Source terms: the special nodes (cells) with the same lists of channel terms share a class, and
+// the host sums each class's terms once per step, 3 (6) values a class: a row of 3 * node classes
+// + 6 * cell classes doubles.  Class numbers stay below 128.
+constexpr int kResidentForces = 256;  // largest row
+constexpr uint8_t kResidentSensor = 0x80;  // node mark: a sensor this tile records
+
+template <typename T>
+struct ResidentArgs {
+  VelocityArgs<T> v;  // state, coefficients, sources and sensors as the per-step kernels take them
+  StressArgs<T> s;    // (amp and trace: the first step's)
+  const ResidentTile* tiles;
+  const uint32_t* crec;  // [cells][4]: 8 x 12-bit local node indices, internal cell id
+  const uint32_t* nrec;  // [tile nodes][4]: 8 x 12-bit local cell slots (own cells, halo, then the
+                         // zero slot of missing cells), internal node id | kResidentOwner
+  const int2* halo;      // exchange slot and tile of each halo cell
+  const int32_t* hcell;  // internal id of each halo cell
+  unsigned long long* xbuf;  // [2][6 * sizeof(T) / 8][nexp]: exported stresses of even and odd steps
+  uint32_t* flag;        // [tiles][kFlagStride]: the step whose exported stresses are written
+  int32_t* status;       // set when a wait ran out
+  uint32_t epoch;        // the state's step, counted over the resident launches
+  int32_t nsteps;        // >= 2
+  int32_t ntiles;
+  int32_t nexp;
+  int32_t max_set;       // largest number of slots of a tile, without the zero slot
+  int32_t max_node;
+  int32_t max_cell;
+  uint32_t* work;        // [tiles][max_node + max_cell][4] when the records do not fit LDS, else null
+  const double* force;   // [nsteps][nforce] summed source terms
+  int32_t nforce;
+  const uint8_t* ncls;   // class of each special node, 0 .. node classes - 1
+  const uint8_t* ccls;   // class of each special cell
+  int32_t cforce0;       // first cell value of a force row
+  int32_t row;           // doubles from one step's trace row to the next's
+};
+
+// LDS of a tile's workgroup: its slots' stresses, its nodes' velocities, the marks and, with
+// `records`, the records; without, the kernel keeps those in `work`.
+inline size_t resident_lds_bytes(int max_set, int max_node, int max_cell, size_t elt, bool records) {
+  const size_t state = ((size_t)6 * (max_set + 1) + (size_t)3 * max_node) * elt;
+  return (state + 15) / 16 * 16 + (size_t)(records ? 17 : 1) * (max_node + max_cell);
+}
+constexpr size_t kResidentStaticLds = 2 * kResidentForces * 8 + 64;  // and what it declares itself
+
+// The launchers live in the kernel library only: builds of the host code without it step with
+// the per-step kernels.
+#define RSG_WEAK __attribute__((weak))
+// Compute units of the current device (1 without cooperative launches), and LDS bytes a
+// workgroup may take.
+RSG_WEAK hipError_t resident_limits(int* cus, size_t* lds);
+// threads: 256, 512 or 1024 per workgroup.
+RSG_WEAK hipError_t launch_resident_f64(const ResidentArgs<double>& a, int threads, hipStream_t s);
+RSG_WEAK hipError_t launch_resident_f32(const ResidentArgs<float>& a, int threads, hipStream_t s);
+
 // NaN boxing of a special-table index.
 inline double box_f64(int32_t idx) {
   uint64_t b = 0x7FF8000000000000ull | (uint64_t)(uint32_t)idx;

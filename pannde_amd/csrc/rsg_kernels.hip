@@ -26,7 +26,7 @@
 
 #include <type_traits>
 
-#include "rsg_internal.h"
+#include "rsg_device.h"
 
 // Occupancy hints (minimum waves per SIMD, 0 = compiler default).
 // Largest workgroup the gather kernels accept.  It bounds the registers the compiler may
@@ -86,44 +86,6 @@ __device__ __forceinline__ int xcd_block(int bid, int nb) {
   return x * q + (x < r ? x : r) + j;
 }
 
-__device__ __forceinline__ bool is_boxed(double v) { return __builtin_isnan(v); }
-__device__ __forceinline__ bool is_boxed(float v) { return __builtin_isnan(v); }
-__device__ __forceinline__ int unbox(double v) {
-  return (int)(uint32_t)(__double_as_longlong(v) & 0xFFFFFFFFll);
-}
-__device__ __forceinline__ int unbox(float v) { return (int)(__float_as_uint(v) & 0x3FFFFFu); }
-
-// RightHex slot patterns: forward and backward vertices (or cell slots) per axis.
-//   x: fwd {1,2,5,6} bwd {0,3,4,7};  y: fwd {2,3,6,7} bwd {0,1,4,5};
-//   z: fwd {4,5,6,7} bwd {0,1,2,3}
-template <int AX>
-__device__ __forceinline__ double diffsum(const double (&f)[8]) {
-  double v = 0.0;
-  if (AX == 0) {
-    v += (f[1] - f[0]); v += (f[2] - f[3]); v += (f[5] - f[4]); v += (f[6] - f[7]);
-  } else if (AX == 1) {
-    v += (f[2] - f[0]); v += (f[3] - f[1]); v += (f[6] - f[4]); v += (f[7] - f[5]);
-  } else {
-    v += (f[4] - f[0]); v += (f[5] - f[1]); v += (f[6] - f[2]); v += (f[7] - f[3]);
-  }
-  return v;
-}
-template <int AX>
-__device__ __forceinline__ float diffsum(const float (&f)[8]) {
-  float v;
-  if (AX == 0) {
-    v = ((f[1] - f[0]) + (f[2] - f[3])) + ((f[5] - f[4]) + (f[6] - f[7]));
-  } else if (AX == 1) {
-    v = ((f[2] - f[0]) + (f[3] - f[1])) + ((f[6] - f[4]) + (f[7] - f[5]));
-  } else {
-    v = ((f[4] - f[0]) + (f[5] - f[1])) + ((f[6] - f[2]) + (f[7] - f[3]));
-  }
-  return v;
-}
-// Derivative from a difference sum: FP64 (value*0.25)/spacing, FP32 value*(0.25/spacing).
-__device__ __forceinline__ double dscale(double v, double sp) { return v * 0.25 / sp; }
-__device__ __forceinline__ float dscale(float v, float inv) { return v * inv; }
-
 // Cells around a node: a missing cell (-1) contributes zero.  LDS-staged gathers need no
 // test, because their missing links point at a staged entry that holds zero.
 template <bool DIRECT, typename T>
@@ -152,36 +114,6 @@ __device__ __forceinline__ void load8_nodes(const T* __restrict__ f, const int (
 }
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef double d2v __attribute__((ext_vector_type(2)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-// One material row (16-byte aligned) as 16-byte loads through the caches: lanes of a
-// wavefront that share a material read the same addresses, which coalesce.
-template <int W>
-__device__ __forceinline__ void load_row(const double* __restrict__ p, double (&out)[W]) {
-  static_assert(W % 2 == 0, "row width");
-  const d2v* q = reinterpret_cast<const d2v*>(p);
-#pragma unroll
-  for (int i = 0; i < W / 2; i++) {
-    const d2v v = q[i];
-    out[2 * i] = v.x;
-    out[2 * i + 1] = v.y;
-  }
-}
-template <int W>
-__device__ __forceinline__ void load_row(const float* __restrict__ p, float (&out)[W]) {
-  static_assert(W % 4 == 0, "row width");
-  const f4v* q = reinterpret_cast<const f4v*>(p);
-#pragma unroll
-  for (int i = 0; i < W / 4; i++) {
-    const f4v v = q[i];
-    out[4 * i] = v.x;
-    out[4 * i + 1] = v.y;
-    out[4 * i + 2] = v.z;
-    out[4 * i + 3] = v.w;
-  }
-}
-
 // Coefficient form of a kernel instance: KM = 0 per-entity arrays, 1 class-table keys,
 // 3 keys packed with the LDS links (a batch launches each form for its own members).
 template <int KM, typename A>
@@ -191,31 +123,6 @@ __device__ __forceinline__ constexpr bool packed(const A&) {
 template <int KM, typename A>
 __device__ __forceinline__ constexpr bool keyed(const A&) {
   return KM == 1 || KM == 3;
-}
-
-// Material/spacing key of an entity, and its special index (or -1).
-template <typename A>
-__device__ __forceinline__ uint32_t resolve_key(const A& a, uint32_t key, int& sp) {
-  if (key & kSpecialKey) {
-    sp = (int)(key & ~kSpecialKey);
-    return a.sp_key[sp];
-  }
-  sp = -1;
-  return key;
-}
-template <typename P, typename T>
-__device__ __forceinline__ void axis_spacings(P axis, uint32_t k, T& sx, T& sy, T& sz) {
-  sx = axis[(k >> 14) & (kAxisClasses - 1)];
-  sy = axis[kAxisClasses + ((k >> 7) & (kAxisClasses - 1))];
-  sz = axis[2 * kAxisClasses + (k & (kAxisClasses - 1))];
-}
-
-// The class tables are written only by the host, so a wavefront-uniform read of them may go
-// through the scalar cache: a pointer in the constant address space lets the compiler use
-// scalar loads (reads only; nothing is ever stored through this path).
-template <typename T>
-__device__ __forceinline__ const __attribute__((address_space(4))) T* as_const(const T* p) {
-  return (const __attribute__((address_space(4))) T*)p;
 }
 
 // 8 x int32 of one entity as two 16-byte loads; read once per step, so non-temporal.
@@ -417,61 +324,24 @@ __device__ __forceinline__ void velocity_apply(const VelocityArgs<T>& a, int n, 
       idt = a.sp_idt[sp];
     }
   }
-  T dx_sxx, dx_sxy, dy_sxy, dx_sxz, dz_sxz, dy_syy, dy_syz, dz_syz, dz_szz;
+  T r[3];
   if constexpr (LDS && RSG_VELOCITY_PAIRS) {
     // S0, S1, S2 are the staged pair rows (Sxx, Sxy), (Sxz, Syy), (Syz, Szz)
-    T f[8], g[8];
-    load8_pairs(S0, in.c, f, g);
-    dx_sxx = dscale(diffsum<0>(f), sx);
-    dx_sxy = dscale(diffsum<0>(g), sx);
-    dy_sxy = dscale(diffsum<1>(g), sy);
-    load8_pairs(S1, in.c, f, g);
-    dx_sxz = dscale(diffsum<0>(f), sx);
-    dz_sxz = dscale(diffsum<2>(f), sz);
-    dy_syy = dscale(diffsum<1>(g), sy);
-    load8_pairs(S2, in.c, f, g);
-    dy_syz = dscale(diffsum<1>(f), sy);
-    dz_syz = dscale(diffsum<2>(f), sz);
-    dz_szz = dscale(diffsum<2>(g), sz);
+    node_rates([&](int p, T(&f)[8], T(&g)[8]) { load8_pairs(p == 0 ? S0 : p == 1 ? S1 : S2, in.c, f, g); }, sx, sy,
+               sz, r);
   } else {
-    T f[8];
-    load8_cells<!LDS>(S0, in.c, f);
-    dx_sxx = dscale(diffsum<0>(f), sx);
-    load8_cells<!LDS>(S5, in.c, f);
-    dx_sxy = dscale(diffsum<0>(f), sx);
-    dy_sxy = dscale(diffsum<1>(f), sy);
-    load8_cells<!LDS>(S4, in.c, f);
-    dx_sxz = dscale(diffsum<0>(f), sx);
-    dz_sxz = dscale(diffsum<2>(f), sz);
-    load8_cells<!LDS>(S1, in.c, f);
-    dy_syy = dscale(diffsum<1>(f), sy);
-    load8_cells<!LDS>(S3, in.c, f);
-    dy_syz = dscale(diffsum<1>(f), sy);
-    dz_syz = dscale(diffsum<2>(f), sz);
-    load8_cells<!LDS>(S2, in.c, f);
-    dz_szz = dscale(diffsum<2>(f), sz);
+    const T* const S[6] = {S0, S5, S4, S1, S3, S2};  // in the order of the pairs
+    node_rates(
+        [&](int p, T(&f)[8], T(&g)[8]) {
+          load8_cells<!LDS>(S[2 * p], in.c, f);
+          load8_cells<!LDS>(S[2 * p + 1], in.c, g);
+        },
+        sx, sy, sz, r);
   }
-
-  T r0 = (dx_sxx + dy_sxy) + dz_sxz;
-  T r1 = (dx_sxy + dy_syy) + dz_syz;
-  T r2 = (dx_sxz + dy_syz) + dz_szz;
-
-  if (sp >= 0) {
-    const int* off = a.sp_off + 4 * (size_t)sp;
-    double fsum[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-      double acc = 0.0;
-      for (int t = off[d]; t < off[d + 1]; t++) acc += a.amp[a.term[t]];
-      fsum[d] = acc;
-    }
-    r0 = r0 + (T)fsum[0];
-    r1 = r1 + (T)fsum[1];
-    r2 = r2 + (T)fsum[2];
-  }
-  const T v0 = in.v0 + idt * r0;
-  const T v1 = in.v1 + idt * r1;
-  const T v2 = in.v2 + idt * r2;
+  if (sp >= 0) add_node_forces(a, sp, r);
+  const T v0 = in.v0 + idt * r[0];
+  const T v1 = in.v1 + idt * r[1];
+  const T v2 = in.v2 + idt * r[2];
   a.V0[n] = v0;
   a.V1[n] = v1;
   a.V2[n] = v2;
@@ -546,11 +416,6 @@ __device__ __forceinline__ T cload(const T* __restrict__ C, int64_t ldc, int j, 
   return STREAM_LOAD(C + idx);
 }
 
-// Index of C_(I,J) (0-based Voigt indices) in the 21-entry upper triangle.
-__host__ __device__ constexpr int tri(int i, int j) {
-  return (i <= j) ? (i * 6 - i * (i - 1) / 2 + (j - i)) : (j * 6 - j * (j - 1) / 2 + (i - j));
-}
-
 // Per-cell operands of the stress update that do not depend on a gather: links,
 // spacings, the 21 C_IJ and the 6 stresses.
 template <typename T>
@@ -593,97 +458,21 @@ __device__ __forceinline__ void stress_load(const StressArgs<T>& a, int e, StrIn
   in.s[5] = a.S5[e];
 }
 
-// S += dt*(C : grad V + m) for one cell from its strain-rate terms; cc(j) is the j-th of
-// the 21 stored C (a class-table row or the cell's own array).
-template <typename T, typename R>
-__device__ __forceinline__ void voigt_update(T dt, R cc, T d00, T d11, T d22, T e12, T e02, T e01,
-                                             const double (&m)[6], int sp, T (&s)[6]) {
-#pragma unroll
-  for (int ks = 0; ks < 6; ks++) {
-    T acc = cc[tri(ks, 0)] * d00 + cc[tri(ks, 1)] * d11 + cc[tri(ks, 2)] * d22 +
-            cc[tri(ks, 3)] * e12 + cc[tri(ks, 4)] * e02 + cc[tri(ks, 5)] * e01;
-    if constexpr (sizeof(T) == 8) {
-      if (sp >= 0) acc = acc + (T)m[ks];
-      s[ks] = s[ks] + dt * acc;  // C is plain C_IJ: S += dt*(C:gradV + m)
-    } else {
-      if (sp >= 0) acc = acc + (T)((double)dt * m[ks]);  // C holds dt*C_IJ
-      s[ks] = s[ks] + acc;
-    }
-  }
-}
-
-// Strain-rate terms of one cell from its 8 vertices: the diagonal D_i V_i and the shear
-// sums D_j V_k + D_k V_j, in the reference's order of operations.
-// With PAIRS, V0 is the staged row of (Vx, Vy) pairs and V1 is unused.
+// The strain-rate terms of one cell; with PAIRS, V0 is the staged row of (Vx, Vy) pairs and V1
+// is unused.
 template <typename T, bool PAIRS = false>
 __device__ __forceinline__ void strain_terms(const T* V0, const T* V1, const T* V2, const int (&c)[8], T sx,
                                              T sy, T sz, T (&d)[6]) {
-  // delV[i][k] = D_i V_k (i: derivative axis, k: velocity component)
-  T f[8];
-  T d00, d10, d20, d01, d11, d21;
-  if constexpr (PAIRS) {
-    T g[8];
-    load8_pairs(V0, c, f, g);
-    d00 = dscale(diffsum<0>(f), sx);
-    d10 = dscale(diffsum<1>(f), sy);
-    d20 = dscale(diffsum<2>(f), sz);
-    d01 = dscale(diffsum<0>(g), sx);
-    d11 = dscale(diffsum<1>(g), sy);
-    d21 = dscale(diffsum<2>(g), sz);
-  } else {
-    load8_nodes(V0, c, f);
-    d00 = dscale(diffsum<0>(f), sx);
-    d10 = dscale(diffsum<1>(f), sy);
-    d20 = dscale(diffsum<2>(f), sz);
-    load8_nodes(V1, c, f);
-    d01 = dscale(diffsum<0>(f), sx);
-    d11 = dscale(diffsum<1>(f), sy);
-    d21 = dscale(diffsum<2>(f), sz);
-  }
-  load8_nodes(V2, c, f);
-  const T d02 = dscale(diffsum<0>(f), sx);
-  const T d12 = dscale(diffsum<1>(f), sy);
-  const T d22 = dscale(diffsum<2>(f), sz);
-  d[0] = d00;
-  d[1] = d11;
-  d[2] = d22;
-  d[3] = d12 + d21;
-  d[4] = d02 + d20;
-  d[5] = d01 + d10;
-}
-
-// Summed moment terms of a special cell, per Voigt component.
-template <typename T>
-__device__ __forceinline__ void cell_moments(const StressArgs<T>& a, int sp, double (&m)[6]) {
-#pragma unroll
-  for (int k = 0; k < 6; k++) m[k] = 0.0;
-  if (sp < 0) return;
-  const int* off = a.sp_off + 7 * (size_t)sp;
-#pragma unroll
-  for (int k = 0; k < 6; k++) {
-    double acc = 0.0;
-    for (int t = off[k]; t < off[k + 1]; t++) acc += a.amp[a.term[t]];
-    m[k] = acc;
-  }
-}
-
-// S += dt*(C : grad V + m) for one cell; cc[j] is the j-th of the 21 stored C (a class-table
-// row or the cell's own array).
-template <typename T, typename R>
-__device__ __forceinline__ void voigt_update(T dt, R cc, const T (&d)[6], const double (&m)[6], int sp,
-                                             T (&s)[6]) {
-#pragma unroll
-  for (int ks = 0; ks < 6; ks++) {
-    T acc = cc[tri(ks, 0)] * d[0] + cc[tri(ks, 1)] * d[1] + cc[tri(ks, 2)] * d[2] +
-            cc[tri(ks, 3)] * d[3] + cc[tri(ks, 4)] * d[4] + cc[tri(ks, 5)] * d[5];
-    if constexpr (sizeof(T) == 8) {
-      if (sp >= 0) acc = acc + (T)m[ks];
-      s[ks] = s[ks] + dt * acc;  // C is plain C_IJ: S += dt*(C:gradV + m)
-    } else {
-      if (sp >= 0) acc = acc + (T)((double)dt * m[ks]);  // C holds dt*C_IJ
-      s[ks] = s[ks] + acc;
-    }
-  }
+  strain_rates(
+      [&](T(&f)[8], T(&g)[8]) {
+        if constexpr (PAIRS) {
+          load8_pairs(V0, c, f, g);
+        } else {
+          load8_nodes(V0, c, f);
+          load8_nodes(V1, c, g);
+        }
+      },
+      [&](T(&f)[8]) { load8_nodes(V2, c, f); }, sx, sy, sz, d);
 }
 
 // S += dt*(C : grad V + m) at cell e, V gathered from V0..V2 (LDS or HBM; with PAIRS, V0 is

@@ -1,0 +1,129 @@
+"""Resident stepping (rsg_resident.hip): many steps of a mesh in one launch, its tiles in LDS.
+
+On the CPU the set-up's plan is walked by a stand-in for the kernel (tests/sanitize/
+resident_stub.cpp), tile by tile with every index checked, and the result compared bit for bit
+with the oracle.  On the GPU the kernel is compared bit for bit with the per-step kernels (a
+handle whose tuning names a workgroup size uses those) and with the oracle."""
+import os
+import shutil
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from conftest import load_golden
+from oracle import oracle_rsg as orc
+from pannde_amd import cases, rsg
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def jobs(name):
+    if name == "one_cell":
+        return cases.al_block(seed=1, nx=1, ny=1, nz=1, nsteps=9, n_sensors=2)
+    if name == "one_tile":  # 500 cells: the most that one tile takes
+        return cases.al_block(seed=2, nx=10, ny=10, nz=5, nsteps=13, n_sensors=200)
+    if name == "two_tiles":
+        return cases.water_column_block(seed=3, nx=8, ny=9, nz=7, nsteps=11)
+    if name == "flat":
+        return cases.al_block(seed=4, nx=61, ny=47, nz=1, nsteps=9, n_sensors=7)
+    if name == "cracked_plate":
+        return cases.cfrp_plate(seed=3, nx=40, ny=36, cells_per_ply=1, nsteps=12, n_holes=2, renumber=True,
+                                crack=cases.Crack((1e-3, 0.9e-3, 16 * 5e-5), 30.0, 0.8e-3, 4e-4))
+    if name == "bracket":
+        return cases.ti_bracket(seed=7, leg=48, width=12, height=9, nsteps=11)
+    if name == "moments":
+        return cases.water_column_block(seed=9, nx=23, ny=14, nz=17, nsteps=9)
+    if name == "rest":  # sensors, no source
+        case = cases.al_block(seed=5, nx=12, ny=11, nz=9, nsteps=8, n_sensors=5)
+        case.force = []
+        return case
+    return load_golden(name)[0]
+
+
+NAMES = ("one_cell", "one_tile", "two_tiles", "flat", "cracked_plate", "bracket", "moments", "rest",
+         "water_column_nodec", "three_transducers")
+
+SCRIPT = r'''
+import sys
+import numpy as np
+sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+import test_resident
+from oracle import oracle_rsg as orc
+from pannde_amd import rsg
+for name in test_resident.NAMES:
+    case = test_resident.jobs(name)
+    V0, S0, t0, tr0 = orc.run_oracle(case)
+    for tuning in (None, dict(coeff_classes=-1), dict(coeff_classes=-1, c_layout=-1)):
+        s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64, tuning=tuning)
+        s.solve(case.nsteps)
+        V, S = s.get_state()
+        tr = s.traces()
+        s.close()
+        assert np.array_equal(V, V0) and np.array_equal(S, S0) and np.array_equal(tr, tr0), (name, tuning)
+        f = rsg.DeviceSolver.from_case(case, rsg.RSG_FP32, tuning=tuning)
+        f.solve(case.nsteps)
+        # FP32 fields after a few steps: a few roundings of 2^-24 each against FP64
+        err = np.abs(f.get_state()[0] - V0).max() / max(np.abs(V0).max(), 1e-300)
+        assert err < 1e-5, (name, tuning, err)
+        f.close()
+print("ok")
+'''
+
+
+@pytest.mark.skipif(shutil.which("g++") is None or not os.path.exists("/opt/rocm/include/hip/hip_runtime_api.h"),
+                    reason="needs g++ and the HIP headers")
+@pytest.mark.timeout(600)
+def test_plan_steps_as_the_oracle(tmp_path):
+    lib = str(tmp_path / "libstub.so")
+    here = os.path.join(ROOT, "tests", "sanitize")
+    cmd = ["g++", "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
+           "-I/opt/rocm/include", os.path.join(ROOT, "pannde_amd", "csrc", "rsg_host.cpp"),
+           os.path.join(here, "hip_host_stub.cpp"), os.path.join(here, "resident_stub.cpp"), "-o", lib, "-lpthread"]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-4000:]
+    # 256 compute units, and 24: larger tiles (the plate: 900 cells each)
+    for cus in ("256", "24"):
+        env = dict(os.environ, PANNDE_RSG_LIB=lib, RESIDENT_CUS=cus)
+        r = subprocess.run([sys.executable, "-c", SCRIPT, ROOT], stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                           text=True, timeout=500, env=env)
+        assert r.returncode == 0 and r.stdout.strip().endswith("ok"), (cus, r.stdout[-4000:])
+
+
+def run(case, precision, tuning, chunks):
+    s = rsg.DeviceSolver.from_case(case, precision, tuning=tuning)
+    for n in chunks:
+        s.solve(n)
+    out = s.get_state() + (s.traces(), s.time)
+    s.close()
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [rsg.RSG_FP64, rsg.RSG_FP32])
+@pytest.mark.parametrize("name", NAMES)
+def test_resident_equals_per_step_kernels(name, precision):
+    """Also split into calls of few and many steps, so that resident and per-step launches (and their
+    amplitude windows) follow each other, and with per-entity coefficients."""
+    case = jobs(name)
+    case.nsteps = 40
+    ref = run(case, precision, dict(block_velocity=256, block_stress=256), [40])
+    if precision == rsg.RSG_FP64:
+        V0, S0, t0, tr0 = orc.run_oracle(case)
+        assert all(np.array_equal(a, b) for a, b in zip(ref, (V0, S0, tr0))) and ref[3] == t0
+    for chunks in ([40], [7, 1, 13, 2, 17]):
+        for tuning in (None, dict(coeff_classes=-1)):
+            got = run(case, precision, tuning, chunks)
+            assert all(np.array_equal(a, b) for a, b in zip(got, ref)), (chunks, tuning)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,dims", [(rsg.RSG_FP64, (64, 52, 41)), (rsg.RSG_FP64, (80, 71, 57)),
+                                            (rsg.RSG_FP32, (80, 71, 57)), (rsg.RSG_FP32, (97, 83, 66))])
+def test_resident_at_its_largest(precision, dims):
+    """Tiles whose records are in LDS and tiles whose are not, up to the last sizes that fit."""
+    case = cases.al_block(seed=6, nx=dims[0], ny=dims[1], nz=dims[2], nsteps=300, n_sensors=9)
+    ref = run(case, precision, dict(block_velocity=256, block_stress=256), [300])
+    got = run(case, precision, None, [300])
+    assert all(np.array_equal(a, b) for a, b in zip(got, ref))
