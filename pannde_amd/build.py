@@ -40,8 +40,8 @@ def build(verbose=False):
     for part in (1, 2, 3, 4):
         jobs.append([HIPCC] + DEVICE_FLAGS + ["-DRSG_PART=%d" % part, "-c", os.path.join(CSRC, "rsg_kernels.hip"),
                                               "-o", os.path.join(bdir, "rsg_kernels_part%d.o" % part)])
-    # the energy reduction and the resident multi-step kernel
-    for name in ("rsg_energy", "rsg_resident"):
+    # the energy reduction, the resident multi-step kernel and the state transfers
+    for name in ("rsg_energy", "rsg_resident", "rsg_state"):
         jobs.append([HIPCC] + DEVICE_FLAGS + ["-c", os.path.join(CSRC, name + ".hip"), "-o",
                                               os.path.join(bdir, name + ".o")])
     objs = [cmd[-1] for cmd in jobs]

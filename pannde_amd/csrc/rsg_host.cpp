@@ -34,6 +34,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <unordered_map>
@@ -324,6 +325,13 @@ struct rsg_instance {
   void* res_flag = nullptr;
   uint32_t res_epoch = 0;         // steps taken by resident launches
 
+  // state transfers: the caller -> internal maps on the device (from the first transfer on) and
+  // each transfer thread's chunk of pinned memory
+  void* node_at_d = nullptr;
+  void* cell_at_d = nullptr;
+  std::vector<void*> chunk;
+  std::vector<hipEvent_t> chunk_ev;
+
   // source / sensor tables
   std::vector<Channel> channels;
   std::vector<int32_t> sensors;
@@ -413,6 +421,10 @@ struct rsg_instance {
       if (stage_ev[i]) (void)hipEventDestroy(stage_ev[i]);
     }
     if (res_status) (void)hipHostFree(res_status);
+    for (void* c : chunk)
+      if (c) (void)hipHostFree(c);
+    for (hipEvent_t e : chunk_ev)
+      if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : tev) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -479,19 +491,21 @@ template <typename F>
 void parallel_tasks(int t, F&& fn) {
   std::vector<std::exception_ptr> errs((size_t)t);
   std::vector<std::thread> workers;
-  for (int w = 1; w < t; w++)
-    workers.emplace_back([&fn, &errs, w]() {
-      try {
-        fn(w);
-      } catch (...) {
-        errs[w] = std::current_exception();
-      }
-    });
+  workers.reserve((size_t)t);
+  auto task = [&fn, &errs](int w) {
+    try {
+      fn(w);
+    } catch (...) {
+      errs[w] = std::current_exception();
+    }
+  };
+  int started = 1;
   try {
-    fn(0);
-  } catch (...) {
-    errs[0] = std::current_exception();
+    for (; started < t; started++) workers.emplace_back(task, started);
+  } catch (const std::system_error&) {  // no thread to be had: the caller takes the rest
   }
+  task(0);
+  for (int w = started; w < t; w++) task(w);
   for (auto& w : workers) w.join();
   for (auto& e : errs)
     if (e) std::rethrow_exception(e);
@@ -1559,6 +1573,126 @@ int energy_on_stream(rsg_instance* h, double* work, double* kinetic, double* str
   return RSG_OK;
 }
 
+// The state as host arrays through whole-array copies, reordered here: for builds of the host
+// code without the kernels of rsg_state.hip.
+int transfer_state_on_host(rsg_instance* h, double* V, double* S, bool write) {
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  const size_t e = h->elt();
+  std::vector<char> buf((size_t)std::max(h->nn, h->nc) * e);
+  auto move = [&](void* dev, int32_t n, const std::vector<int32_t>& of, double* host) -> int {
+    auto each = [&](auto* b) {
+      using T = std::remove_reference_t<decltype(*b)>;
+      for (int32_t i = 0; i < n; i++)
+        if (write)
+          b[i] = (T)host[of[i]];
+        else
+          host[of[i]] = (double)b[i];
+    };
+    auto convert = [&]() { e == 8 ? each((double*)buf.data()) : each((float*)buf.data()); };
+    if (write) convert();
+    HIP_TRY(copy_on(write ? dev : buf.data(), write ? buf.data() : dev, (size_t)n * e,
+                    write ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, h->stream));
+    if (!write) convert();
+    return RSG_OK;
+  };
+  int rc;
+  if (V)
+    for (int d = 0; d < 3; d++)
+      if ((rc = move(h->V[d], h->nn, h->node_of, V + (size_t)d * h->nn))) return rc;
+  if (S)
+    for (int s = 0; s < 6; s++)
+      if ((rc = move(h->S[s], h->nc, h->cell_of, S + (size_t)s * h->nc))) return rc;
+  return RSG_OK;
+}
+
+// The state to or from the caller's arrays (either may be null), in chunks: a kernel moves each
+// between the state and pinned memory, reordered, and a host thread copies it.  A state of more
+// than 128 Ki values takes up to setup_threads() threads, each with a chunk of its own, so
+// launches, bus and host copies overlap (one thread's copy of fresh pages is far below the bus).
+template <typename T>
+int transfer_chunks(rsg_instance* h, double* V, double* S, bool write) {
+  const int64_t nv = (int64_t)3 * h->nn, g0 = V ? 0 : nv, g1 = S ? nv + (int64_t)6 * h->nc : nv;
+  const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
+  const int threads = (int)std::max<int64_t>(1, std::min<int64_t>({(g1 - g0) >> 17, setup_threads(), hw}));
+  const int64_t size = std::min<int64_t>(rsg::kStateChunk, (g1 - g0 + threads - 1) / threads);
+  const int64_t chunks = (g1 - g0 + size - 1) / size;
+  if ((int)h->chunk.size() < threads) {
+    h->chunk.resize(threads, nullptr);
+    h->chunk_ev.resize(threads, nullptr);
+  }
+  rsg::StateArgs<T> a;
+  for (int d = 0; d < 3; d++) a.V[d] = (T*)h->V[d];
+  for (int s = 0; s < 6; s++) a.S[s] = (T*)h->S[s];
+  a.node_at = (const int32_t*)h->node_at_d;
+  a.cell_at = (const int32_t*)h->cell_at_d;
+  a.nn = h->nn;
+  a.nc = h->nc;
+  // values [g, g + n) between a chunk and the caller's arrays
+  auto copy = [&](int64_t g, int n, T* c) {
+    for (int64_t at = g; at < g + n;) {
+      const int64_t end = at < nv ? std::min<int64_t>(nv, g + n) : g + n;
+      double* user = at < nv ? V + at : S + (at - nv);
+      T* x = c + (at - g);
+      if (write)
+        for (int64_t i = 0; i < end - at; i++) x[i] = (T)user[i];
+      else
+        for (int64_t i = 0; i < end - at; i++) user[i] = (double)x[i];
+      at = end;
+    }
+  };
+  auto work = [&](int w) -> int {
+    if (w > 0) HIP_TRY(hipSetDevice(h->device));
+    if (!h->chunk[w]) {
+      // sized for this handle's largest transfer
+      const size_t most = std::min<int64_t>(rsg::kStateChunk, nv + (int64_t)6 * h->nc) * sizeof(T);
+      HIP_TRY(hipHostMalloc(&h->chunk[w], most, hipHostMallocDefault));
+    }
+    if (!h->chunk_ev[w]) HIP_TRY(hipEventCreateWithFlags(&h->chunk_ev[w], hipEventDisableTiming));
+    T* c = (T*)h->chunk[w];
+    for (int64_t k = w; k < chunks; k += threads) {
+      const int64_t g = g0 + k * size;
+      const int n = (int)std::min<int64_t>(size, g1 - g);
+      if (write) copy(g, n, c);
+      if constexpr (sizeof(T) == 8)
+        HIP_TRY(rsg::launch_state_f64(a, g, n, c, write, h->stream));
+      else
+        HIP_TRY(rsg::launch_state_f32(a, g, n, c, write, h->stream));
+      HIP_TRY(hipEventRecord(h->chunk_ev[w], h->stream));
+      HIP_TRY(hipEventSynchronize(h->chunk_ev[w]));  // the chunk is the thread's again
+      if (!write) copy(g, n, c);
+    }
+    return RSG_OK;
+  };
+  std::vector<int> rcs((size_t)threads, RSG_OK);
+  std::vector<std::string> errs((size_t)threads);
+  parallel_tasks(threads, [&](int w) {
+    rcs[w] = work(w);
+    if (rcs[w]) errs[w] = g_last_error;
+  });
+  for (int w = 0; w < threads; w++)
+    if (rcs[w]) {
+      g_last_error = errs[w];
+      return rcs[w];
+    }
+  return RSG_OK;
+}
+
+int transfer_state(rsg_instance* h, double* V, double* S, bool write) {
+  if (!V && !S) return RSG_OK;
+  try {
+    if (!rsg::launch_state_f64) return transfer_state_on_host(h, V, S, write);
+    int rc;
+    if (!h->node_at_d) {
+      if (!h->cell_at_d && (rc = upload(h, &h->cell_at_d, std::vector<int32_t>(h->cell_at)))) return rc;
+      if ((rc = upload(h, &h->node_at_d, std::vector<int32_t>(h->node_at)))) return rc;
+      if ((rc = finish_uploads(h))) return rc;
+    }
+    return h->precision == RSG_FP64 ? transfer_chunks<double>(h, V, S, write) : transfer_chunks<float>(h, V, S, write);
+  } catch (const std::bad_alloc&) {
+    return fail(RSG_ERR_NOMEM, "host allocation failed");
+  }
+}
+
 int check_mesh(const rsg_mesh_desc* m) {
   if (!m) return fail(RSG_ERR_ARG, "mesh is null");
   if (m->n_nodes <= 0 || m->n_cells <= 0)
@@ -2308,57 +2442,15 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
 int rsg_get_state(rsg_handle h, double* V, double* S) {
   Range range_("rsg_get_state");
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
-  HIP_TRY(hipStreamSynchronize(h->stream));
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
-  if (int rc = check_resident(h)) return rc;
-  const size_t e = h->elt();
-  std::vector<char> buf((size_t)std::max(h->nn, h->nc) * e);
-  auto fetch = [&](void* src, int32_t n, const std::vector<int32_t>& of, double* dst) -> int {
-    HIP_TRY(copy_on(buf.data(), src, (size_t)n * e, hipMemcpyDeviceToHost, h->stream));
-    if (e == 8) {
-      const double* b = (const double*)buf.data();
-      for (int32_t i = 0; i < n; i++) dst[of[i]] = b[i];
-    } else {
-      const float* b = (const float*)buf.data();
-      for (int32_t i = 0; i < n; i++) dst[of[i]] = (double)b[i];
-    }
-    return RSG_OK;
-  };
-  int rc;
-  if (V)
-    for (int d = 0; d < 3; d++)
-      if ((rc = fetch(h->V[d], h->nn, h->node_of, V + (size_t)d * h->nn))) return rc;
-  if (S)
-    for (int s = 0; s < 6; s++)
-      if ((rc = fetch(h->S[s], h->nc, h->cell_of, S + (size_t)s * h->nc))) return rc;
-  return RSG_OK;
+  const int rc = transfer_state(h, V, S, false);
+  return rc ? rc : check_resident(h);
 }
 
 int rsg_set_state(rsg_handle h, const double* V, const double* S) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   if (h->in_batch) return fail(RSG_ERR_STATE, "the handle is in a batch; remove it first");
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  const size_t e = h->elt();
-  std::vector<char> buf((size_t)std::max(h->nn, h->nc) * e);
-  auto put = [&](void* dst, int32_t n, const std::vector<int32_t>& of, const double* src) -> int {
-    if (e == 8) {
-      double* b = (double*)buf.data();
-      for (int32_t i = 0; i < n; i++) b[i] = src[of[i]];
-    } else {
-      float* b = (float*)buf.data();
-      for (int32_t i = 0; i < n; i++) b[i] = (float)src[of[i]];
-    }
-    HIP_TRY(copy_on(dst, buf.data(), (size_t)n * e, hipMemcpyHostToDevice, h->stream));
-    return RSG_OK;
-  };
-  int rc;
-  if (V)
-    for (int d = 0; d < 3; d++)
-      if ((rc = put(h->V[d], h->nn, h->node_of, V + (size_t)d * h->nn))) return rc;
-  if (S)
-    for (int s = 0; s < 6; s++)
-      if ((rc = put(h->S[s], h->nc, h->cell_of, S + (size_t)s * h->nc))) return rc;
-  return RSG_OK;
+  return transfer_state(h, const_cast<double*>(V), const_cast<double*>(S), true);
 }
 
 int rsg_get_traces(rsg_handle h, int64_t first, int64_t n, double* out) {

@@ -250,8 +250,8 @@ inline size_t resident_lds_bytes(int max_set, int max_node, int max_cell, size_t
 }
 constexpr size_t kResidentStaticLds = 2 * kResidentForces * 8 + 64;  // and what it declares itself
 
-// The launchers live in the kernel library only: builds of the host code without it step with
-// the per-step kernels.
+// These launchers, and those of the state transfers, live in the kernel library only: builds of
+// the host code without it step with the per-step kernels and reorder states on the host.
 #define RSG_WEAK __attribute__((weak))
 // Compute units of the current device (1 without cooperative launches), and LDS bytes a
 // workgroup may take.
@@ -259,6 +259,23 @@ RSG_WEAK hipError_t resident_limits(int* cus, size_t* lds);
 // threads: 256, 512 or 1024 per workgroup.
 RSG_WEAK hipError_t launch_resident_f64(const ResidentArgs<double>& a, int threads, hipStream_t s);
 RSG_WEAK hipError_t launch_resident_f32(const ResidentArgs<float>& a, int threads, hipStream_t s);
+
+// ---------------------------------------------------------------- state transfers (rsg_state.hip)
+template <typename T>
+struct StateArgs {
+  T* V[3];
+  T* S[6];
+  const int32_t* node_at;  // caller -> internal
+  const int32_t* cell_at;
+  int32_t nn, nc;
+};
+constexpr int kStateChunk = 1 << 18;  // values a chunk holds
+// Moves values [g0, g0 + n) of the caller's V[3][nn], S[6][nc] from the state to a chunk of pinned
+// host memory, or with `write` from the chunk to the state.
+RSG_WEAK hipError_t launch_state_f64(const StateArgs<double>& a, int64_t g0, int n, double* chunk, bool write,
+                                     hipStream_t s);
+RSG_WEAK hipError_t launch_state_f32(const StateArgs<float>& a, int64_t g0, int n, float* chunk, bool write,
+                                     hipStream_t s);
 
 // NaN boxing of a special-table index.
 inline double box_f64(int32_t idx) {

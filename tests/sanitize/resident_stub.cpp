@@ -1,4 +1,4 @@
-// resident_stub.cpp -- the resident kernel's launchers on the CPU, over the host stand-ins for the
+// resident_stub.cpp -- the resident kernel's and the state transfers' launchers on the CPU, over the host stand-ins for the
 // HIP runtime (hip_host_stub.cpp).  TEST INFRASTRUCTURE ONLY: it walks the tiles, records, halo and
 // exchange slots exactly as the kernel does (each tile with its own copy of its slots and nodes, the
 // exported stresses through the double-buffered exchange), with every index checked, so a plan that
@@ -225,5 +225,26 @@ hipError_t resident_limits(int* cus, size_t* lds) {
 }
 hipError_t launch_resident_f64(const ResidentArgs<double>& a, int threads, hipStream_t) { return run(a, threads); }
 hipError_t launch_resident_f32(const ResidentArgs<float>& a, int threads, hipStream_t) { return run(a, threads); }
+
+// State transfers, as rsg_state.hip makes them.
+template <typename T>
+static hipError_t state(const StateArgs<T>& a, int64_t g0, int n, T* chunk, bool write) {
+  CHECK(n > 0 && n <= kStateChunk && g0 >= 0 && g0 + n <= (int64_t)3 * a.nn + (int64_t)6 * a.nc);
+  for (int i = 0; i < n; i++) {
+    const int64_t g = g0 + i, v = (int64_t)3 * a.nn;
+    T* x = g < v ? a.V[g / a.nn] + a.node_at[g % a.nn] : a.S[(g - v) / a.nc] + a.cell_at[(g - v) % a.nc];
+    if (write)
+      *x = chunk[i];
+    else
+      chunk[i] = *x;
+  }
+  return hipSuccess;
+}
+hipError_t launch_state_f64(const StateArgs<double>& a, int64_t g0, int n, double* c, bool w, hipStream_t) {
+  return state(a, g0, n, c, w);
+}
+hipError_t launch_state_f32(const StateArgs<float>& a, int64_t g0, int n, float* c, bool w, hipStream_t) {
+  return state(a, g0, n, c, w);
+}
 
 }  // namespace rsg
