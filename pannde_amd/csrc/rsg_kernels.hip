@@ -79,11 +79,15 @@ namespace rsg {
 namespace {
 
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup i -> XCD i % 8).
-// Give XCD x the contiguous logical range [x*q + min(x,r), ...) instead.
-__device__ __forceinline__ int xcd_block(int bid, int nb) {
+// Give XCD x the contiguous logical range [x*q + min(x,r), ...) instead, from its first block on or
+// with `down` from its last.  The velocity kernel goes up and the stress kernel down, so each
+// starts where the other ended, on the state that is still in the 256 MiB memory-side cache
+// (both up: the bracket of 9.4 M cells 270 us a step in FP32 and 524 in FP64, against 239 and
+// 498; a million cells in FP64 62 against 59, the 3.9 M-cell plate 184 against 181).
+__device__ __forceinline__ int xcd_block(int bid, int nb, bool down) {
   const int x = bid & 7, j = bid >> 3;
   const int q = nb >> 3, r = nb & 7;
-  return x * q + (x < r ? x : r) + j;
+  return x * q + (x < r ? x : r) + (down ? q + (x < r ? 1 : 0) - 1 - j : j);
 }
 
 // Cells around a node: a missing cell (-1) contributes zero.  LDS-staged gathers need no
@@ -595,13 +599,13 @@ __device__ __forceinline__ void stress_body(const StressArgs<T>& a, int b, unsig
 template <typename T, bool LDS, int U, int CPT, int KM>
 __global__ __launch_bounds__(RSG_MAX_BLOCK) RSG_VELOCITY_ATTR void velocity_kernel(VelocityArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  velocity_body<T, LDS, U, CPT, KM>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x, smem);
+  velocity_body<T, LDS, U, CPT, KM>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x, false) : (int)blockIdx.x, smem);
 }
 
 template <typename T, bool LDS, int U, int CPT, int KM>
 __global__ __launch_bounds__(RSG_MAX_BLOCK) RSG_STRESS_ATTR void stress_kernel(StressArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  stress_body<T, LDS, U, CPT, KM>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x, smem);
+  stress_body<T, LDS, U, CPT, KM>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x, true) : (int)blockIdx.x, smem);
 }
 
 // Batched launches walk a table of n (instance, block) items.  The host stores the items
