@@ -65,6 +65,7 @@ struct VelocityArgs {
   int32_t n;
   int32_t xcd;  // 1: remap workgroups so each XCD owns a contiguous range
   int32_t cpt;  // entities per thread: a workgroup covers cpt * blockDim.x nodes
+  int32_t stream;  // 1: non-temporal loads of what a step reads once (links, keys, lists)
   // LDS staging (lconn != nullptr): per-block unique cell lists and 16-bit local links
   const int32_t* u_off;    // [nblocks+1]
   const int32_t* ulist;    // cells staged by each block
@@ -111,6 +112,7 @@ struct StressArgs {
   int32_t n;
   int32_t xcd;
   int32_t cpt;             // cells per thread
+  int32_t stream;          // as for VelocityArgs (and the per-cell C)
   const int32_t* u_off;    // LDS staging: per-block unique node lists
   const int32_t* ulist;
   const uint16_t* lconn;   // [n][8] block-local vertex index

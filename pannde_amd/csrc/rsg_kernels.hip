@@ -52,17 +52,6 @@
 #define RSG_VELOCITY_ATTR
 #endif
 
-// Loads of data read once per step (links, keys, gather lists, per-entity C): non-temporal
-// by default; RSG_CACHED_LINKS=1 makes them ordinary loads so they can stay cached.
-#ifndef RSG_CACHED_LINKS
-#define RSG_CACHED_LINKS 0
-#endif
-#if RSG_CACHED_LINKS
-#define STREAM_LOAD(p) (*(p))
-#else
-#define STREAM_LOAD(p) __builtin_nontemporal_load(p)
-#endif
-
 // Velocity staging layout: 1 (default) keeps the six staged stress components as three rows
 // of pairs, so one LDS read returns two components of a cell; 0 keeps six rows.
 #ifndef RSG_VELOCITY_PAIRS
@@ -88,6 +77,17 @@ __device__ __forceinline__ int xcd_block(int bid, int nb, bool down) {
   const int x = bid & 7, j = bid >> 3;
   const int q = nb >> 3, r = nb & 7;
   return x * q + (x < r ? x : r) + (down ? q + (x < r ? 1 : 0) - 1 - j : j);
+}
+
+// Loads of data read once per step (links, keys, gather lists, per-entity C).  NT: non-temporal, so
+// that on a mesh whose step does not fit the 256 MiB memory-side cache they leave it to the state,
+// which the next kernel reads again; else ordinary loads, which stay cached for the next step.
+template <bool NT, typename P>
+__device__ __forceinline__ P stream_load(const P* p) {
+  if constexpr (NT)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
 }
 
 // Cells around a node: a missing cell (-1) contributes zero.  LDS-staged gathers need no
@@ -129,19 +129,21 @@ __device__ __forceinline__ constexpr bool keyed(const A&) {
   return KM == 1 || KM == 3;
 }
 
-// 8 x int32 of one entity as two 16-byte loads; read once per step, so non-temporal.
+// 8 x int32 of one entity as two 16-byte loads.
+template <bool NT>
 __device__ __forceinline__ void load_conn(const int32_t* __restrict__ conn, int i, int (&c)[8]) {
   const v4i* p = reinterpret_cast<const v4i*>(conn) + 2 * (size_t)i;
-  const v4i lo = STREAM_LOAD(p);
-  const v4i hi = STREAM_LOAD(p + 1);
+  const v4i lo = stream_load<NT>(p);
+  const v4i hi = stream_load<NT>(p + 1);
   c[0] = lo.x; c[1] = lo.y; c[2] = lo.z; c[3] = lo.w;
   c[4] = hi.x; c[5] = hi.y; c[6] = hi.z; c[7] = hi.w;
 }
 
 // 8 x uint16 block-local indices of one entity as one 16-byte load (0xFFFF = none, returned
 // as `none`).
+template <bool NT>
 __device__ __forceinline__ void load_lconn(const uint16_t* __restrict__ lconn, int i, int (&c)[8], int none) {
-  const v4i w = STREAM_LOAD(reinterpret_cast<const v4i*>(lconn) + (size_t)i);
+  const v4i w = stream_load<NT>(reinterpret_cast<const v4i*>(lconn) + (size_t)i);
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     const uint32_t u = (uint32_t)w[k];
@@ -153,8 +155,9 @@ __device__ __forceinline__ void load_lconn(const uint16_t* __restrict__ lconn, i
 
 // 8 block-local indices (10 bits each, kNoLink = none, returned as `none`) and the key of one
 // entity, one 16-byte load.
+template <bool NT>
 __device__ __forceinline__ uint32_t load_lkey(const uint32_t* __restrict__ lkey, int i, int (&c)[8], int none) {
-  const v4i w = STREAM_LOAD(reinterpret_cast<const v4i*>(lkey) + (size_t)i);
+  const v4i w = stream_load<NT>(reinterpret_cast<const v4i*>(lkey) + (size_t)i);
   const uint32_t w0 = (uint32_t)w.x, w1 = (uint32_t)w.y, w2 = (uint32_t)w.z;
   const uint32_t l[8] = {w0 & kNoLink, (w0 >> 10) & kNoLink, (w0 >> 20) & kNoLink, w1 & kNoLink,
                          (w1 >> 10) & kNoLink, (w1 >> 20) & kNoLink, w2 & kNoLink, (w2 >> 10) & kNoLink};
@@ -194,7 +197,7 @@ __device__ __forceinline__ void zero_staged(T* lds, int ld, int zero) {
 // list holds one word per 4 LDS slots, start << 2 | (len - 1), and slot 4c + k takes entity
 // start + k when k < len (the other slots of the chunk stay unwritten: no link points at
 // them).
-template <typename T, int NCOMP, int U, bool CHUNKS = false, bool PAIRS = false>
+template <typename T, int NCOMP, int U, bool NT, bool CHUNKS = false, bool PAIRS = false>
 __device__ __forceinline__ void stage(T* lds, int ld, const int32_t* __restrict__ u_off,
                                       const int32_t* __restrict__ ulist, int b,
                                       const T* const (&src)[NCOMP], int zero, bool chunked = false) {
@@ -207,7 +210,7 @@ __device__ __forceinline__ void stage(T* lds, int ld, const int32_t* __restrict_
 #pragma unroll
         for (int u = 0; u < U; u++) {
           const int i = threadIdx.x + u * blockDim.x;
-          const int w = STREAM_LOAD(ulist + c0 + (i < nu ? (i >> 2) : 0));
+          const int w = stream_load<NT>(ulist + c0 + (i < nu ? (i >> 2) : 0));
           on[u] = i < nu && (i & 3) <= (w & 3);
           g[u] = on[u] ? (w >> 2) + (i & 3) : 0;
         }
@@ -221,7 +224,7 @@ __device__ __forceinline__ void stage(T* lds, int ld, const int32_t* __restrict_
           if (on[u]) put_staged<T, NCOMP, PAIRS>(lds, ld, threadIdx.x + u * blockDim.x, v[u]);
       } else {
         for (int i = threadIdx.x; i < nu; i += blockDim.x) {
-          const int w = STREAM_LOAD(ulist + c0 + (i >> 2));
+          const int w = stream_load<NT>(ulist + c0 + (i >> 2));
           if ((i & 3) > (w & 3)) continue;
           const int g = (w >> 2) + (i & 3);
           T v[NCOMP];
@@ -241,7 +244,7 @@ __device__ __forceinline__ void stage(T* lds, int ld, const int32_t* __restrict_
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int i = threadIdx.x + u * blockDim.x;
-      g[u] = STREAM_LOAD(ulist + u0 + (i < nu ? i : 0));
+      g[u] = stream_load<NT>(ulist + u0 + (i < nu ? i : 0));
     }
     T v[U][NCOMP];
 #pragma unroll
@@ -255,7 +258,7 @@ __device__ __forceinline__ void stage(T* lds, int ld, const int32_t* __restrict_
     }
   } else {
     for (int i = threadIdx.x; i < nu; i += blockDim.x) {
-      const int g = STREAM_LOAD(ulist + u0 + i);
+      const int g = stream_load<NT>(ulist + u0 + i);
       T v[NCOMP];
 #pragma unroll
       for (int k = 0; k < NCOMP; k++) v[k] = src[k][g];
@@ -274,18 +277,18 @@ struct VelIn {
   T idt, sx, sy, sz, v0, v1, v2;
 };
 
-template <typename T, bool LDS, int KM>
+template <typename T, bool LDS, int KM, bool NT>
 __device__ __forceinline__ void velocity_load(const VelocityArgs<T>& a, int n, VelIn<T>& in) {
   if constexpr (LDS) {
     if (packed<KM>(a))
-      in.key = load_lkey(a.lkey, n, in.c, a.max_u);  // missing cells -> the zero entry
+      in.key = load_lkey<NT>(a.lkey, n, in.c, a.max_u);  // missing cells -> the zero entry
     else
-      load_lconn(a.lconn, n, in.c, a.max_u);
+      load_lconn<NT>(a.lconn, n, in.c, a.max_u);
   } else {
-    load_conn(a.ncell, n, in.c);
+    load_conn<NT>(a.ncell, n, in.c);
   }
   if (keyed<KM>(a)) {
-    if (!(LDS && packed<KM>(a))) in.key = STREAM_LOAD(a.key + n);
+    if (!(LDS && packed<KM>(a))) in.key = stream_load<NT>(a.key + n);
     in.idt = in.sx = in.sy = in.sz = T(0);
   } else {
     in.key = 0;
@@ -363,13 +366,13 @@ __device__ __forceinline__ void velocity_apply(const VelocityArgs<T>& a, int n, 
 // (CPT * blockDim.x nodes, thread t taking nodes t, t + blockDim.x, ...).  With LDS the
 // chunk's unique cells are staged first; the streaming operands of the first two nodes
 // are requested before the staging so their latency overlaps it.
-template <typename T, bool LDS, int U, int CPT, int KM>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT>
 __device__ __forceinline__ void velocity_body(const VelocityArgs<T>& a, int b, unsigned char* smem) {
   const int bd = (int)blockDim.x;
   const int base = b * CPT * bd + (int)threadIdx.x;
   VelIn<T> in, next;
-  velocity_load<T, LDS, KM>(a, base < a.n ? base : a.n - 1, in);  // tail threads load a valid node
-  if constexpr (CPT > 1) velocity_load<T, LDS, KM>(a, base + bd < a.n ? base + bd : a.n - 1, next);
+  velocity_load<T, LDS, KM, NT>(a, base < a.n ? base : a.n - 1, in);  // tail threads load a valid node
+  if constexpr (CPT > 1) velocity_load<T, LDS, KM, NT>(a, base + bd < a.n ? base + bd : a.n - 1, next);
   const T* S0 = a.S0;
   const T* S1 = a.S1;
   const T* S2 = a.S2;
@@ -383,14 +386,14 @@ __device__ __forceinline__ void velocity_body(const VelocityArgs<T>& a, int b, u
     if constexpr (RSG_VELOCITY_PAIRS) {
       // pairs in the order the update reads them: (Sxx, Sxy), (Sxz, Syy), (Syz, Szz)
       const T* const src[6] = {a.S0, a.S5, a.S4, a.S1, a.S3, a.S2};
-      stage<T, 6, U, true, true>(lds, ld, a.u_off, a.ulist, b, src, a.max_u, a.uchunk != 0);
+      stage<T, 6, U, NT, true, true>(lds, ld, a.u_off, a.ulist, b, src, a.max_u, a.uchunk != 0);
       S0 = lds;
       S1 = lds + 2 * ld;
       S2 = lds + 4 * ld;
       S3 = S4 = S5 = nullptr;
     } else {
       const T* const src[6] = {a.S0, a.S1, a.S2, a.S3, a.S4, a.S5};
-      stage<T, 6, U, true>(lds, ld, a.u_off, a.ulist, b, src, a.max_u, a.uchunk != 0);
+      stage<T, 6, U, NT, true>(lds, ld, a.u_off, a.ulist, b, src, a.max_u, a.uchunk != 0);
       S0 = lds;
       S1 = lds + ld;
       S2 = lds + 2 * ld;
@@ -407,17 +410,17 @@ __device__ __forceinline__ void velocity_body(const VelocityArgs<T>& a, int b, u
     const int n = base + j * bd;
     if (n >= a.n) break;
     in = next;
-    if (j + 1 < CPT) velocity_load<T, LDS, KM>(a, n + bd < a.n ? n + bd : a.n - 1, next);
+    if (j + 1 < CPT) velocity_load<T, LDS, KM, NT>(a, n + bd < a.n ? n + bd : a.n - 1, next);
     velocity_apply<T, LDS, KM>(a, n, in, S0, S1, S2, S3, S4, S5);
   }
 }
 
-template <typename T>
+template <bool NT, typename T>
 __device__ __forceinline__ T cload(const T* __restrict__ C, int64_t ldc, int j, int i) {
   // ldc > 0: [21][ldc] arrays; ldc == 0: blocks of 64 cells, [n/64][21][64], so one
   // wavefront's 21 coefficients are a single contiguous run
   const int64_t idx = ldc ? (int64_t)j * ldc + i : ((int64_t)(i >> 6) * 21 + j) * 64 + (i & 63);
-  return STREAM_LOAD(C + idx);
+  return stream_load<NT>(C + idx);
 }
 
 // Per-cell operands of the stress update that do not depend on a gather: links,
@@ -431,18 +434,18 @@ struct StrIn {
   T s[6];
 };
 
-template <typename T, bool LDS, int KM>
+template <typename T, bool LDS, int KM, bool NT>
 __device__ __forceinline__ void stress_load(const StressArgs<T>& a, int e, StrIn<T>& in) {
   if constexpr (LDS) {
     if (packed<KM>(a))
-      in.key = load_lkey(a.lkey, e, in.c, -1);  // a cell has all 8 vertices
+      in.key = load_lkey<NT>(a.lkey, e, in.c, -1);  // a cell has all 8 vertices
     else
-      load_lconn(a.lconn, e, in.c, -1);
+      load_lconn<NT>(a.lconn, e, in.c, -1);
   } else {
-    load_conn(a.cnode, e, in.c);
+    load_conn<NT>(a.cnode, e, in.c);
   }
   if (keyed<KM>(a)) {
-    if (!(LDS && packed<KM>(a))) in.key = STREAM_LOAD(a.key + e);
+    if (!(LDS && packed<KM>(a))) in.key = stream_load<NT>(a.key + e);
     in.sx = in.sy = in.sz = T(0);
 #pragma unroll
     for (int j = 0; j < 21; j++) in.cc[j] = T(0);
@@ -452,7 +455,7 @@ __device__ __forceinline__ void stress_load(const StressArgs<T>& a, int e, StrIn
     in.sy = a.dcy[e];
     in.sz = a.dcz[e];
 #pragma unroll
-    for (int j = 0; j < 21; j++) in.cc[j] = cload(a.C, a.ldc, j, e);
+    for (int j = 0; j < 21; j++) in.cc[j] = cload<NT>(a.C, a.ldc, j, e);
   }
   in.s[0] = a.S0[e];
   in.s[1] = a.S1[e];
@@ -563,13 +566,13 @@ __device__ __forceinline__ void stress_apply(const StressArgs<T>& a, int e, StrI
 // Every operand that does not depend on a gather is requested first, so a cell's whole
 // streaming traffic (links, spacings, 21 C, 6 S) is in flight at once and its latency
 // overlaps the LDS staging of the chunk's unique nodes.
-template <typename T, bool LDS, int U, int CPT, int KM>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT>
 __device__ __forceinline__ void stress_body(const StressArgs<T>& a, int b, unsigned char* smem) {
   const int bd = (int)blockDim.x;
   const int base = b * CPT * bd + (int)threadIdx.x;
   StrIn<T> in, next;
-  stress_load<T, LDS, KM>(a, base < a.n ? base : a.n - 1, in);  // tail threads load a valid cell
-  if constexpr (CPT > 1) stress_load<T, LDS, KM>(a, base + bd < a.n ? base + bd : a.n - 1, next);
+  stress_load<T, LDS, KM, NT>(a, base < a.n ? base : a.n - 1, in);  // tail threads load a valid cell
+  if constexpr (CPT > 1) stress_load<T, LDS, KM, NT>(a, base + bd < a.n ? base + bd : a.n - 1, next);
   const T* V0 = a.V0;
   const T* V1 = a.V1;
   const T* V2 = a.V2;
@@ -577,7 +580,7 @@ __device__ __forceinline__ void stress_body(const StressArgs<T>& a, int b, unsig
   if constexpr (LDS) {
     T* lds = reinterpret_cast<T*>(smem);
     const T* const src[3] = {a.V0, a.V1, a.V2};
-    stage<T, 3, U, false, PAIRS>(lds, a.max_u, a.u_off, a.ulist, b, src, -1);
+    stage<T, 3, U, NT, false, PAIRS>(lds, a.max_u, a.u_off, a.ulist, b, src, -1);
     V0 = lds;
     V1 = PAIRS ? nullptr : lds + a.max_u;
     V2 = lds + 2 * a.max_u;
@@ -590,22 +593,22 @@ __device__ __forceinline__ void stress_body(const StressArgs<T>& a, int b, unsig
     const int e = base + j * bd;
     if (e >= a.n) break;
     in = next;
-    if (j + 1 < CPT) stress_load<T, LDS, KM>(a, e + bd < a.n ? e + bd : a.n - 1, next);
+    if (j + 1 < CPT) stress_load<T, LDS, KM, NT>(a, e + bd < a.n ? e + bd : a.n - 1, next);
     stress_apply<T, KM, PAIRS>(a, e, in, V0, V1, V2);
   }
 }
 
 // Single-instance launches: one workgroup per block, XCD-contiguous block order.
-template <typename T, bool LDS, int U, int CPT, int KM>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT>
 __global__ __launch_bounds__(RSG_MAX_BLOCK) RSG_VELOCITY_ATTR void velocity_kernel(VelocityArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  velocity_body<T, LDS, U, CPT, KM>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x, false) : (int)blockIdx.x, smem);
+  velocity_body<T, LDS, U, CPT, KM, NT>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x, false) : (int)blockIdx.x, smem);
 }
 
-template <typename T, bool LDS, int U, int CPT, int KM>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT>
 __global__ __launch_bounds__(RSG_MAX_BLOCK) RSG_STRESS_ATTR void stress_kernel(StressArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  stress_body<T, LDS, U, CPT, KM>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x, true) : (int)blockIdx.x, smem);
+  stress_body<T, LDS, U, CPT, KM, NT>(a, a.xcd ? xcd_block(blockIdx.x, gridDim.x, true) : (int)blockIdx.x, smem);
 }
 
 // Batched launches walk a table of n (instance, block) items.  The host stores the items
@@ -628,7 +631,7 @@ __device__ __forceinline__ void velocity_item(const BatchDesc<T>* __restrict__ d
   VelocityArgs<T> a = d->v;
   a.amp = d->amp_base + (size_t)k * d->nch;
   a.trace = d->trace_base ? d->trace_base + (size_t)(d->trace_row0 + k) * d->row : nullptr;
-  velocity_body<T, LDS, U, CPT, KM>(a, it.y, smem);
+  velocity_body<T, LDS, U, CPT, KM, true>(a, it.y, smem);
 }
 
 template <typename T, bool LDS, int U, int CPT, int KM>
@@ -638,7 +641,7 @@ __device__ __forceinline__ void stress_item(const BatchDesc<T>* __restrict__ des
   const BatchDesc<T>* d = desc + (it.x & (kMaxBatchSlots - 1));
   StressArgs<T> a = d->s;
   a.amp = d->amp_base + (size_t)k * d->nch;
-  stress_body<T, LDS, U, CPT, KM>(a, it.y, smem);
+  stress_body<T, LDS, U, CPT, KM, true>(a, it.y, smem);
 }
 
 template <typename T, bool LDS, int U, int CPT, int KM, bool PERSIST>
@@ -715,12 +718,20 @@ hipError_t with_variant(bool lds, int max_u, int block, int cpt, int km, F&& f) 
   }
 }
 
+// Kernel instances that also come with ordinary loads of the once-a-step data: the staged ones of
+// the default shapes.
+constexpr bool cacheable(bool lds, int u, int cpt) { return lds && u > 0 && cpt <= 2; }
+
 template <typename T>
 hipError_t launch_velocity(const VelocityArgs<T>& a, int block, hipStream_t s) {
   const bool lds = a.lconn != nullptr || a.lkey != nullptr;
   return with_variant(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : 0, [&](auto L, auto U, auto C, auto K) {
-    return launch1d(velocity_kernel<T, decltype(L)::value, decltype(U)::value, decltype(C)::value, decltype(K)::value>,
-                    a, a.n, block, lds ? velocity_lds_bytes(a.max_u, sizeof(T)) : 0, s);
+    constexpr bool l = decltype(L)::value;
+    constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
+    const size_t bytes = lds ? velocity_lds_bytes(a.max_u, sizeof(T)) : 0;
+    if constexpr (cacheable(l, u, c))
+      if (!a.stream) return launch1d(velocity_kernel<T, l, u, c, m, false>, a, a.n, block, bytes, s);
+    return launch1d(velocity_kernel<T, l, u, c, m, true>, a, a.n, block, bytes, s);
   });
 }
 
@@ -728,8 +739,12 @@ template <typename T>
 hipError_t launch_stress(const StressArgs<T>& a, int block, hipStream_t s) {
   const bool lds = a.lconn != nullptr || a.lkey != nullptr;
   return with_variant(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : 0, [&](auto L, auto U, auto C, auto K) {
-    return launch1d(stress_kernel<T, decltype(L)::value, decltype(U)::value, decltype(C)::value, decltype(K)::value>,
-                    a, a.n, block, lds ? (size_t)3 * a.max_u * sizeof(T) : 0, s);
+    constexpr bool l = decltype(L)::value;
+    constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
+    const size_t bytes = lds ? (size_t)3 * a.max_u * sizeof(T) : 0;
+    if constexpr (cacheable(l, u, c))
+      if (!a.stream) return launch1d(stress_kernel<T, l, u, c, m, false>, a, a.n, block, bytes, s);
+    return launch1d(stress_kernel<T, l, u, c, m, true>, a, a.n, block, bytes, s);
   });
 }
 
