@@ -29,6 +29,7 @@
 #include <cstring>
 #include <ctime>
 #include <exception>
+#include <iterator>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -45,6 +46,7 @@
 #include "rsg_resident_plan.h"
 
 namespace {
+void leave_resident_order(const rsg_instance* h);
 
 thread_local std::string g_last_error;
 
@@ -235,6 +237,23 @@ struct DevBuf {
   size_t bytes() const { return n * sizeof(T); }
 };
 
+// Resident launches of several tiles fill the GPU, so they run one at a time on a device: each
+// waits for the last one that another handle made there.
+struct ResidentOrder {
+  std::mutex mu;
+  std::unordered_map<int, rsg_instance*> last;  // by device
+};
+ResidentOrder& resident_order() {
+  static ResidentOrder o;
+  return o;
+}
+// Before the handle's event goes (its stream is idle).
+void leave_resident_order(const rsg_instance* h) {
+  ResidentOrder& o = resident_order();
+  std::lock_guard<std::mutex> lock(o.mu);
+  for (auto it = o.last.begin(); it != o.last.end();) it = it->second == h ? o.last.erase(it) : std::next(it);
+}
+
 constexpr int kBlockSteps = 256;   // steps whose amplitudes are staged per upload
 constexpr int kTraceCapSteps = 4096;
 
@@ -323,6 +342,9 @@ struct rsg_instance {
   int32_t res_nclasses = -1;
   std::vector<std::vector<int32_t>> res_force;
   DevBuf<uint8_t> res_ncls, res_ccls;
+  void* res_ctrl = nullptr;
+  uint32_t res_seq = 0;            // launches so far
+  hipEvent_t res_event = nullptr;  // behind the last one
   int32_t* res_status = nullptr;  // pinned, from the first resident launch on
   void* res_flag = nullptr;
   uint32_t res_epoch = 0;         // steps taken by resident launches
@@ -422,6 +444,8 @@ struct rsg_instance {
       if (stage[i]) (void)hipHostFree(stage[i]);
       if (stage_ev[i]) (void)hipEventDestroy(stage_ev[i]);
     }
+    leave_resident_order(this);
+    if (res_event) (void)hipEventDestroy(res_event);
     if (res_status) (void)hipHostFree(res_status);
     for (void* c : chunk)
       if (c) (void)hipHostFree(c);
@@ -1321,8 +1345,8 @@ int build_tables(rsg_instance* h) {
 
 // Fails when a wait of the resident kernel ran out in work that has been synchronized.
 int check_resident(rsg_instance* h) {
-  if (h->res_status && *h->res_status)
-    return fail(RSG_ERR_DEVICE, "the resident step kernel's workgroups did not all run at once");
+  if (h->res_status && __atomic_load_n(h->res_status + rsg::kResidentLost, __ATOMIC_RELAXED))
+    return fail(RSG_ERR_DEVICE, "the resident step kernel's workgroups lost each other");
   return RSG_OK;
 }
 
@@ -1416,10 +1440,11 @@ int ensure_events(rsg_instance* h, size_t n) {
   return RSG_OK;
 }
 
-// A resident launch of several tiles takes at least this many steps: a cooperative launch costs
-// about 20 us more than a plain one (32,000 cells, FP64: 4 steps 43.5 us against 38.2 with the
-// per-step kernels, 6 steps 51.8 against 57.2).
-constexpr int kResidentMinSteps = 6;
+// A resident launch of several tiles takes at least this many steps: loading and storing the tiles
+// and agreeing on the start cost about what the resident steps save on two to four per-step ones
+// (back to back, us, resident / per-step kernels: 32,000 cells FP64 4 steps 33 / 39, 6 steps 40 /
+// 58; 259,000 cells FP32 4 steps 49 / 46, 6 steps 63 / 68).
+constexpr int kResidentMinSteps = 5;
 
 // kb steps in one launch of the resident kernel; *done says whether it was launched.
 template <typename T>
@@ -1427,8 +1452,12 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
                  const double* force, size_t row, bool* done) {
   *done = false;
   if (!h->res_status) {
-    HIP_TRY(hipHostMalloc((void**)&h->res_status, sizeof(int32_t), hipHostMallocDefault));
-    *h->res_status = 0;
+    HIP_TRY(hipHostMalloc((void**)&h->res_status, rsg::kResidentStatus * sizeof(int32_t), hipHostMallocDefault));
+    memset(h->res_status, 0, rsg::kResidentStatus * sizeof(int32_t));
+  }
+  if (__atomic_load_n(h->res_status + rsg::kResidentAlone, __ATOMIC_RELAXED)) {
+    h->res_tiles = 0;  // the GPU is shared with work that keeps the tiles apart
+    return RSG_OK;
   }
   rsg::ResidentArgs<T> a;
   a.v = va;
@@ -1439,6 +1468,8 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   a.halo = (const int2*)h->res_halo;
   a.hcell = (const int32_t*)h->res_hcell;
   a.xbuf = (unsigned long long*)h->res_xbuf;
+  a.ctrl = (uint32_t*)h->res_ctrl;
+  a.seq = h->res_seq + 1;
   a.status = h->res_status;
   a.flag = (uint32_t*)h->res_flag;
   a.epoch = h->res_epoch;
@@ -1455,16 +1486,27 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   a.ccls = h->res_ccls.p;
   a.cforce0 = 3 * h->res_nclasses;
   a.row = (int32_t)row;
+  auto launch = [&]() -> hipError_t {
+    if constexpr (sizeof(T) == 8)
+      return rsg::launch_resident_f64(a, h->res_threads, h->stream);
+    else
+      return rsg::launch_resident_f32(a, h->res_threads, h->stream);
+  };
   hipError_t e;
-  if constexpr (sizeof(T) == 8)
-    e = rsg::launch_resident_f64(a, h->res_threads, h->stream);
-  else
-    e = rsg::launch_resident_f32(a, h->res_threads, h->stream);
-  if (e == hipErrorCooperativeLaunchTooLarge) {  // not all tiles fit this GPU at once
-    h->res_tiles = 0;
-    return RSG_OK;
+  if (h->res_tiles == 1) {
+    e = launch();
+  } else {
+    if (!h->res_event) HIP_TRY(hipEventCreateWithFlags(&h->res_event, hipEventDisableTiming));
+    ResidentOrder& o = resident_order();
+    std::lock_guard<std::mutex> lock(o.mu);
+    rsg_instance*& last = o.last[h->device];
+    if (last && last != h) HIP_TRY(rsg::resident_after(h->stream, last->res_event));
+    e = launch();
+    if (e == hipSuccess) e = hipEventRecord(h->res_event, h->stream);
+    if (e == hipSuccess) last = h;
   }
   if (e != hipSuccess) return fail(RSG_ERR_DEVICE, "resident launch: %s", hipGetErrorString(e));
+  h->res_seq++;
   h->res_epoch += (uint32_t)kb;
   *done = true;
   return RSG_OK;
@@ -2236,6 +2278,11 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     if ((rc = upload(h.get(), &h->res_hcell, std::move(p.hcell)))) return rc;
     if ((rc = upload(h.get(), &h->res_flag, std::vector<uint32_t>((size_t)tiles * rsg::kFlagStride, 0)))) return rc;
     if ((rc = h->dalloc(&h->res_xbuf, (size_t)12 * p.nexp * e))) return rc;
+    // PANNDE_RSG_RESIDENT=alone (tests): the count of started tiles begins where it never meets a
+    // launch's total, so every launch decides against its steps
+    const char* alone = std::getenv("PANNDE_RSG_RESIDENT");
+    const uint32_t started = alone && !strcmp(alone, "alone") ? 1u << 31 : 0;
+    if ((rc = upload(h.get(), &h->res_ctrl, std::vector<uint32_t>{started, 0}))) return rc;
     if (rsg::resident_lds_bytes(h->res_set, h->res_node, h->res_cell, e, true) + rsg::kResidentStaticLds > lds &&
         (rc = h->dalloc(&h->res_work, (size_t)16 * tiles * (h->res_node + h->res_cell))))
       return rc;

@@ -215,6 +215,10 @@ constexpr int kFlagStride = 32;                   // a flag per 128-byte line
 constexpr int kResidentForces = 256;  // largest row
 constexpr uint8_t kResidentSensor = 0x80;  // node mark: a sensor this tile records
 
+// Status words, 1 when: a launch's tiles did not get onto the GPU together and one workgroup made
+// its steps (later launches should not try); a wait between tiles ran out (the state is lost).
+constexpr int kResidentAlone = 0, kResidentLost = 1, kResidentStatus = 2;
+
 template <typename T>
 struct ResidentArgs {
   VelocityArgs<T> v;  // state, coefficients, sources and sensors as the per-step kernels take them
@@ -227,7 +231,9 @@ struct ResidentArgs {
   const int32_t* hcell;  // internal id of each halo cell
   unsigned long long* xbuf;  // [2][6 * sizeof(T) / 8][nexp]: exported stresses of even and odd steps
   uint32_t* flag;        // [tiles][kFlagStride]: the step whose exported stresses are written
-  int32_t* status;       // set when a wait ran out
+  uint32_t* ctrl;        // [2]: tiles started, over all launches; the last decision (several tiles)
+  uint32_t seq;          // number of the launch, from 1
+  int32_t* status;       // [kResidentStatus], pinned
   uint32_t epoch;        // the state's step, counted over the resident launches
   int32_t nsteps;        // >= 2
   int32_t ntiles;
@@ -255,9 +261,10 @@ constexpr size_t kResidentStaticLds = 2 * kResidentForces * 8 + 64;  // and what
 // These launchers, and those of the state transfers, live in the kernel library only: builds of
 // the host code without it step with the per-step kernels and reorder states on the host.
 #define RSG_WEAK __attribute__((weak))
-// Compute units of the current device (1 without cooperative launches), and LDS bytes a
-// workgroup may take.
+// Compute units of the current device, and LDS bytes a workgroup may take.
 RSG_WEAK hipError_t resident_limits(int* cus, size_t* lds);
+// Work queued on s from now on waits for the event.
+RSG_WEAK hipError_t resident_after(hipStream_t s, hipEvent_t e);
 // threads: 256, 512 or 1024 per workgroup.
 RSG_WEAK hipError_t launch_resident_f64(const ResidentArgs<double>& a, int threads, hipStream_t s);
 RSG_WEAK hipError_t launch_resident_f32(const ResidentArgs<float>& a, int threads, hipStream_t s);

@@ -223,6 +223,7 @@ hipError_t resident_limits(int* cus, size_t* lds) {
   *lds = 160 * 1024;
   return hipSuccess;
 }
+hipError_t resident_after(hipStream_t, hipEvent_t) { return hipSuccess; }
 hipError_t launch_resident_f64(const ResidentArgs<double>& a, int threads, hipStream_t) { return run(a, threads); }
 hipError_t launch_resident_f32(const ResidentArgs<float>& a, int threads, hipStream_t) { return run(a, threads); }
 

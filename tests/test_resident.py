@@ -119,6 +119,42 @@ def test_resident_equals_per_step_kernels(name, precision):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("precision", [rsg.RSG_FP64, rsg.RSG_FP32])
+@pytest.mark.parametrize("name", ("two_tiles", "cracked_plate", "moments", "rest"))
+def test_launch_that_decides_against_its_steps(name, precision, monkeypatch):
+    """Tiles that do not get onto the GPU together: one workgroup makes the steps, and the handle
+    goes on with the per-step kernels."""
+    case = jobs(name)
+    for tuning in (None, dict(coeff_classes=-1)):
+        per_step = dict(block_velocity=256, block_stress=256, **(tuning or {}))
+        ref = run(case, precision, per_step, [7, 9, 6])
+        with monkeypatch.context() as m:
+            m.setenv("PANNDE_RSG_RESIDENT", "alone")
+            got = run(case, precision, tuning, [7, 9, 6])
+        assert all(np.array_equal(a, b) for a, b in zip(got, ref)), tuning
+
+
+@pytest.mark.gpu
+def test_handles_on_several_threads():
+    """Resident launches of several handles take turns on the GPU."""
+    import threading
+
+    case = jobs("moments")
+    ref = run(case, rsg.RSG_FP64, dict(block_velocity=256, block_stress=256), [60])
+    out = [None] * 5
+
+    def work(i):
+        out[i] = run(case, rsg.RSG_FP64, None, [20, 5, 6, 9, 20])
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(out))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(o is not None and all(np.array_equal(a, b) for a, b in zip(o, ref)) for o in out)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("precision,dims", [(rsg.RSG_FP64, (64, 52, 41)), (rsg.RSG_FP64, (80, 71, 57)),
                                             (rsg.RSG_FP32, (80, 71, 57)), (rsg.RSG_FP32, (97, 83, 66))])
 def test_resident_at_its_largest(precision, dims):
