@@ -49,6 +49,40 @@ __device__ __forceinline__ float diffsum(const float (&f)[8]) {
 __device__ __forceinline__ double dscale(double v, double sp) { return v * 0.25 / sp; }
 __device__ __forceinline__ float dscale(float v, float inv) { return v * inv; }
 
+// A spacing as the resident kernel divides by it.  FP32 multiplies by its inverse anyway; FP64 takes
+// the same quotients as dscale, bit for bit, from the spacing's reciprocal: 4 fused operations
+// each instead of the 11 of an IEEE division.  With r = RN(1/d) and e = RN((1 - d r) r),
+// q = x r + x e is x/d to well under an ulp, so x - q d is exact and q + (x - q d) r rounds to the
+// correctly rounded quotient (Markstein, IBM J. Res. Dev. 34, 1990), where nothing under- or
+// overflows.
+struct Recip {
+  double d, r, e;
+};
+__device__ __forceinline__ void set_spacing(double d, Recip& s) {
+  // a spacing of no usual size: every quotient comes out NaN and is taken by an IEEE division
+  const bool usual = fabs(d) > 0x1p-60 && fabs(d) < 0x1p60;
+  s.d = d;
+  s.r = usual ? 1.0 / d : __builtin_nan("");
+  s.e = __builtin_fma(-d, s.r, 1.0) * s.r;
+}
+__device__ __forceinline__ void set_spacing(float inv, float& s) { s = inv; }
+__device__ __forceinline__ double quotient(double v, const Recip& s) {
+  const double x = v * 0.25;
+  const double q = __builtin_fma(x, s.r, x * s.e);
+  return __builtin_fma(__builtin_fma(-q, s.d, x), s.r, q);
+}
+__device__ __forceinline__ float quotient(float v, float inv) { return v * inv; }
+// Nonzero difference sums below 2^kTinySum go the long way: x - q d would underflow.  (A zero's
+// exponent reads as 0.)  A wave's sums are rarely there but for the front of a pulse, long before
+// it can be seen.
+constexpr int kTinySum = -890;
+__device__ __forceinline__ int least_exponent(const double (&v)[9]) {
+  int e = __builtin_amdgcn_frexp_exp(v[0]);
+#pragma unroll
+  for (int i = 1; i < 9; i++) e = min(e, (int)__builtin_amdgcn_frexp_exp(v[i]));
+  return e;
+}
+
 typedef double d2v __attribute__((ext_vector_type(2)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
@@ -146,50 +180,105 @@ __device__ __forceinline__ void voigt_update(T dt, R cc, const T (&d)[6], const 
 // The velocity rates of a node before its sources, div S with the reference's order of
 // operations.  pair(p, f, g) reads components 2p and 2p + 1 of (Sxx, Sxy, Sxz, Syy, Syz, Szz)
 // at the node's 8 cells (0 at a missing one).
-template <typename T, typename L>
-__device__ __forceinline__ void node_rates(L&& pair, T sx, T sy, T sz, T (&r)[3]) {
-  T f[8], g[8];
-  pair(0, f, g);
-  const T dx_sxx = dscale(diffsum<0>(f), sx);
-  const T dx_sxy = dscale(diffsum<0>(g), sx);
-  const T dy_sxy = dscale(diffsum<1>(g), sy);
-  pair(1, f, g);
-  const T dx_sxz = dscale(diffsum<0>(f), sx);
-  const T dz_sxz = dscale(diffsum<2>(f), sz);
-  const T dy_syy = dscale(diffsum<1>(g), sy);
-  pair(2, f, g);
-  const T dy_syz = dscale(diffsum<1>(f), sy);
-  const T dz_syz = dscale(diffsum<2>(f), sz);
-  const T dz_szz = dscale(diffsum<2>(g), sz);
+template <typename T, typename D>
+__device__ __forceinline__ void sum_rates(D&& div, const T (&v)[9], T (&r)[3]) {
+  const T dx_sxx = div(v[0], 0), dx_sxy = div(v[1], 0), dx_sxz = div(v[2], 0);
+  const T dy_sxy = div(v[3], 1), dy_syy = div(v[4], 1), dy_syz = div(v[5], 1);
+  const T dz_sxz = div(v[6], 2), dz_syz = div(v[7], 2), dz_szz = div(v[8], 2);
   r[0] = (dx_sxx + dy_sxy) + dz_sxz;
   r[1] = (dx_sxy + dy_syy) + dz_syz;
   r[2] = (dx_sxz + dy_syz) + dz_szz;
+}
+template <typename T, typename L>
+__device__ __forceinline__ void node_sums(L&& pair, T (&v)[9]) {
+  T f[8], g[8];
+  pair(0, f, g);
+  v[0] = diffsum<0>(f);
+  v[1] = diffsum<0>(g);
+  v[3] = diffsum<1>(g);
+  pair(1, f, g);
+  v[2] = diffsum<0>(f);
+  v[6] = diffsum<2>(f);
+  v[4] = diffsum<1>(g);
+  pair(2, f, g);
+  v[5] = diffsum<1>(f);
+  v[7] = diffsum<2>(f);
+  v[8] = diffsum<2>(g);
+}
+template <typename T, typename L>
+__device__ __forceinline__ void node_rates(L&& pair, T sx, T sy, T sz, T (&r)[3]) {
+  T v[9];
+  node_sums(pair, v);
+  sum_rates([&](T x, int ax) { return dscale(x, ax == 0 ? sx : ax == 1 ? sy : sz); }, v, r);
 }
 
 // Strain-rate terms of one cell from its 8 vertices: the diagonal D_i V_i and the shear
 // sums D_j V_k + D_k V_j, in the reference's order of operations.  xy(f, g) reads Vx and Vy at
 // the vertices, z(f) reads Vz.
-template <typename T, typename LXY, typename LZ>
-__device__ __forceinline__ void strain_rates(LXY&& xy, LZ&& z, T sx, T sy, T sz, T (&d)[6]) {
-  // dik = D_i V_k (i: derivative axis, k: velocity component)
-  T f[8], g[8];
-  xy(f, g);
-  const T d00 = dscale(diffsum<0>(f), sx);
-  const T d10 = dscale(diffsum<1>(f), sy);
-  const T d20 = dscale(diffsum<2>(f), sz);
-  const T d01 = dscale(diffsum<0>(g), sx);
-  const T d11 = dscale(diffsum<1>(g), sy);
-  const T d21 = dscale(diffsum<2>(g), sz);
-  z(f);
-  const T d02 = dscale(diffsum<0>(f), sx);
-  const T d12 = dscale(diffsum<1>(f), sy);
-  const T d22 = dscale(diffsum<2>(f), sz);
-  d[0] = d00;
-  d[1] = d11;
-  d[2] = d22;
+template <typename T, typename D>
+__device__ __forceinline__ void sum_strains(D&& div, const T (&v)[9], T (&d)[6]) {
+  // v[3 i + k]: the difference sum of D_i V_k (i: derivative axis, k: velocity component)
+  d[0] = div(v[0], 0);
+  d[1] = div(v[4], 1);
+  d[2] = div(v[8], 2);
+  const T d12 = div(v[5], 1), d21 = div(v[7], 2), d02 = div(v[2], 0), d20 = div(v[6], 2);
+  const T d01 = div(v[1], 0), d10 = div(v[3], 1);
   d[3] = d12 + d21;
   d[4] = d02 + d20;
   d[5] = d01 + d10;
+}
+template <typename T, typename LXY, typename LZ>
+__device__ __forceinline__ void cell_sums(LXY&& xy, LZ&& z, T (&v)[9]) {
+  T f[8], g[8];
+  xy(f, g);
+  v[0] = diffsum<0>(f);
+  v[3] = diffsum<1>(f);
+  v[6] = diffsum<2>(f);
+  v[1] = diffsum<0>(g);
+  v[4] = diffsum<1>(g);
+  v[7] = diffsum<2>(g);
+  z(f);
+  v[2] = diffsum<0>(f);
+  v[5] = diffsum<1>(f);
+  v[8] = diffsum<2>(f);
+}
+template <typename T, typename LXY, typename LZ>
+__device__ __forceinline__ void strain_rates(LXY&& xy, LZ&& z, T sx, T sy, T sz, T (&d)[6]) {
+  T v[9];
+  cell_sums(xy, z, v);
+  sum_strains([&](T x, int ax) { return dscale(x, ax == 0 ? sx : ax == 1 ? sy : sz); }, v, d);
+}
+
+// The same with quotients from reciprocals; what they may not give goes through dscale.
+template <typename L>
+__device__ __forceinline__ void node_rates(L&& pair, const Recip (&s)[3], double (&r)[3]) {
+  double v[9];
+  node_sums(pair, v);
+  sum_rates([&](double x, int ax) { return quotient(x, s[ax]); }, v, r);
+  if (__builtin_isnan((r[0] + r[1]) + r[2]) || least_exponent(v) < kTinySum) {
+    asm volatile("" ::: "memory");  // read again rather than held in registers
+    node_sums(pair, v);
+    sum_rates([&](double x, int ax) { return dscale(x, s[ax].d); }, v, r);
+  }
+}
+template <typename L>
+__device__ __forceinline__ void node_rates(L&& pair, const float (&s)[3], float (&r)[3]) {
+  node_rates(pair, s[0], s[1], s[2], r);
+}
+template <typename LXY, typename LZ>
+__device__ __forceinline__ void strain_rates(LXY&& xy, LZ&& z, const Recip (&s)[3], double (&d)[6]) {
+  double v[9];
+  cell_sums(xy, z, v);
+  sum_strains([&](double x, int ax) { return quotient(x, s[ax]); }, v, d);
+  if (__builtin_isnan(((d[0] + d[1]) + (d[2] + d[3])) + (d[4] + d[5])) || least_exponent(v) < kTinySum) {
+    asm volatile("" ::: "memory");
+    cell_sums(xy, z, v);
+    sum_strains([&](double x, int ax) { return dscale(x, s[ax].d); }, v, d);
+  }
+}
+template <typename LXY, typename LZ>
+__device__ __forceinline__ void strain_rates(LXY&& xy, LZ&& z, const float (&s)[3], float (&d)[6]) {
+  strain_rates(xy, z, s[0], s[1], s[2], d);
 }
 
 // Summed force terms of a special node, added to its rates.

@@ -299,11 +299,11 @@ struct rsg_instance {
   uint32_t* nkey = nullptr;
   void* nmat = nullptr;   // [materials] dt/rho
   void* naxis = nullptr;  // [3][kAxisClasses] node spacings
-  int32_t n_nmat = -1;
+  int32_t n_nmat = -1, n_naxis = 0;  // materials; most spacings along an axis
   uint32_t* ckey = nullptr;
   void* cmat = nullptr;   // [materials][kMatRow] C
   void* caxis = nullptr;  // [3][kAxisClasses] cell spacings
-  int32_t n_cmat = -1;
+  int32_t n_cmat = -1, n_caxis = 0;
   std::vector<uint32_t> nkey_h, ckey_h;  // keys without the special flag, internal order
   // LDS staging plans (null lconn: direct gathers)
   int32_t* v_uoff = nullptr;
@@ -335,6 +335,7 @@ struct rsg_instance {
   void* res_halo = nullptr;
   void* res_hcell = nullptr;
   void* res_xbuf = nullptr;
+  size_t res_lds_room = 0;   // LDS a tile leaves free
   void* res_work = nullptr;  // the kernel's records where they do not fit LDS
   // source terms as the resident kernel takes them: one list of channels per class and component
   // (res_force: the node classes, 3 lists each, then the cell classes, 6 each); -1 node classes:
@@ -346,8 +347,6 @@ struct rsg_instance {
   uint32_t res_seq = 0;            // launches so far
   hipEvent_t res_event = nullptr;  // behind the last one
   int32_t* res_status = nullptr;  // pinned, from the first resident launch on
-  void* res_flag = nullptr;
-  uint32_t res_epoch = 0;         // steps taken by resident launches
 
   // state transfers: the caller -> internal maps on the device (from the first transfer on) and
   // each transfer thread's chunk of pinned memory
@@ -955,7 +954,7 @@ bool classify_rows(int32_t n, F&& row, std::vector<int32_t>& row_of, std::vector
 // would; entity() must be safe to call from several threads.
 template <typename T, int W, int ROW, typename F>
 int make_keys(rsg_instance* h, int32_t n, F&& entity, std::vector<uint32_t>& keys, void** mat_table,
-              void** axis_table, int32_t* materials) {
+              void** axis_table, int32_t* materials, int32_t* spacings) {
   *materials = -1;
   keys.resize(n);
   struct Chunk {
@@ -1059,6 +1058,7 @@ int make_keys(rsg_instance* h, int32_t n, F&& entity, std::vector<uint32_t>& key
   if ((rc = upload(h, mat_table, std::move(mt)))) return rc;
   if ((rc = upload(h, axis_table, std::move(at)))) return rc;
   *materials = (int32_t)nm;
+  *spacings = (int32_t)std::max({axv[0].size(), axv[1].size(), axv[2].size()});
   return RSG_OK;
 }
 
@@ -1465,14 +1465,12 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   a.tiles = (const rsg::ResidentTile*)h->res_tile;
   a.crec = (const uint32_t*)h->res_crec;
   a.nrec = (const uint32_t*)h->res_nrec;
-  a.halo = (const int2*)h->res_halo;
+  a.halo = (const int32_t*)h->res_halo;
   a.hcell = (const int32_t*)h->res_hcell;
   a.xbuf = (unsigned long long*)h->res_xbuf;
   a.ctrl = (uint32_t*)h->res_ctrl;
   a.seq = h->res_seq + 1;
   a.status = h->res_status;
-  a.flag = (uint32_t*)h->res_flag;
-  a.epoch = h->res_epoch;
   a.nsteps = kb;
   a.ntiles = h->res_tiles;
   a.nexp = h->res_nexp;
@@ -1486,6 +1484,9 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   a.ccls = h->res_ccls.p;
   a.cforce0 = 3 * h->res_nclasses;
   a.row = (int32_t)row;
+  a.nmat = std::max(0, h->n_nmat);
+  a.tables = h->n_nmat <= rsg::kResidentClasses && std::max(h->n_naxis, h->n_caxis) <= rsg::kResidentClasses &&
+             h->res_lds_room >= rsg::resident_table_bytes(h->elt());
   auto launch = [&]() -> hipError_t {
     if constexpr (sizeof(T) == 8)
       return rsg::launch_resident_f64(a, h->res_threads, h->stream);
@@ -1507,7 +1508,6 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   }
   if (e != hipSuccess) return fail(RSG_ERR_DEVICE, "resident launch: %s", hipGetErrorString(e));
   h->res_seq++;
-  h->res_epoch += (uint32_t)kb;
   *done = true;
   return RSG_OK;
 }
@@ -2055,8 +2055,8 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
         for (int d = 0; d < 3; d++) sp[d] = (T)dn[d][i];
       };
       rc = precision == RSG_FP64
-               ? make_keys<double, 1, 1>(h.get(), nn, entity, h->nkey_h, &h->nmat, &h->naxis, &h->n_nmat)
-               : make_keys<float, 1, 1>(h.get(), nn, entity, h->nkey_h, &h->nmat, &h->naxis, &h->n_nmat);
+               ? make_keys<double, 1, 1>(h.get(), nn, entity, h->nkey_h, &h->nmat, &h->naxis, &h->n_nmat, &h->n_naxis)
+               : make_keys<float, 1, 1>(h.get(), nn, entity, h->nkey_h, &h->nmat, &h->naxis, &h->n_nmat, &h->n_naxis);
       if (rc) return rc;
     }
     if (h->n_nmat < 0) {
@@ -2186,8 +2186,10 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
           for (int d = 0; d < 3; d++) sp[d] = (T)dc[d][i];
         };
         rc = precision == RSG_FP64
-                 ? make_keys<double, 21, rsg::kMatRow>(h.get(), nc, entity, h->ckey_h, &h->cmat, &h->caxis, &h->n_cmat)
-                 : make_keys<float, 21, rsg::kMatRow>(h.get(), nc, entity, h->ckey_h, &h->cmat, &h->caxis, &h->n_cmat);
+                 ? make_keys<double, 21, rsg::kMatRow>(h.get(), nc, entity, h->ckey_h, &h->cmat, &h->caxis, &h->n_cmat,
+                                                           &h->n_caxis)
+                 : make_keys<float, 21, rsg::kMatRow>(h.get(), nc, entity, h->ckey_h, &h->cmat, &h->caxis, &h->n_cmat,
+                                                           &h->n_caxis);
         if (rc) return rc;
       }
     }
@@ -2240,9 +2242,9 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
   };
   // Resident stepping where the tiles fit the GPU's LDS all at once (FP64 to about 350,000 cells,
   // FP32 to about 600,000) and the caller left the kernel choices to the library.  Measured per
-  // step against the two per-step kernels (us, aluminium blocks): 480 cells 9.7 -> 4.4 in FP64 and
-  // 9.4 -> 2.8 in FP32, 32,000 cells 10.7 -> 5.3 and 9.9 -> 4.3, 131,000 cells 13.3 -> 7.8 and
-  // 11.0 -> 5.0, 320,000 cells 22.4 -> 14.5 and 14.2 -> 8.6, 541,000 cells in FP32 20.4 -> 12.2.
+  // step against the two per-step kernels (us, aluminium blocks): 480 cells 8.9 -> 4.1 in FP64 and
+  // 8.3 -> 2.7 in FP32, 32,000 cells 9.7 -> 4.4 and 8.9 -> 3.5, 131,000 cells 12.8 -> 6.4 and
+  // 10.0 -> 4.5, 259,000 cells 18.2 -> 11.0 and 12.0 -> 6.9, 531,000 cells in FP32 20.4 -> 11.5.
   const bool chosen = tuning && (tuning->block_velocity || tuning->block_stress || tuning->per_thread_velocity ||
                                  tuning->per_thread_stress || tuning->lds_velocity || tuning->lds_stress);
   auto resident_part = [&]() -> int {
@@ -2262,8 +2264,9 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     auto run = [](int n, auto&& fn) { parallel_each(n, fn); };
     if (!rsg::build_resident_plan(m, max_tiles, lds, e, run, p)) return RSG_OK;
     // Threads past a tile's nodes still pay: other waves read the halo and take the cells (32,000
-    // cells in tiles of 125, 216 nodes: FP64 5.3 us a step with 256 threads, 4.6 with 512, FP32 4.3
-    // and 3.6; tiles of 64, 125 nodes: no difference).
+    // cells in tiles of 125, 216 nodes: FP64 5.0 us a step with 256 threads, 4.4 with 512, FP32 4.0
+    // and 3.5; tiles of 512, 729 nodes: 7.7 with 512, 6.4 with 1024, FP32 5.6 and 4.5; tiles of 64,
+    // 125 nodes: no difference).
     h->res_threads = p.max_node <= 128 ? 256 : p.max_node <= 512 ? 512 : 1024;
     h->res_nexp = p.nexp;
     h->res_set = p.max_set;
@@ -2276,16 +2279,17 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     if ((rc = upload(h.get(), &h->res_nrec, std::move(p.nrec)))) return rc;
     if ((rc = upload(h.get(), &h->res_halo, std::move(p.halo)))) return rc;
     if ((rc = upload(h.get(), &h->res_hcell, std::move(p.hcell)))) return rc;
-    if ((rc = upload(h.get(), &h->res_flag, std::vector<uint32_t>((size_t)tiles * rsg::kFlagStride, 0)))) return rc;
-    if ((rc = h->dalloc(&h->res_xbuf, (size_t)12 * p.nexp * e))) return rc;
+    if ((rc = h->dalloc(&h->res_xbuf, (size_t)24 * p.nexp * e))) return rc;
     // PANNDE_RSG_RESIDENT=alone (tests): the count of started tiles begins where it never meets a
     // launch's total, so every launch decides against its steps
     const char* alone = std::getenv("PANNDE_RSG_RESIDENT");
     const uint32_t started = alone && !strcmp(alone, "alone") ? 1u << 31 : 0;
     if ((rc = upload(h.get(), &h->res_ctrl, std::vector<uint32_t>{started, 0}))) return rc;
-    if (rsg::resident_lds_bytes(h->res_set, h->res_node, h->res_cell, e, true) + rsg::kResidentStaticLds > lds &&
-        (rc = h->dalloc(&h->res_work, (size_t)16 * tiles * (h->res_node + h->res_cell))))
-      return rc;
+    const bool records = rsg::resident_lds_bytes(h->res_set, h->res_node, h->res_cell, e, true) +
+                             rsg::kResidentStaticLds <= lds;
+    if (!records && (rc = h->dalloc(&h->res_work, (size_t)16 * tiles * (h->res_node + h->res_cell)))) return rc;
+    h->res_lds_room = lds - rsg::kResidentStaticLds -
+                      rsg::resident_lds_bytes(h->res_set, h->res_node, h->res_cell, e, records);
     h->res_tiles = tiles;
     return RSG_OK;
   };

@@ -208,7 +208,6 @@ struct ResidentTile {
 };
 constexpr uint32_t kResidentOwner = 0x80000000u;  // node record: this tile writes the node's results
 
-constexpr int kFlagStride = 32;                   // a flag per 128-byte line
 // Source terms: the special nodes (cells) with the same lists of channel terms share a class, and
 // the host sums each class's terms once per step, 3 (6) values a class: a row of 3 * node classes
 // + 6 * cell classes doubles.  Class numbers stay below 128.
@@ -227,14 +226,12 @@ struct ResidentArgs {
   const uint32_t* crec;  // [cells][4]: 8 x 12-bit local node indices, internal cell id
   const uint32_t* nrec;  // [tile nodes][4]: 8 x 12-bit local cell slots (own cells, halo, then the
                          // zero slot of missing cells), internal node id | kResidentOwner
-  const int2* halo;      // exchange slot and tile of each halo cell
+  const int32_t* halo;   // exchange slot of each halo cell
   const int32_t* hcell;  // internal id of each halo cell
-  unsigned long long* xbuf;  // [2][6 * sizeof(T) / 8][nexp]: exported stresses of even and odd steps
-  uint32_t* flag;        // [tiles][kFlagStride]: the step whose exported stresses are written
+  unsigned long long* xbuf;  // [4][6 * sizeof(T) / 8][nexp]: exported stresses of four steps in turn
   uint32_t* ctrl;        // [2]: tiles started, over all launches; the last decision (several tiles)
   uint32_t seq;          // number of the launch, from 1
   int32_t* status;       // [kResidentStatus], pinned
-  uint32_t epoch;        // the state's step, counted over the resident launches
   int32_t nsteps;        // >= 2
   int32_t ntiles;
   int32_t nexp;
@@ -248,15 +245,24 @@ struct ResidentArgs {
   const uint8_t* ccls;   // class of each special cell
   int32_t cforce0;       // first cell value of a force row
   int32_t row;           // doubles from one step's trace row to the next's
+  int32_t nmat;          // values of dt/rho in v.cls
+  int32_t tables;        // 1: the class tables' spacings and dt/rho are held in LDS
 };
+
+// The class tables in LDS, for meshes of at most kResidentClasses spacings along each axis and
+// values of dt/rho: node and cell spacings (FP64: with their reciprocals) and dt/rho.
+constexpr int kResidentClasses = 16;
+inline size_t resident_table_bytes(size_t elt) {
+  return kResidentClasses * ((size_t)6 * (elt == 8 ? 32 : 4) + elt);
+}
 
 // LDS of a tile's workgroup: its slots' stresses, its nodes' velocities, the marks and, with
 // `records`, the records; without, the kernel keeps those in `work`.
 inline size_t resident_lds_bytes(int max_set, int max_node, int max_cell, size_t elt, bool records) {
   const size_t state = ((size_t)6 * (max_set + 1) + (size_t)3 * max_node) * elt;
-  return (state + 15) / 16 * 16 + (size_t)(records ? 17 : 1) * (max_node + max_cell);
+  return ((state + 15) / 16 * 16 + (size_t)(records ? 17 : 1) * (max_node + max_cell) + 15) / 16 * 16;
 }
-constexpr size_t kResidentStaticLds = 2 * kResidentForces * 8 + 64;  // and what it declares itself
+constexpr size_t kResidentStaticLds = 2 * kResidentForces * 8 + 192;  // and what it declares itself
 
 // These launchers, and those of the state transfers, live in the kernel library only: builds of
 // the host code without it step with the per-step kernels and reorder states on the host.

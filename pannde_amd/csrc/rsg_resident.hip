@@ -14,17 +14,28 @@
 //   4. updates the cells that other tiles read, publishing each, then the rest.
 //
 // Exchange across the XCDs' separate L2s: the words are written and read with agent-scope
-// relaxed atomics.  The waves that write exported cells wait until their stores are out, and the
-// last of them sets the tile's flag to the step; a reader loads a cell's words after it has seen
-// the flag of the cell's tile.  The stresses after step g go to buffer g % 2: a tile that has the
-// whole halo of step g knows that its neighbours have finished step g and so have read g - 1.
-// Each flag has a cache line of its own, which only its readers poll.
+// relaxed atomics, and a word's arrival is its own signal: every word is kEmptyWord until it is
+// written, and a reader loads a cell's words until none is empty, so a step has one trip through
+// memory (store, load) between two tiles.  (A flag per tile instead, set when its stores are out
+// and read before the words, made it three: see the figures below.)
+// The stresses before step k of a launch are in buffer k % 4.  A tile that has its whole halo of
+// step k - 1 knows that its neighbours, the readers of its cells, are done with k - 2's; at the
+// start of step k it empties that buffer for k + 2 and waits for these stores before it publishes
+// k + 1, so a reader that has a cell's words of k + 1 finds those of k + 2 empty or written.  All
+// buffers are emptied before the workgroups agree on the start.
 //
-// What bounds it: up to some 30,000 cells the exchange (store, flag, load: about 1.7 us a step) and
-// the dependent latency of two updates; above, the FP64 arithmetic and the LDS reads of a tile
-// (24 reads of 16 bytes a node).  Every byte of state stays on the chip, so memory does not.
-// Aluminium block of 32,000 cells on an MI355X: 10.7 us a step with the per-step kernels, 5.3 here
-// (FP64), 9.9 and 4.3 (FP32).
+// A step reads memory for nothing but its halo: the class tables are in LDS, FP64 with reciprocals
+// of the spacings (see Recip), because a load in an update waits behind the exchange's stores.
+//
+// What bounds it: up to some 30,000 cells the trip of the exchange and the dependent latency of two
+// updates (node and cell about 2,000 cycles each, with a wave or two per SIMD); above, the
+// arithmetic and the LDS reads of a tile (24 reads of 16 bytes a node).  Every byte of state stays
+// on the chip, so memory does not.  Aluminium blocks on an MI355X, us a step FP64 / FP32, with the
+// per-step kernels, with a flag per tile, spacings through the caches and IEEE divisions, and now:
+// 480 cells 8.9/8.3, 4.5/2.8, 4.1/2.7; 32,000 cells 9.7/8.9, 4.5/3.6, 4.4/3.5; 131,000 cells
+// 12.8/10.0, 7.4/4.9, 6.4/4.5; 259,000 cells 18.2/12.0, 12.3/7.9, 11.0/6.9.
+// (Three lanes to a node and a cell, each with a third of the differences, gained nothing: 32,000
+// cells 4.3 us, 3.6 in FP32; the LDS reads and their latency remain.)
 //
 // The workgroups wait for each other, so they must all be on the GPU at once.  There are no more
 // of them than compute units, and the host lets one resident launch run at a time, but another
@@ -34,6 +45,8 @@
 // steps of such a one by itself, slowly, and tells the host not to try again.  (A cooperative
 // launch would see to it too, but costs 20 us and the host's wait for it, and on ROCm 7 its queue
 // slows the streams created after it: a batch's two lanes took 5.4 ms for 2.0 ms of work.)
+#include <type_traits>
+
 #include "rsg_device.h"
 
 namespace rsg {
@@ -82,6 +95,10 @@ __device__ __forceinline__ void unpack12(const v4u& w, int (&c)[8]) {
 }
 
 typedef unsigned long long word;
+// What an exchange word holds until it is written: a NaN (two, in FP32) that no arithmetic gives.
+// A stress that a caller gave these very bits is sent with another payload.
+constexpr word kEmptyWord = 0xFFFADE17FFFADE17ull;
+__device__ __forceinline__ word sent(word w) { return w == kEmptyWord ? w ^ 1 : w; }
 __device__ __forceinline__ void put_word(word* p, word w) {
   __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -103,6 +120,8 @@ struct Packed {
       for (int k = 0; k < 3; k++)
         w[k] = (word)__float_as_uint(o[2 * k]) | ((word)__float_as_uint(o[2 * k + 1]) << 32);
     }
+#pragma unroll
+    for (int k = 0; k < kWords; k++) w[k] = sent(w[k]);
   }
   __device__ __forceinline__ void unpack(T (&o)[6]) const {
     if constexpr (sizeof(T) == 8) {
@@ -127,13 +146,22 @@ __device__ __forceinline__ void put_slot(T* S, int i, const T (&v)[6]) {
   for (int p = 0; p < 3; p++) q[p] = P{v[2 * p], v[2 * p + 1]};
 }
 
-// Waits until every lane's flag (nullptr: none) has reached `want`; false when the wait ran out
-// (here or in another workgroup).
-__device__ __forceinline__ bool wait_flags(const uint32_t* flag, uint32_t want, int32_t* status) {
+// Loads the words of the exchanged cell at x (`on`: the lane has one), as often as it takes until
+// every lane of the wave has its whole cell; false when the wait ran out (here or in another
+// workgroup).
+template <typename T>
+__device__ __forceinline__ bool fetch_cell(const word* x, int nexp, bool on, int32_t* status, Packed<T>& w) {
   uint64_t t0 = 0;
   for (uint32_t spin = 1;; spin++) {
-    const uint32_t f = flag ? __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : want;
-    if (__all((int32_t)(f - want) >= 0)) return true;
+    if (on) {
+      bool full = true;
+#pragma unroll
+      for (int q = 0; q < Packed<T>::kWords; q++) w.w[q] = get_word(x + q * (size_t)nexp);
+#pragma unroll
+      for (int q = 0; q < Packed<T>::kWords; q++) full &= w.w[q] != kEmptyWord;
+      on = !full;
+    }
+    if (!__any(on)) return true;
     if ((spin & 1023u) == 0) {
       const uint64_t t = wall_clock64();
       if (t0 == 0) t0 = t;
@@ -152,6 +180,11 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
   typedef T P __attribute__((ext_vector_type(2)));
   T* const S = reinterpret_cast<T*>(smem);  // [max_set + 1][6]: own cells, halo, zero
   T* const V = S + 6 * (a.max_set + 1);     // [max_node][3]
+  // spacings with their reciprocals in FP64
+  using Sp = typename std::conditional<sizeof(T) == 8, Recip, float>::type;
+  struct alignas(sizeof(T) == 8 ? 16 : 4) Entry {
+    Sp s;
+  };
   unsigned char* const rest = smem + ((6 * (a.max_set + 1) + 3 * a.max_node) * sizeof(T) + 15) / 16 * 16;
   // records: 8 x 12-bit links, then the key (or the id, for per-entity coefficients)
   v4u* nrec;
@@ -163,12 +196,19 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
   // marks of the special nodes and cells: 1 + the class of their source terms, a node's sensor
   uint8_t* const nmark = REC ? reinterpret_cast<uint8_t*>(crec + a.max_cell) : rest;
   uint8_t* const cmark = nmark + a.max_node;
+  // the class tables: spacings of the nodes and the cells ([axis][class]), then dt/rho
+  unsigned char* const after = cmark + a.max_cell;
+  Entry* const naxis = reinterpret_cast<Entry*>(smem + ((after - smem) + 15) / 16 * 16);
+  Entry* const caxis = naxis + 3 * kResidentClasses;
+  T* const ncls = reinterpret_cast<T*>(caxis + 3 * kResidentClasses);
   __shared__ double force[2][kResidentForces];  // of the even and the odd steps
-  __shared__ int sensors;  // the tile records some
-  __shared__ int published;  // waves that have published a step's exported cells, over all steps
+  // the tile's sensors, slot << 12 | node; more than the list holds are looked up every step
+  constexpr int kListed = 32;
+  __shared__ int sensors;
+  __shared__ uint32_t sensor[kListed];
   const ResidentTile tl = a.tiles[blockIdx.x];
   const int t = threadIdx.x;
-  const int rt = t ^ (THREADS - 64);  // the waves in reverse order
+  const int rt = THREADS - 64 - (t & ~63) + (t & 63);  // the waves in reverse order
 
   T* const Sg[6] = {a.s.S0, a.s.S1, a.s.S2, a.s.S3, a.s.S4, a.s.S5};
   auto load_stress = [&](int e, int slot) {
@@ -178,14 +218,31 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
     put_slot(S, slot, o);
   };
   __shared__ int go;  // the launch's steps are made
+  constexpr int W = Packed<T>::kWords;
+  const size_t xstep = (size_t)W * a.nexp;  // words of an exchange buffer
+  auto empty = [&](word* x) {
+    for (int i = t; i < tl.nexp; i += THREADS)
+#pragma unroll
+      for (int q = 0; q < W; q++) put_word(x + q * (size_t)a.nexp + i, kEmptyWord);
+  };
   bool last = false;
+  for (int b = 0; b < 4; b++) empty(a.xbuf + b * xstep + tl.exp0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
   if (t == 0) {
-    sensors = published = 0;
+    sensors = 0;
     if (a.ntiles > 1)
       last = __hip_atomic_fetch_add(a.ctrl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 ==
              a.seq * (uint32_t)a.ntiles;
   }
   __syncthreads();
+  if (a.tables && t < 3 * kResidentClasses) {
+    const int at = t / kResidentClasses * kAxisClasses + t % kResidentClasses;
+    if constexpr (NKEY) set_spacing(a.v.axis[at], naxis[t].s);
+    if constexpr (CKEY) set_spacing(a.s.axis[at], caxis[t].s);
+    if constexpr (NKEY)
+      if (t < a.nmat) ncls[t] = a.v.cls[t];
+  }
   for (int i = t; i < tl.ncell; i += THREADS) {
     v4u r = reinterpret_cast<const v4u*>(a.crec)[tl.cell0 + i];
     const int e = (int)r.w;
@@ -220,7 +277,9 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
       mark = a.ncls[sp] + 1;
       if (owner && a.v.sp_sens[sp] >= 0) {
         mark |= kResidentSensor;
-        sensors = 1;
+        const uint32_t slot = (uint32_t)a.v.sp_sens[sp];
+        const int at = atomicAdd(&sensors, slot < 1u << 20 ? 1 : kListed + 1);
+        if (at < kListed) sensor[at] = slot << 12 | (uint32_t)i;
       }
     }
     nrec[i] = r;
@@ -230,35 +289,43 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
     V[3 * i + 2] = a.v.V2[n];
   }
   if (t < 6) S[6 * (tl.ncell + tl.nhalo) + t] = T(0);  // where the links to missing cells point
-  constexpr int W = Packed<T>::kWords;
-  const int2 none = {0, 0};
-  const int2 first = rt < tl.nhalo ? a.halo[tl.halo0 + rt] : none;  // exchange slot, tile
-  // waves that publish exported cells each step
-  const int pub_waves = min((tl.nexp + 63) / 64, THREADS / 64);
+  const int first = rt < tl.nhalo ? a.halo[tl.halo0 + rt] : 0;  // exchange slot
 
   const VelocityArgs<T>& va = a.v;
   const StressArgs<T>& sa = a.s;
   const double* now = force[0];  // this step's source terms
+  // spacings of class key k, from LDS or through the caches
+  auto spacings = [&](const Entry* table, const T* axis, uint32_t k, Sp (&sp)[3]) {
+    if (a.tables) {
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+        sp[d] = table[d * kResidentClasses + ((k >> (14 - 7 * d)) & (kResidentClasses - 1))].s;
+    } else {
+      T x[3];
+      axis_spacings(axis, k, x[0], x[1], x[2]);
+#pragma unroll
+      for (int d = 0; d < 3; d++) set_spacing(x[d], sp[d]);
+    }
+  };
   auto node_update = [&](int i) {
     const v4u rec = nrec[i];
-    T idt, sx, sy, sz;
+    T idt;
+    Sp sp[3];
     bool special = false;
     if constexpr (NKEY) {
       special = rec.w & kSpecialKey;
       const uint32_t k = rec.w & ~kSpecialKey;
-      const uint32_t k0 = __builtin_amdgcn_readfirstlane(k);
-      if (__all(k == k0)) {
-        idt = as_const(va.cls)[k0 >> kMatShift];
-        axis_spacings(as_const(va.axis), k0, sx, sy, sz);
-      } else {
-        idt = va.cls[k >> kMatShift];
-        axis_spacings(va.axis, k, sx, sy, sz);
-      }
+      spacings(naxis, va.axis, k, sp);
+      // (one read from a chosen address would be a flat load, which waits for all others)
+      if (a.tables)
+        idt = ncls[k >> kMatShift];
+      else
+        idt = as_const(va.cls)[k >> kMatShift];
     } else {
       idt = va.idt[rec.w];
-      sx = va.dnx[rec.w];
-      sy = va.dny[rec.w];
-      sz = va.dnz[rec.w];
+      set_spacing(va.dnx[rec.w], sp[0]);
+      set_spacing(va.dny[rec.w], sp[1]);
+      set_spacing(va.dnz[rec.w], sp[2]);
       if (is_boxed(idt)) {
         special = true;
         idt = va.sp_idt[unbox(idt)];
@@ -269,6 +336,9 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
     T r[3];
     node_rates(
         [&](int p, T(&f)[8], T(&g)[8]) {
+          // one pair's reads at a time: all three do not fit the 128 registers of 1024 threads (and
+          // spilling them cost 259,000 cells 13.7 us a step against 11.0)
+          if constexpr (sizeof(T) == 8 && THREADS == 1024) asm volatile("" ::: "memory");
           const P* q = reinterpret_cast<const P*>(S) + p;
 #pragma unroll
           for (int k = 0; k < 8; k++) {
@@ -277,7 +347,7 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
             g[k] = w.y;
           }
         },
-        sx, sy, sz, r);
+        sp, r);
     if (special) {
       const double* f = now + 3 * ((nmark[i] & ~kResidentSensor) - 1);
 #pragma unroll
@@ -299,14 +369,16 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
     const v4u rec = crec[i];
     int c[8];
     unpack12(rec, c);
-    T s[6];
+    T s[6], d[6];
+    auto own = [&]() {  // after the differences, which need the registers
+      asm volatile("" ::: "memory");
 #pragma unroll
-    for (int p = 0; p < 3; p++) {
-      const P w = reinterpret_cast<const P*>(S)[3 * i + p];
-      s[slot_comp(2 * p)] = w.x;
-      s[slot_comp(2 * p + 1)] = w.y;
-    }
-    T d[6];
+      for (int p = 0; p < 3; p++) {
+        const P w = reinterpret_cast<const P*>(S)[3 * i + p];
+        s[slot_comp(2 * p)] = w.x;
+        s[slot_comp(2 * p + 1)] = w.y;
+      }
+    };
     double m[6] = {0, 0, 0, 0, 0, 0};
     int sp = -1;
     auto xy = [&](T(&f)[8], T(&g)[8]) {
@@ -320,26 +392,31 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
 #pragma unroll
       for (int k = 0; k < 8; k++) f[k] = V[3 * c[k] + 2];
     };
+    Sp sd[3];
     if constexpr (CKEY) {
       if (rec.w & kSpecialKey) sp = 0;
       const uint32_t k = rec.w & ~kSpecialKey;
-      const uint32_t k0 = __builtin_amdgcn_readfirstlane(k);
-      T sx, sy, sz;
-      if (__all(k == k0))
-        axis_spacings(as_const(sa.axis), k0, sx, sy, sz);
-      else
-        axis_spacings(sa.axis, k, sx, sy, sz);
+      spacings(caxis, sa.axis, k, sd);
+      // the first lane's material row is requested before the differences need it
       const uint32_t mat = k >> kMatShift;
-      uint32_t m0 = k0 >> kMatShift;
-      strain_rates<T>(xy, z, sx, sy, sz, d);
+      uint32_t m0 = __builtin_amdgcn_readfirstlane(mat);
+      const auto row0 = as_const(sa.cls + (size_t)m0 * kMatRow);
+      T c0[21];
+#pragma unroll
+      for (int q = 0; q < 21; q++) c0[q] = row0[q];
+      strain_rates(xy, z, sd, d);
+      own();
       moments(i, sp, m);
-      // one pass per distinct material of the wavefront, its row through the scalar cache
-      for (;;) {
-        if (mat == m0) {
-          voigt_update(sa.dt, as_const(sa.cls + (size_t)m0 * kMatRow), d, m, sp, s);
-          break;
+      if (__all(mat == m0)) {
+        voigt_update(sa.dt, c0, d, m, sp, s);
+      } else {  // one pass per distinct material of the wavefront
+        for (;;) {
+          if (mat == m0) {
+            voigt_update(sa.dt, as_const(sa.cls + (size_t)m0 * kMatRow), d, m, sp, s);
+            break;
+          }
+          m0 = __builtin_amdgcn_readfirstlane(mat);
         }
-        m0 = __builtin_amdgcn_readfirstlane(mat);
       }
     } else {
       const int e = (int)rec.w;
@@ -353,7 +430,11 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
         sp = 0;
         sx = sa.sp_dcx[unbox(sx)];
       }
-      strain_rates<T>(xy, z, sx, sy, sz, d);
+      set_spacing(sx, sd[0]);
+      set_spacing(sy, sd[1]);
+      set_spacing(sz, sd[2]);
+      strain_rates(xy, z, sd, d);
+      own();
       moments(i, sp, m);
       voigt_update(sa.dt, cc, d, m, sp, s);
     }
@@ -378,22 +459,19 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
       if (k + 1 < a.nsteps) f0 = a.force[(size_t)(k + 1) * a.nforce + t];
     }
     __syncthreads();  // the step before's stresses are in LDS, and its velocities are read
+    if (k > 2 && k + 2 < a.nsteps) empty(a.xbuf + ((k + 2) % 4) * xstep + tl.exp0);
 #pragma unroll 1
     for (int i = t; i < tl.nown; i += THREADS) node_update(i);
     if (tl.nhalo > 0) {
       if (k > 0) {
-        const word* x = a.xbuf + (size_t)((a.epoch + k) & 1) * a.nexp * W;
+        const word* x = a.xbuf + (k % 4) * xstep;
         for (int i = rt; (i & ~63) < tl.nhalo; i += THREADS) {
           const bool on = i < tl.nhalo;
-          const int2 h = i == rt || !on ? first : a.halo[tl.halo0 + i];
-          if (alive)
-            alive = wait_flags(on ? a.flag + (size_t)kFlagStride * h.y : nullptr, a.epoch + (uint32_t)k, a.status);
-          asm volatile("" ::: "memory");  // the loads below stay behind the wait
+          const int h = i == rt || !on ? first : a.halo[tl.halo0 + i];
+          Packed<T> w = {};
+          if (alive) alive = fetch_cell<T>(x + h, a.nexp, on, a.status, w);
           if (on) {
-            Packed<T> w;
             T o[6];
-#pragma unroll
-            for (int q = 0; q < W; q++) w.w[q] = get_word(x + q * (size_t)a.nexp + h.x);
             w.unpack(o);
             put_slot(S, tl.ncell + i, o);
           }
@@ -403,9 +481,10 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
 #pragma unroll 1
       for (int i = tl.nown + t; i < tl.nnode; i += THREADS) node_update(i);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied words are out
     __syncthreads();  // the velocities are in LDS, and the stresses are read
     const bool publish = k + 1 < a.nsteps;  // the last step's stresses go to the state alone
-    word* const x = a.xbuf + (size_t)((a.epoch + k + 1) & 1) * a.nexp * W + tl.exp0;
+    word* const x = a.xbuf + ((k + 1) % 4) * xstep + tl.exp0;
 #pragma unroll 1
     for (int i = t; i < tl.nexp; i += THREADS) {
       T o[6];
@@ -417,19 +496,20 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
         for (int q = 0; q < W; q++) put_word(x + q * (size_t)a.nexp + i, w.w[q]);
       }
     }
-    if (publish && tl.nexp > (t & ~63)) {
-      // the wave whose stores are the last to be out sets the flag
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if ((t & 63) == 0 && atomicAdd(&published, 1) == (k + 1) * pub_waves - 1)
-        __hip_atomic_store(a.flag + (size_t)kFlagStride * blockIdx.x, a.epoch + (uint32_t)k + 1u, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
 #pragma unroll 1
     for (int i = tl.nexp + rt; i < tl.ncell; i += THREADS) {
       T o[6];
       cell_update(i, o);
     }
-    if (sensors)  // this step's velocities stay in LDS until the next barrier
+    // this step's velocities stay in LDS until the next barrier
+    if (sensors <= kListed) {
+      if (rt < sensors) {
+        const uint32_t w = sensor[rt];
+        double* out = va.trace + (size_t)k * a.row + 3 * (w >> 12);
+#pragma unroll
+        for (int d = 0; d < 3; d++) out[d] = (double)V[3 * (w & 0xFFF) + d];
+      }
+    } else {
       for (int i = rt; i < tl.nnode; i += THREADS)
         if (nmark[i] & kResidentSensor) {
           const int n = (int)(a.nrec[4 * (size_t)(tl.node0 + i) + 3] & ~kResidentOwner);
@@ -442,6 +522,7 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
 #pragma unroll
           for (int d = 0; d < 3; d++) out[d] = (double)V[3 * i + d];
         }
+    }
   }
   __syncthreads();
 
@@ -596,7 +677,8 @@ hipError_t launch_resident(const ResidentArgs<T>& a, int threads, hipStream_t st
                    : threads == 1024 ? resident_fn<T, 1024>(nkey, ckey, rec)
                                      : nullptr;
   if (!fn) return hipErrorInvalidValue;
-  const size_t lds = resident_lds_bytes(a.max_set, a.max_node, a.max_cell, sizeof(T), rec);
+  const size_t lds = resident_lds_bytes(a.max_set, a.max_node, a.max_cell, sizeof(T), rec) +
+                     (a.tables ? resident_table_bytes(sizeof(T)) : 0);
   void* args[1] = {const_cast<void*>(static_cast<const void*>(&a))};
   const hipError_t e = hipLaunchKernel(fn, dim3(a.ntiles), dim3(threads), args, lds, st);
   if (e != hipSuccess || a.ntiles == 1) return e;

@@ -27,8 +27,7 @@ struct ResidentMesh {
 struct ResidentPlan {
   std::vector<ResidentTile> tiles;
   std::vector<uint32_t> crec, nrec;
-  std::vector<int2> halo;
-  std::vector<int32_t> hcell;
+  std::vector<int32_t> halo, hcell;
   int32_t nexp = 0, max_set = 0, max_node = 0, max_cell = 0;
 };
 
@@ -184,8 +183,7 @@ bool build_resident_plan(const ResidentMesh& m, int32_t max_tiles, size_t lds_li
   p.crec.resize((size_t)m.nc * 4);
   struct Part {
     std::vector<uint32_t> nrec;
-    std::vector<int2> halo;
-    std::vector<int32_t> hcell;
+    std::vector<int32_t> halo, hcell;
   };
   std::vector<Part> parts(nt);
   const int groups = (int)std::min<int32_t>(nt, std::min<int64_t>(8, ((int64_t)m.nc + (1 << 14) - 1) / (1 << 14)));
@@ -222,7 +220,7 @@ bool build_resident_plan(const ResidentMesh& m, int32_t max_tiles, size_t lds_li
       std::sort(around.begin(), around.end());
       for (auto& x : around) {
         cell_tag[x.second] = stamp | (int64_t)(tl.ncell + part.halo.size());
-        part.halo.push_back(int2{x.first, tile_of[x.second]});
+        part.halo.push_back(x.first);
         part.hcell.push_back(m.cell_at[x.second]);
       }
       tl.nhalo = (int32_t)part.halo.size();

@@ -1,7 +1,7 @@
 // resident_stub.cpp -- the resident kernel's and the state transfers' launchers on the CPU, over the host stand-ins for the
 // HIP runtime (hip_host_stub.cpp).  TEST INFRASTRUCTURE ONLY: it walks the tiles, records, halo and
 // exchange slots exactly as the kernel does (each tile with its own copy of its slots and nodes, the
-// exported stresses through the double-buffered exchange), with every index checked, so a plan that
+// exported stresses through the four-buffer exchange), with every index checked, so a plan that
 // steps a mesh correctly here gives the kernel the right data.
 #include <hip/hip_runtime_api.h>
 
@@ -81,17 +81,20 @@ hipError_t run(const ResidentArgs<T>& a, int threads) {
       for (int d = 0; d < 3; d++) V[t][3 * i + d] = Vg[d][n];
     }
   }
+  std::fill(xb, xb + (size_t)24 * a.nexp, T(NAN));  // empty
   for (int k = 0; k < a.nsteps; k++) {
     const double* force = a.force + (size_t)k * a.nforce;
     for (int t = 0; t < a.ntiles; t++) {
       const ResidentTile& tl = a.tiles[t];
       if (k > 0)
         for (int i = 0; i < tl.nhalo; i++) {
-          const int x = a.halo[tl.halo0 + i].x, o = a.halo[tl.halo0 + i].y;
-          CHECK(o >= 0 && o < a.ntiles && x >= a.tiles[o].exp0 && x < a.tiles[o].exp0 + a.tiles[o].nexp);
-          CHECK(a.flag[(size_t)kFlagStride * o] == a.epoch + (uint32_t)k);
-          for (int q = 0; q < 6; q++) S[t][6 * (tl.ncell + i) + q] = xb[at(a, (a.epoch + k) & 1, x, q)];
+          const int x = a.halo[tl.halo0 + i];
+          CHECK(x >= 0 && x < a.nexp && (x < tl.exp0 || x >= tl.exp0 + tl.nexp));
+          for (int q = 0; q < 6; q++) S[t][6 * (tl.ncell + i) + q] = xb[at(a, k % 4, x, q)];
         }
+      if (k > 2 && k + 2 < a.nsteps)
+        for (int x = tl.exp0; x < tl.exp0 + tl.nexp; x++)
+          for (int q = 0; q < 6; q++) xb[at(a, (k + 2) % 4, x, q)] = T(NAN);
       for (int i = 0; i < tl.nnode; i++) {
         const uint32_t* r = &a.nrec[4 * (size_t)(tl.node0 + i)];
         const int n = (int)(r[3] & ~kResidentOwner);
@@ -188,10 +191,9 @@ hipError_t run(const ResidentArgs<T>& a, int threads) {
             if (special >= 0) acc = acc + (T)((double)a.s.dt * m);
             s = s + acc;
           }
-          if (i < tl.nexp && k + 1 < a.nsteps) xb[at(a, (a.epoch + k + 1) & 1, tl.exp0 + i, q)] = s;
+          if (i < tl.nexp && k + 1 < a.nsteps) xb[at(a, (k + 1) % 4, tl.exp0 + i, q)] = s;
         }
       }
-      if (k + 1 < a.nsteps) a.flag[(size_t)kFlagStride * t] = a.epoch + (uint32_t)k + 1;
     }
   }
   std::vector<char> cell(a.s.n, 0), node(a.v.n, 0);

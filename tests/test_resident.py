@@ -163,3 +163,43 @@ def test_resident_at_its_largest(precision, dims):
     ref = run(case, precision, dict(block_velocity=256, block_stress=256), [300])
     got = run(case, precision, None, [300])
     assert all(np.array_equal(a, b) for a, b in zip(got, ref))
+
+
+def graded_mesh(classes, scale):
+    """A block of 260 x 6 x 5 cells with `classes` spacings along x, its lengths times `scale`."""
+    case = cases.al_block(seed=8, nx=260, ny=6, nz=5, nsteps=6, n_sensors=3)
+    rng = np.random.default_rng(classes)
+    widths = rng.choice(rng.uniform(0.6e-4, 2.0e-4, classes), 260)
+    case.x = np.concatenate([[0.0], np.cumsum(widths)])[np.rint(case.x / 1e-4).astype(int)] * scale
+    case.y, case.z = case.y * scale, case.z * scale
+    case.force = []
+    return case
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [rsg.RSG_FP64, rsg.RSG_FP32])
+@pytest.mark.parametrize("classes,scale", [(1, 1.0), (5, 1.0), (40, 1.0), (260, 1.0), (5, 1e-17), (1, 2.0 ** 70)])
+def test_quotients_of_any_size(classes, scale, precision):
+    """Spacings from the LDS tables, the caches and per-node arrays, usual and not, and states whose
+    values lie anywhere between the denormals and infinity: each difference quotient is the rounded
+    quotient of the per-step kernels (and the oracle)."""
+    case = graded_mesh(classes, scale)
+    rng = np.random.default_rng(3)
+    nn, nc = case.x.shape[0], case.cells.shape[0]
+    top = 1000 if precision == rsg.RSG_FP64 else 100
+    for low, special in ((-1074, False), (-1000, False), (-900, True), (0, True)):
+        V, S = (rng.uniform(-2, 2, (k, n)) * 2.0 ** rng.integers(max(low, -1070), top if low == 0 else low + 200, (k, n))
+                for k, n in ((3, nn), (6, nc)))
+        for a in (V, S):
+            a[rng.random(a.shape) < 0.3] = 0.0
+            if special:
+                a[rng.random(a.shape) < 1e-3] = np.inf
+                a[rng.random(a.shape) < 1e-3] = np.nan
+        out = []
+        for tuning in (dict(block_velocity=256, block_stress=256), None):
+            s = rsg.DeviceSolver.from_case(case, precision, tuning=tuning)
+            s.set_state(V, S)
+            s.solve(6)
+            out.append(s.get_state() + (s.traces(),))
+            s.close()
+        assert all(np.array_equal(a, b, equal_nan=True) for a, b in zip(*out)), low
