@@ -254,6 +254,7 @@ void leave_resident_order(const rsg_instance* h) {
   for (auto it = o.last.begin(); it != o.last.end();) it = it->second == h ? o.last.erase(it) : std::next(it);
 }
 
+constexpr int64_t kCacheBytes = (int64_t)256 << 20;  // the GPU's memory-side cache
 constexpr int kBlockSteps = 256;   // steps whose amplitudes are staged per upload
 constexpr int kTraceCapSteps = 4096;
 
@@ -269,6 +270,7 @@ struct rsg_instance {
   int block_v = 256, block_s = 256;
   int cpt_v = 1, cpt_s = 1;       // entities per thread
   int stream_v = 1, stream_s = 1;  // non-temporal loads of what a step reads once
+  int64_t once_v = 0, once_s = 0;  // its bytes, per kernel
   bool in_batch = false;          // stepped by a batch, not by rsg_step
   hipStream_t batch_stream = nullptr;  // the batch's stream while in_batch
   int xcd = 1;                    // XCD-contiguous workgroup remap
@@ -2343,14 +2345,14 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
   // 2.6 M FP64 (186 + 42 + 41) 131 / 121 / 132; the plate FP32 (140 + 64 + 62) 96 / 93 / 102 and
   // FP64 (280 + 64 + 62) 184 / 187 / 191; a graded part of 0.45 M FP64 (33 + 7 + 94) 41 / 40 / 39.
   {
-    const int64_t e = (int64_t)h->elt(), room = (int64_t)256 << 20, cache = room - room / 10;
+    const int64_t e = (int64_t)h->elt(), cache = kCacheBytes - kCacheBytes / 10;
     const int64_t state = e * (3 * (int64_t)nn + 6 * (int64_t)nc);
-    const int64_t once_v = (int64_t)nn * ((h->v_lkey || h->v_lconn ? 16 : 32) + (h->nkey ? 4 : 0)) + h->v_list_bytes +
+    h->once_v = (int64_t)nn * ((h->v_lkey || h->v_lconn ? 16 : 32) + (h->nkey ? 4 : 0)) + h->v_list_bytes +
                            (h->n_nmat < 0 ? 4 * e * nn : 0);
-    const int64_t once_s = (int64_t)nc * ((h->s_lkey || h->s_lconn ? 16 : 32) + (h->ckey ? 4 : 0)) + h->s_list_bytes +
+    h->once_s = (int64_t)nc * ((h->s_lkey || h->s_lconn ? 16 : 32) + (h->ckey ? 4 : 0)) + h->s_list_bytes +
                            (h->n_cmat < 0 ? 24 * e * nc : 0);
-    h->stream_v = state + once_v > cache;
-    h->stream_s = state + once_v + once_s > cache;
+    h->stream_v = state + h->once_v > cache;
+    h->stream_s = state + h->once_v + h->once_s > cache;
   }
   CREATE_PHASE("arrays");
   // zero state (TransducerModel.cpp:150-159)
@@ -2704,11 +2706,12 @@ struct rsg_batch_s {
     bool lds_v, lds_s;         // LDS staging
     int32_t max_u_v, max_u_s;  // largest staged set of a member
     int32_t block_v, block_s, cpt_v, cpt_s;  // the members' workgroup sizes and per-thread counts
+    bool stream;               // non-temporal loads of what a step reads once
     bool operator==(const Launch& o) const {
       return off_v == o.off_v && off_s == o.off_s && n_v == o.n_v && n_s == o.n_s && grid_v == o.grid_v &&
              grid_s == o.grid_s && km_v == o.km_v && km_s == o.km_s && lds_v == o.lds_v && lds_s == o.lds_s &&
              max_u_v == o.max_u_v && max_u_s == o.max_u_s && block_v == o.block_v && block_s == o.block_s &&
-             cpt_v == o.cpt_v && cpt_s == o.cpt_s;
+             cpt_v == o.cpt_v && cpt_s == o.cpt_s && stream == o.stream;
     }
   };
   struct Lane {
@@ -2902,16 +2905,16 @@ int batch_launch_block(rsg_batch_s* b, rsg_batch_s::Lane& ln) {
         hipError_t e;
         if (sizeof(T) == 8) {
           e = rsg::launch_batch_f64((const rsg::BatchDesc<double>*)desc, wv + g.off_v, g.n_v, k, g.grid_v, g.block_v,
-                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, true, ln.stream, graph, node);
+                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, g.stream, true, ln.stream, graph, node);
           if (e != hipSuccess) return e;
           e = rsg::launch_batch_f64((const rsg::BatchDesc<double>*)desc, ws + g.off_s, g.n_s, k, g.grid_s, g.block_s,
-                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, false, ln.stream, graph, node);
+                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, g.stream, false, ln.stream, graph, node);
         } else {
           e = rsg::launch_batch_f32((const rsg::BatchDesc<float>*)desc, wv + g.off_v, g.n_v, k, g.grid_v, g.block_v,
-                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, true, ln.stream, graph, node);
+                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, g.stream, true, ln.stream, graph, node);
           if (e != hipSuccess) return e;
           e = rsg::launch_batch_f32((const rsg::BatchDesc<float>*)desc, ws + g.off_s, g.n_s, k, g.grid_s, g.block_s,
-                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, false, ln.stream, graph, node);
+                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, g.stream, false, ln.stream, graph, node);
         }
         if (e != hipSuccess) return e;
       }
@@ -3016,6 +3019,10 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
       const auto f = config(b->slots[i].h);
       if (std::find(configs.begin(), configs.end(), f) == configs.end()) configs.push_back(f);
     }
+  int32_t busy_lanes = 0;
+  for (int q = 0; q < rsg_batch_s::kMaxLanes; q++)
+    busy_lanes += std::any_of(b->slots.begin(), b->slots.end(),
+                              [&](const rsg_batch_s::Slot& sl) { return active(sl) && sl.lane == q; });
   ln.layout.clear();
   size_t ov = 0, os = 0;
   std::vector<size_t> members;
@@ -3024,7 +3031,7 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
     const int32_t cv = f[2] * f[4], cs = f[3] * f[5];
     for (size_t i = 0; i < b->slots.size();) {
       members.clear();
-      int64_t bytes = 0;
+      int64_t bytes = 0, once = 0;
       int32_t nv = 0, ns = 0;
       for (; i < b->slots.size(); i++) {
         if (!kmax[i]) continue;
@@ -3033,6 +3040,7 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
         const int64_t sb = state_bytes(b, h);
         if (!members.empty() && b->group_bytes > 0 && bytes + sb > b->group_bytes) break;
         bytes += sb;
+        once += h->once_v + h->once_s;
         members.push_back(i);
         nv += (h->nn + cv - 1) / cv;
         ns += (h->nc + cs - 1) / cs;
@@ -3084,6 +3092,12 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
       g.block_s = f[3];
       g.cpt_v = f[4];
       g.cpt_s = f[5];
+      // Links, keys and lists stay cached where the lanes' groups, this one's size each, do not
+      // exceed the memory-side cache by more than a third.  Measured, 2 lanes, us a step,
+      // non-temporal / cached by the two groups' MiB: FP32 105 57.6 / 51.3, 202 1023 / 922, 270 1003 /
+      // 925, 406 955 / 961, 540 941 / 1003; FP64 75 56.1 / 48.9, 298 888 / 857 and 313 / 295, 362
+      // 875 / 881.
+      g.stream = busy_lanes * (bytes + once) > kCacheBytes / 3 * 4;
       g.lds_v = lds_v;
       g.lds_s = lds_s;
       g.max_u_v = lds_v ? mu_v : 0;

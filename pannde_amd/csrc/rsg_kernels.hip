@@ -621,7 +621,7 @@ __global__ __launch_bounds__(RSG_MAX_BLOCK) RSG_STRESS_ATTR void stress_kernel(S
 // of different lengths stop exactly at their own step count.  The table and the
 // descriptors live in device memory, so a graph of these launches stays valid while
 // instances join and leave.
-template <typename T, bool LDS, int U, int CPT, int KM>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT>
 __device__ __forceinline__ void velocity_item(const BatchDesc<T>* __restrict__ desc, int2 it, int k,
                                               unsigned char* smem) {
   // the item carries the instance's step count for this block, so the branch needs no
@@ -631,43 +631,43 @@ __device__ __forceinline__ void velocity_item(const BatchDesc<T>* __restrict__ d
   VelocityArgs<T> a = d->v;
   a.amp = d->amp_base + (size_t)k * d->nch;
   a.trace = d->trace_base ? d->trace_base + (size_t)(d->trace_row0 + k) * d->row : nullptr;
-  velocity_body<T, LDS, U, CPT, KM, true>(a, it.y, smem);
+  velocity_body<T, LDS, U, CPT, KM, NT>(a, it.y, smem);
 }
 
-template <typename T, bool LDS, int U, int CPT, int KM>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT>
 __device__ __forceinline__ void stress_item(const BatchDesc<T>* __restrict__ desc, int2 it, int k,
                                             unsigned char* smem) {
   if (it.x < 0 || k >= (it.x >> kItemSlotBits)) return;
   const BatchDesc<T>* d = desc + (it.x & (kMaxBatchSlots - 1));
   StressArgs<T> a = d->s;
   a.amp = d->amp_base + (size_t)k * d->nch;
-  stress_body<T, LDS, U, CPT, KM, true>(a, it.y, smem);
+  stress_body<T, LDS, U, CPT, KM, NT>(a, it.y, smem);
 }
 
-template <typename T, bool LDS, int U, int CPT, int KM, bool PERSIST>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT, bool PERSIST>
 __global__ __launch_bounds__(RSG_MAX_BLOCK) RSG_VELOCITY_ATTR void velocity_batch_kernel(
     const BatchDesc<T>* __restrict__ desc, const int2* __restrict__ items, int n, int k) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (!PERSIST) {
-    if ((int)blockIdx.x < n) velocity_item<T, LDS, U, CPT, KM>(desc, items[blockIdx.x], k, smem);
+    if ((int)blockIdx.x < n) velocity_item<T, LDS, U, CPT, KM, NT>(desc, items[blockIdx.x], k, smem);
     return;
   }
   for (int p = blockIdx.x; p < n; p += gridDim.x) {
-    velocity_item<T, LDS, U, CPT, KM>(desc, items[p], k, smem);
+    velocity_item<T, LDS, U, CPT, KM, NT>(desc, items[p], k, smem);
     __syncthreads();  // the next item reuses the LDS
   }
 }
 
-template <typename T, bool LDS, int U, int CPT, int KM, bool PERSIST>
+template <typename T, bool LDS, int U, int CPT, int KM, bool NT, bool PERSIST>
 __global__ __launch_bounds__(RSG_MAX_BLOCK) RSG_STRESS_ATTR void stress_batch_kernel(
     const BatchDesc<T>* __restrict__ desc, const int2* __restrict__ items, int n, int k) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (!PERSIST) {
-    if ((int)blockIdx.x < n) stress_item<T, LDS, U, CPT, KM>(desc, items[blockIdx.x], k, smem);
+    if ((int)blockIdx.x < n) stress_item<T, LDS, U, CPT, KM, NT>(desc, items[blockIdx.x], k, smem);
     return;
   }
   for (int p = blockIdx.x; p < n; p += gridDim.x) {
-    stress_item<T, LDS, U, CPT, KM>(desc, items[p], k, smem);
+    stress_item<T, LDS, U, CPT, KM, NT>(desc, items[p], k, smem);
     __syncthreads();
   }
 }
@@ -719,7 +719,7 @@ hipError_t with_variant(bool lds, int max_u, int block, int cpt, int km, F&& f) 
 }
 
 // Kernel instances that also come with ordinary loads of the once-a-step data: the staged ones of
-// the default shapes.
+// the default shapes (and of a batch's default grid).
 constexpr bool cacheable(bool lds, int u, int cpt) { return lds && u > 0 && cpt <= 2; }
 
 template <typename T>
@@ -778,8 +778,8 @@ hipError_t launch_stress_f32(const StressArgs<float>& a, int block, hipStream_t 
 #if RSG_PART == 0 || RSG_PART >= 3
 template <typename T>
 hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, int k, int grid, int block,
-                        bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
-                        hipGraphNode_t* node) {
+                        bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
+                        hipGraph_t graph, hipGraphNode_t* node) {
   if (grid <= 0 || n <= 0) return hipSuccess;
   if (reinterpret_cast<uintptr_t>(table) % alignof(int2)) return hipErrorInvalidValue;
   const int2* items = reinterpret_cast<const int2*>(table);
@@ -789,10 +789,14 @@ hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, i
   return with_variant(lds, max_u, block, cpt, km, [&](auto L, auto U, auto C, auto K) {
     constexpr bool l = decltype(L)::value;
     constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
-    const void* fn = velocity ? (persist ? reinterpret_cast<const void*>(&velocity_batch_kernel<T, l, u, c, m, true>)
-                                         : reinterpret_cast<const void*>(&velocity_batch_kernel<T, l, u, c, m, false>))
-                              : (persist ? reinterpret_cast<const void*>(&stress_batch_kernel<T, l, u, c, m, true>)
-                                         : reinterpret_cast<const void*>(&stress_batch_kernel<T, l, u, c, m, false>));
+    auto pick = [&](auto NT, auto P) {
+      constexpr bool nt = decltype(NT)::value, p = decltype(P)::value;
+      return velocity ? reinterpret_cast<const void*>(&velocity_batch_kernel<T, l, u, c, m, nt, p>)
+                      : reinterpret_cast<const void*>(&stress_batch_kernel<T, l, u, c, m, nt, p>);
+    };
+    const void* fn = persist ? pick(std::true_type(), std::true_type()) : pick(std::true_type(), std::false_type());
+    if constexpr (cacheable(l, u, c))
+      if (!stream && !persist) fn = pick(std::false_type(), std::false_type());
     if (graph) {
       void* args[4] = {(void*)&desc, (void*)&items, (void*)&n, (void*)&k};
       hipKernelNodeParams p{};
@@ -814,17 +818,17 @@ hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, i
 
 #if RSG_PART == 0 || RSG_PART == 3
 hipError_t launch_batch_f64(const BatchDesc<double>* d, const int32_t* table, int n, int k, int grid, int block,
-                            bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
-                            hipGraphNode_t* node) {
-  return launch_batch<double>(d, table, n, k, grid, block, lds, max_u, cpt, km, velocity, s, graph, node);
+                            bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
+                            hipGraph_t graph, hipGraphNode_t* node) {
+  return launch_batch<double>(d, table, n, k, grid, block, lds, max_u, cpt, km, stream, velocity, s, graph, node);
 }
 #endif
 
 #if RSG_PART == 0 || RSG_PART == 4
 hipError_t launch_batch_f32(const BatchDesc<float>* d, const int32_t* table, int n, int k, int grid, int block,
-                            bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
-                            hipGraphNode_t* node) {
-  return launch_batch<float>(d, table, n, k, grid, block, lds, max_u, cpt, km, velocity, s, graph, node);
+                            bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
+                            hipGraph_t graph, hipGraphNode_t* node) {
+  return launch_batch<float>(d, table, n, k, grid, block, lds, max_u, cpt, km, stream, velocity, s, graph, node);
 }
 #endif
 
