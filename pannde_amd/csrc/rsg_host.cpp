@@ -2702,16 +2702,16 @@ struct rsg_batch_s {
     int64_t off_v, off_s;
     int32_t n_v, n_s;          // table lengths (padded)
     int32_t grid_v, grid_s;
-    int32_t km_v, km_s;        // coefficient forms (0 arrays, 1 keys, 3 keys packed with links)
+    int32_t km_v, km_s;        // coefficient forms (0 arrays, 1 keys, 3 keys packed with links) and
+                               // rsg::kBatchCached
     bool lds_v, lds_s;         // LDS staging
     int32_t max_u_v, max_u_s;  // largest staged set of a member
     int32_t block_v, block_s, cpt_v, cpt_s;  // the members' workgroup sizes and per-thread counts
-    bool stream;               // non-temporal loads of what a step reads once
     bool operator==(const Launch& o) const {
       return off_v == o.off_v && off_s == o.off_s && n_v == o.n_v && n_s == o.n_s && grid_v == o.grid_v &&
              grid_s == o.grid_s && km_v == o.km_v && km_s == o.km_s && lds_v == o.lds_v && lds_s == o.lds_s &&
              max_u_v == o.max_u_v && max_u_s == o.max_u_s && block_v == o.block_v && block_s == o.block_s &&
-             cpt_v == o.cpt_v && cpt_s == o.cpt_s && stream == o.stream;
+             cpt_v == o.cpt_v && cpt_s == o.cpt_s;
     }
   };
   struct Lane {
@@ -2905,16 +2905,16 @@ int batch_launch_block(rsg_batch_s* b, rsg_batch_s::Lane& ln) {
         hipError_t e;
         if (sizeof(T) == 8) {
           e = rsg::launch_batch_f64((const rsg::BatchDesc<double>*)desc, wv + g.off_v, g.n_v, k, g.grid_v, g.block_v,
-                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, g.stream, true, ln.stream, graph, node);
+                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, true, ln.stream, graph, node);
           if (e != hipSuccess) return e;
           e = rsg::launch_batch_f64((const rsg::BatchDesc<double>*)desc, ws + g.off_s, g.n_s, k, g.grid_s, g.block_s,
-                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, g.stream, false, ln.stream, graph, node);
+                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, false, ln.stream, graph, node);
         } else {
           e = rsg::launch_batch_f32((const rsg::BatchDesc<float>*)desc, wv + g.off_v, g.n_v, k, g.grid_v, g.block_v,
-                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, g.stream, true, ln.stream, graph, node);
+                                    g.lds_v, g.max_u_v, g.cpt_v, g.km_v, true, ln.stream, graph, node);
           if (e != hipSuccess) return e;
           e = rsg::launch_batch_f32((const rsg::BatchDesc<float>*)desc, ws + g.off_s, g.n_s, k, g.grid_s, g.block_s,
-                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, g.stream, false, ln.stream, graph, node);
+                                    g.lds_s, g.max_u_s, g.cpt_s, g.km_s, false, ln.stream, graph, node);
         }
         if (e != hipSuccess) return e;
       }
@@ -3079,6 +3079,12 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
           t[2 * p + 1] = src < cnt ? natural[2 * src + 1] : 0;
         }
       }
+      // Links, keys and lists stay cached where the lanes' groups, this one's size each, do not
+      // exceed the memory-side cache by more than a third.  Measured, 2 lanes, us a step,
+      // non-temporal / cached by the two groups' MiB: FP32 105 57.6 / 51.3, 202 1023 / 922, 270 1003 /
+      // 925, 406 955 / 961, 540 941 / 1003; FP64 75 56.1 / 48.9, 298 888 / 857 and 313 / 295, 362
+      // 875 / 881.
+      const int32_t cached = busy_lanes * (bytes + once) <= kCacheBytes / 3 * 4 ? rsg::kBatchCached : 0;
       rsg_batch_s::Launch g;
       g.off_v = (int64_t)ov;
       g.off_s = (int64_t)os;
@@ -3086,18 +3092,12 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
       g.n_s = qs;
       g.grid_v = b->dense ? qv : b->grid;
       g.grid_s = b->dense ? qs : b->grid;
-      g.km_v = f[0];
-      g.km_s = f[1];
+      g.km_v = f[0] | cached;
+      g.km_s = f[1] | cached;
       g.block_v = f[2];
       g.block_s = f[3];
       g.cpt_v = f[4];
       g.cpt_s = f[5];
-      // Links, keys and lists stay cached where the lanes' groups, this one's size each, do not
-      // exceed the memory-side cache by more than a third.  Measured, 2 lanes, us a step,
-      // non-temporal / cached by the two groups' MiB: FP32 105 57.6 / 51.3, 202 1023 / 922, 270 1003 /
-      // 925, 406 955 / 961, 540 941 / 1003; FP64 75 56.1 / 48.9, 298 888 / 857 and 313 / 295, 362
-      // 875 / 881.
-      g.stream = busy_lanes * (bytes + once) > kCacheBytes / 3 * 4;
       g.lds_v = lds_v;
       g.lds_s = lds_s;
       g.max_u_v = lds_v ? mu_v : 0;

@@ -170,15 +170,17 @@ hipError_t launch_stress_f32(const StressArgs<float>& a, int block, hipStream_t 
 // order, 8-byte aligned, (-1, 0) for an empty item; lds selects LDS staging (max_u: the
 // largest staged set of any instance), cpt the entities per thread (1, 2 or 4), km the
 // coefficient form of every instance the table names (0 per-entity arrays, 1 class-table
-// keys, 3 keys packed with the LDS links), stream as the arguments' own.  With graph != nullptr the launch is added to
+// keys, 3 keys packed with the LDS links; kBatchCached added: ordinary loads of what a step
+// reads once).  With graph != nullptr the launch is added to
 // the graph as a kernel node that depends on *node (when not null) and *node becomes the
 // new node; otherwise it is enqueued on s.
+constexpr int kBatchCached = 8;
 hipError_t launch_batch_f64(const BatchDesc<double>* d, const int32_t* table, int n, int k, int grid, int block,
-                            bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
-                            hipGraph_t graph, hipGraphNode_t* node);
+                            bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
+                            hipGraphNode_t* node);
 hipError_t launch_batch_f32(const BatchDesc<float>* d, const int32_t* table, int n, int k, int grid, int block,
-                            bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
-                            hipGraph_t graph, hipGraphNode_t* node);
+                            bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
+                            hipGraphNode_t* node);
 // Energy: partials into a.partial, then their fixed-order sum into out[0] (kinetic) and
 // out[1] (strain); both device addresses.  nblocks <= kEnergyMaxBlocks.
 hipError_t launch_energy_f64(const EnergyArgs<double>& a, int nblocks, double* out, hipStream_t s);

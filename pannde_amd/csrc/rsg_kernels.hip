@@ -778,8 +778,10 @@ hipError_t launch_stress_f32(const StressArgs<float>& a, int block, hipStream_t 
 #if RSG_PART == 0 || RSG_PART >= 3
 template <typename T>
 hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, int k, int grid, int block,
-                        bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
-                        hipGraph_t graph, hipGraphNode_t* node) {
+                        bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
+                        hipGraphNode_t* node) {
+  const bool cached = km & kBatchCached;
+  km &= ~kBatchCached;
   if (grid <= 0 || n <= 0) return hipSuccess;
   if (reinterpret_cast<uintptr_t>(table) % alignof(int2)) return hipErrorInvalidValue;
   const int2* items = reinterpret_cast<const int2*>(table);
@@ -796,7 +798,7 @@ hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, i
     };
     const void* fn = persist ? pick(std::true_type(), std::true_type()) : pick(std::true_type(), std::false_type());
     if constexpr (cacheable(l, u, c))
-      if (!stream && !persist) fn = pick(std::false_type(), std::false_type());
+      if (cached && !persist) fn = pick(std::false_type(), std::false_type());
     if (graph) {
       void* args[4] = {(void*)&desc, (void*)&items, (void*)&n, (void*)&k};
       hipKernelNodeParams p{};
@@ -818,17 +820,17 @@ hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, i
 
 #if RSG_PART == 0 || RSG_PART == 3
 hipError_t launch_batch_f64(const BatchDesc<double>* d, const int32_t* table, int n, int k, int grid, int block,
-                            bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
-                            hipGraph_t graph, hipGraphNode_t* node) {
-  return launch_batch<double>(d, table, n, k, grid, block, lds, max_u, cpt, km, stream, velocity, s, graph, node);
+                            bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
+                            hipGraphNode_t* node) {
+  return launch_batch<double>(d, table, n, k, grid, block, lds, max_u, cpt, km, velocity, s, graph, node);
 }
 #endif
 
 #if RSG_PART == 0 || RSG_PART == 4
 hipError_t launch_batch_f32(const BatchDesc<float>* d, const int32_t* table, int n, int k, int grid, int block,
-                            bool lds, int max_u, int cpt, int km, bool stream, bool velocity, hipStream_t s,
-                            hipGraph_t graph, hipGraphNode_t* node) {
-  return launch_batch<float>(d, table, n, k, grid, block, lds, max_u, cpt, km, stream, velocity, s, graph, node);
+                            bool lds, int max_u, int cpt, int km, bool velocity, hipStream_t s, hipGraph_t graph,
+                            hipGraphNode_t* node) {
+  return launch_batch<float>(d, table, n, k, grid, block, lds, max_u, cpt, km, velocity, s, graph, node);
 }
 #endif
 
