@@ -143,6 +143,30 @@ __host__ __device__ constexpr int tri(int i, int j) {
   return (i <= j) ? (i * 6 - i * (i - 1) / 2 + (j - i)) : (j * 6 - j * (j - 1) / 2 + (i - j));
 }
 
+// The 21 stiffness entries of cell e from the per-cell arrays, AXIAL: nine of them and the row of the
+// others.  load(p) reads one value.
+template <bool AXIAL, typename T, typename L>
+__device__ __forceinline__ void cell_constants(const StressArgs<T>& a, int e, L&& load, T (&cc)[21]) {
+  // ldc > 0: [entries][ldc] arrays; ldc == 0: blocks of 64 cells, [n/64][entries][64], so one
+  // wavefront's coefficients are a single contiguous run
+  constexpr int N = AXIAL ? kAxialEntries : 21;
+  const T* p = a.C + (a.ldc ? (int64_t)e : (int64_t)(e >> 6) * (N * 64) + (e & 63));
+  const int64_t step = a.ldc ? a.ldc : 64;
+#pragma unroll
+  for (int j = 0; j < 21; j++) {
+    const int q = AXIAL ? axial_entry(j) : j;
+    cc[j] = q >= 0 ? load(p + q * step) : as_const(a.crow)[j];
+  }
+}
+template <typename T>
+__device__ __forceinline__ void cell_constants(const StressArgs<T>& a, int e, T (&cc)[21]) {
+  auto plain = [](const T* p) { return *p; };
+  if (a.crow)
+    cell_constants<true>(a, e, plain, cc);
+  else
+    cell_constants<false>(a, e, plain, cc);
+}
+
 // Summed moment terms of a special cell, per Voigt component.
 template <typename T>
 __device__ __forceinline__ void cell_moments(const StressArgs<T>& a, int sp, double (&m)[6]) {

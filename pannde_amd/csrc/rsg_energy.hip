@@ -23,7 +23,7 @@
 
 #include <mutex>
 
-#include "rsg_internal.h"
+#include "rsg_device.h"
 
 // Work area of rsg_energy_noalloc: the partials of kEnergyMaxBlocks workgroups and the two
 // totals (16 KiB), one copy per GPU for the life of the process.  Host code never uses this
@@ -46,11 +46,10 @@ __device__ void cell_stiffness(const StressArgs<T>& a, double inv_scale, int e, 
 #pragma unroll
     for (int j = 0; j < 21; j++) c[j] = (double)row[j] * inv_scale;
   } else {
+    T cc[21];
+    cell_constants(a, e, cc);
 #pragma unroll
-    for (int j = 0; j < 21; j++) {
-      const int64_t idx = a.ldc ? (int64_t)j * a.ldc + e : ((int64_t)(e >> 6) * 21 + j) * 64 + (e & 63);
-      c[j] = (double)a.C[idx] * inv_scale;
-    }
+    for (int j = 0; j < 21; j++) c[j] = (double)cc[j] * inv_scale;
   }
 }
 

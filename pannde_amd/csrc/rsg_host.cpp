@@ -294,6 +294,7 @@ struct rsg_instance {
   void* dn[3] = {nullptr, nullptr, nullptr};
   void* C = nullptr;
   int64_t ldc = 0;
+  void* crow = nullptr;  // the entries that are not per cell
   void* dc[3] = {nullptr, nullptr, nullptr};
   int32_t* ncell = nullptr;
   int32_t* cnode = nullptr;
@@ -1410,6 +1411,7 @@ void fill_args(rsg_instance* h, rsg::VelocityArgs<T>& va, rsg::StressArgs<T>& sa
   sa.V2 = (const T*)h->V[2];
   sa.C = (const T*)h->C;
   sa.ldc = h->ldc;
+  sa.crow = (const T*)h->crow;
   sa.dcx = (const T*)h->dc[0];
   sa.dcy = (const T*)h->dc[1];
   sa.dcz = (const T*)h->dc[2];
@@ -2196,12 +2198,30 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
       }
     }
     if (h->n_cmat < 0) {
-      std::vector<double> C((size_t)21 * ncp, 0.0);
-      for (int32_t i = 0; i < nc; i++)
-        for (int j = 0; j < 21; j++) {
-          const size_t idx = h->c_blocked ? ((size_t)(i >> 6) * 21 + j) * 64 + (i & 63) : (size_t)j * ncp + i;
-          C[idx] = c_entry(i, j);
-        }
+      // the nine axial entries alone where every other entry is one value for all cells
+      double row[21];
+      for (int j = 0; j < 21; j++) row[j] = c_entry(0, j);
+      std::atomic<bool> axial{true};
+      parallel_ranges(nc, [&](int64_t b, int64_t e) {
+        for (int j = 0; j < 21; j++)
+          if (rsg::axial_entry(j) < 0 && model->cij[j].type != RSG_FIELD_CONSTANT)
+            for (int64_t i = b; i < e && axial.load(std::memory_order_relaxed); i++) {
+              const double c = c_entry((int32_t)i, j);
+              if (memcmp(&c, &row[j], sizeof(c))) axial = false;
+            }
+      });
+      const int64_t width = axial ? rsg::kAxialEntries : 21;
+      std::vector<double> C((size_t)(width * ncp), 0.0);
+      parallel_ranges(nc, [&](int64_t b, int64_t e) {
+        for (int64_t i = b; i < e; i++)
+          for (int j = 0; j < 21; j++) {
+            const int q = axial ? rsg::axial_entry(j) : j;
+            if (q < 0) continue;
+            const int64_t idx = h->c_blocked ? ((i >> 6) * width + q) * 64 + (i & 63) : q * ncp + i;
+            C[(size_t)idx] = c_entry((int32_t)i, j);
+          }
+      });
+      if (axial && (rc = upload_real(h.get(), &h->crow, std::vector<double>(row, row + 21)))) return rc;
       for (int d = 0; d < 3; d++)
         if ((rc = upload_real(h.get(), &h->dc[d], dc[d]))) return rc;
       if ((rc = upload_real(h.get(), &h->C, std::move(C)))) return rc;
@@ -2350,7 +2370,7 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     h->once_v = (int64_t)nn * ((h->v_lkey || h->v_lconn ? 16 : 32) + (h->nkey ? 4 : 0)) + h->v_list_bytes +
                            (h->n_nmat < 0 ? 4 * e * nn : 0);
     h->once_s = (int64_t)nc * ((h->s_lkey || h->s_lconn ? 16 : 32) + (h->ckey ? 4 : 0)) + h->s_list_bytes +
-                           (h->n_cmat < 0 ? 24 * e * nc : 0);
+                           (h->n_cmat < 0 ? (h->crow ? 3 + rsg::kAxialEntries : 24) * e * nc : 0);
     h->stream_v = state + h->once_v > cache;
     h->stream_s = state + h->once_v + h->once_s > cache;
   }
@@ -3010,7 +3030,7 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
   // configuration, each group within the state budget (an instance larger than the budget
   // forms a group of its own)
   auto config = [](const rsg_instance* h) -> std::array<int32_t, 8> {
-    return {h->v_lkey ? 3 : h->nkey ? 1 : 0, h->s_lkey ? 3 : h->ckey ? 1 : 0, h->block_v, h->block_s, h->cpt_v,
+    return {h->v_lkey ? 3 : h->nkey ? 1 : 0, h->s_lkey ? 3 : h->ckey ? 1 : h->crow ? 2 : 0, h->block_v, h->block_s, h->cpt_v,
             h->cpt_s, (h->v_lconn || h->v_lkey) ? 1 : 0, (h->s_lconn || h->s_lkey) ? 1 : 0};
   };
   std::vector<std::array<int32_t, 8>> configs;  // distinct configurations, first seen first

@@ -28,6 +28,13 @@ constexpr uint32_t kSpecialKey = 0x80000000u;
 constexpr int kMatShift = 21;
 constexpr int kMaxMaterials = 1024;
 constexpr int kAxisClasses = 128;  // spacing classes per axis; tables are [3][kAxisClasses]
+// Entries of the 21 that a material with axes along the coordinate axes has (C11, C12, C13, C22, C23,
+// C33, C44, C55, C66).  Per-cell arrays hold these alone where each of the others is the same for
+// all cells, as in a part whose stiffness varies but not its symmetry: 72 of 168 bytes a cell.
+constexpr int kAxialEntries = 9;
+constexpr int axial_entry(int j) {  // its place among them, or -1
+  return j < 3 ? j : j == 6 ? 3 : j == 7 ? 4 : j == 11 ? 5 : j == 15 ? 6 : j == 18 ? 7 : j == 20 ? 8 : -1;
+}
 constexpr int kMatRow = 24;        // cell material row: the 21 C as the C array holds them, padded
 constexpr uint32_t kNoLink = 0x3FF;  // packed 10-bit link: no neighbour
 constexpr int kMaxPackedSet = 1022;  // largest staged set whose local indices fit 10 bits
@@ -105,6 +112,7 @@ struct StressArgs {
   const T* V2;
   const T* C;    // [21][ldc]: FP64 C_IJ; FP32 dt*C_IJ (FP64 product, rounded)
   int64_t ldc;   // leading dimension of C (>= n), or 0 for the 64-cell blocked layout
+  const T* crow;  // [21], where C holds kAxialEntries per cell: what the others are for all cells
   const T* dcx;  // FP64: cell spacing dxc (NaN-boxed for special cells); FP32: 0.25/dxc
   const T* dcy;
   const T* dcz;

@@ -118,8 +118,8 @@ __device__ __forceinline__ void load8_nodes(const T* __restrict__ f, const int (
 }
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-// Coefficient form of a kernel instance: KM = 0 per-entity arrays, 1 class-table keys,
-// 3 keys packed with the LDS links (a batch launches each form for its own members).
+// Coefficient form of a kernel instance: KM = 0 per-entity arrays, 2 per-cell arrays of the axial
+// entries (stress kernels), 1 class-table keys, 3 keys packed with the LDS links (a batch launches each form for its own members).
 template <int KM, typename A>
 __device__ __forceinline__ constexpr bool packed(const A&) {
   return KM == 3;
@@ -415,14 +415,6 @@ __device__ __forceinline__ void velocity_body(const VelocityArgs<T>& a, int b, u
   }
 }
 
-template <bool NT, typename T>
-__device__ __forceinline__ T cload(const T* __restrict__ C, int64_t ldc, int j, int i) {
-  // ldc > 0: [21][ldc] arrays; ldc == 0: blocks of 64 cells, [n/64][21][64], so one
-  // wavefront's 21 coefficients are a single contiguous run
-  const int64_t idx = ldc ? (int64_t)j * ldc + i : ((int64_t)(i >> 6) * 21 + j) * 64 + (i & 63);
-  return stream_load<NT>(C + idx);
-}
-
 // Per-cell operands of the stress update that do not depend on a gather: links,
 // spacings, the 21 C_IJ and the 6 stresses.
 template <typename T>
@@ -454,8 +446,7 @@ __device__ __forceinline__ void stress_load(const StressArgs<T>& a, int e, StrIn
     in.sx = a.dcx[e];
     in.sy = a.dcy[e];
     in.sz = a.dcz[e];
-#pragma unroll
-    for (int j = 0; j < 21; j++) in.cc[j] = cload<NT>(a.C, a.ldc, j, e);
+    cell_constants<KM == 2>(a, e, [](const T* p) { return stream_load<NT>(p); }, in.cc);
   }
   in.s[0] = a.S0[e];
   in.s[1] = a.S1[e];
@@ -684,7 +675,7 @@ hipError_t launch1d(K kernel, const Args& a, int n, int block, size_t lds, hipSt
 
 // Picks the kernel instance: direct gathers, or LDS staging with U = ceil(max_u/block)
 // entries per thread (general loop beyond 4), for 1, 2 or 4 entities per thread.
-template <typename F>
+template <bool STRESS, typename F>
 hipError_t with_variant(bool lds, int max_u, int block, int cpt, int km, F&& f) {
   auto by_u = [&](auto cptc, auto kmc) -> hipError_t {
     if (!lds) {
@@ -713,6 +704,9 @@ hipError_t with_variant(bool lds, int max_u, int block, int cpt, int km, F&& f) 
   switch (km) {
     case 0: return by_cpt(std::integral_constant<int, 0>());
     case 1: return by_cpt(std::integral_constant<int, 1>());
+    case 2:
+      if constexpr (STRESS) return by_cpt(std::integral_constant<int, 2>());
+      return hipErrorInvalidValue;
     case 3: return by_cpt(std::integral_constant<int, 3>());
     default: return hipErrorInvalidValue;
   }
@@ -725,7 +719,7 @@ constexpr bool cacheable(bool lds, int u, int cpt) { return lds && u > 0 && cpt 
 template <typename T>
 hipError_t launch_velocity(const VelocityArgs<T>& a, int block, hipStream_t s) {
   const bool lds = a.lconn != nullptr || a.lkey != nullptr;
-  return with_variant(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : 0, [&](auto L, auto U, auto C, auto K) {
+  return with_variant<false>(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : 0, [&](auto L, auto U, auto C, auto K) {
     constexpr bool l = decltype(L)::value;
     constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
     const size_t bytes = lds ? velocity_lds_bytes(a.max_u, sizeof(T)) : 0;
@@ -738,7 +732,7 @@ hipError_t launch_velocity(const VelocityArgs<T>& a, int block, hipStream_t s) {
 template <typename T>
 hipError_t launch_stress(const StressArgs<T>& a, int block, hipStream_t s) {
   const bool lds = a.lconn != nullptr || a.lkey != nullptr;
-  return with_variant(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : 0, [&](auto L, auto U, auto C, auto K) {
+  return with_variant<true>(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : a.crow ? 2 : 0, [&](auto L, auto U, auto C, auto K) {
     constexpr bool l = decltype(L)::value;
     constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
     const size_t bytes = lds ? (size_t)3 * a.max_u * sizeof(T) : 0;
@@ -788,13 +782,15 @@ hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, i
   if (block < 64 || block > RSG_MAX_BLOCK || (block % 64) != 0) return hipErrorInvalidValue;
   const size_t bytes = !lds ? 0 : velocity ? velocity_lds_bytes(max_u, sizeof(T)) : (size_t)3 * max_u * sizeof(T);
   const bool persist = grid != n;
-  return with_variant(lds, max_u, block, cpt, km, [&](auto L, auto U, auto C, auto K) {
+  auto launch = [&](auto V, auto L, auto U, auto C, auto K) {
     constexpr bool l = decltype(L)::value;
     constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
     auto pick = [&](auto NT, auto P) {
       constexpr bool nt = decltype(NT)::value, p = decltype(P)::value;
-      return velocity ? reinterpret_cast<const void*>(&velocity_batch_kernel<T, l, u, c, m, nt, p>)
-                      : reinterpret_cast<const void*>(&stress_batch_kernel<T, l, u, c, m, nt, p>);
+      if constexpr (decltype(V)::value)
+        return reinterpret_cast<const void*>(&velocity_batch_kernel<T, l, u, c, m, nt, p>);
+      else
+        return reinterpret_cast<const void*>(&stress_batch_kernel<T, l, u, c, m, nt, p>);
     };
     const void* fn = persist ? pick(std::true_type(), std::true_type()) : pick(std::true_type(), std::false_type());
     if constexpr (cacheable(l, u, c))
@@ -813,7 +809,11 @@ hipError_t launch_batch(const BatchDesc<T>* desc, const int32_t* table, int n, i
     }
     void* args[4] = {(void*)&desc, (void*)&items, (void*)&n, (void*)&k};
     return hipLaunchKernel(fn, dim3(grid), dim3(block), args, bytes, s);
-  });
+  };
+  if (velocity)
+    return with_variant<false>(lds, max_u, block, cpt, km,
+                               [&](auto... x) { return launch(std::true_type(), x...); });
+  return with_variant<true>(lds, max_u, block, cpt, km, [&](auto... x) { return launch(std::false_type(), x...); });
 }
 
 #endif

@@ -423,9 +423,7 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
       T sx = sa.dcx[e];
       const T sy = sa.dcy[e], sz = sa.dcz[e];
       T cc[21];
-#pragma unroll
-      for (int q = 0; q < 21; q++)
-        cc[q] = sa.C[sa.ldc ? (int64_t)q * sa.ldc + e : ((int64_t)(e >> 6) * 21 + q) * 64 + (e & 63)];
+      cell_constants(sa, e, cc);
       if (is_boxed(sx)) {
         sp = 0;
         sx = sa.sp_dcx[unbox(sx)];
@@ -624,9 +622,7 @@ __global__ __launch_bounds__(1024) void resident_alone_kernel(ResidentArgs<T> a)
             sp = unbox(sx);
             sx = sa.sp_dcx[sp];
           }
-#pragma unroll
-          for (int q = 0; q < 21; q++)
-            cc[q] = sa.C[sa.ldc ? (int64_t)q * sa.ldc + e : ((int64_t)(e >> 6) * 21 + q) * 64 + (e & 63)];
+          cell_constants(sa, e, cc);
         }
         double m[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll

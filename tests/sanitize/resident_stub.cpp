@@ -158,8 +158,12 @@ hipError_t run(const ResidentArgs<T>& a, int threads) {
           for (int q = 0; q < 21; q++) cc[q] = a.s.cls[(size_t)(w >> kMatShift) * kMatRow + q];
           for (int d = 0; d < 3; d++) sp[d] = a.s.axis[d * kAxisClasses + (w >> (14 - 7 * d) & (kAxisClasses - 1))];
         } else {
-          for (int q = 0; q < 21; q++)
-            cc[q] = a.s.C[a.s.ldc ? (int64_t)q * a.s.ldc + e : ((int64_t)(e >> 6) * 21 + q) * 64 + (e & 63)];
+          const int width = a.s.crow ? kAxialEntries : 21;
+          for (int j = 0; j < 21; j++) {
+            const int q = a.s.crow ? axial_entry(j) : j;
+            cc[j] = q < 0 ? a.s.crow[j]
+                          : a.s.C[a.s.ldc ? (int64_t)q * a.s.ldc + e : ((int64_t)(e >> 6) * width + q) * 64 + (e & 63)];
+          }
           sp[0] = a.s.dcx[e], sp[1] = a.s.dcy[e], sp[2] = a.s.dcz[e];
           if (std::isnan(sp[0])) {
             uint64_t bits = 0;
