@@ -479,8 +479,8 @@ template <typename T, int KM, bool PAIRS = false>
 __device__ __forceinline__ void stress_apply(const StressArgs<T>& a, int e, StrIn<T>& in, const T* V0,
                                              const T* V1, const T* V2) {
   T d[6];
-  double m[6];
   int sp = -1;
+  auto m = [&](int k) { return cell_moment(a, sp, k); };
   if (keyed<KM>(a)) {
     // class tables: spacings and material row through the scalar cache where the
     // wavefront shares them
@@ -504,7 +504,6 @@ __device__ __forceinline__ void stress_apply(const StressArgs<T>& a, int e, StrI
 #pragma unroll
       for (int j = 0; j < 21; j++) c0[j] = row0[j];
       strain_terms<T, PAIRS>(V0, V1, V2, in.c, sx, sy, sz, d);
-      cell_moments(a, sp, m);
       if (__all(mat == m0)) {
         voigt_update(a.dt, c0, d, m, sp, in.s);
       } else {
@@ -531,7 +530,6 @@ __device__ __forceinline__ void stress_apply(const StressArgs<T>& a, int e, StrI
         for (int j = 0; j < 21; j++) cc[j] = row[j];
       }
       strain_terms<T, PAIRS>(V0, V1, V2, in.c, sx, sy, sz, d);
-      cell_moments(a, sp, m);
       voigt_update(a.dt, cc, d, m, sp, in.s);
     }
   } else {
@@ -542,7 +540,6 @@ __device__ __forceinline__ void stress_apply(const StressArgs<T>& a, int e, StrI
       sx = a.sp_dcx[sp];
     }
     strain_terms<T, PAIRS>(V0, V1, V2, in.c, sx, in.sy, in.sz, d);
-    cell_moments(a, sp, m);
     voigt_update(a.dt, in.cc, d, m, sp, in.s);
   }
   a.S0[e] = in.s[0];

@@ -357,13 +357,6 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
     for (int d = 0; d < 3; d++) V[3 * i + d] = V[3 * i + d] + idt * r[d];
   };
 
-  auto moments = [&](int i, int sp, double (&m)[6]) {
-    if (sp < 0) return;
-    const double* f = now + a.cforce0 + 6 * (cmark[i] - 1);
-#pragma unroll
-    for (int q = 0; q < 6; q++) m[q] = f[q];
-  };
-
   // Steps the cell in its slot; o: its new stresses in slot order.
   auto cell_update = [&](int i, T (&o)[6]) {
     const v4u rec = crec[i];
@@ -379,8 +372,15 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
         s[slot_comp(2 * p + 1)] = w.y;
       }
     };
-    double m[6] = {0, 0, 0, 0, 0, 0};
     int sp = -1;
+    double terms[6] = {0, 0, 0, 0, 0, 0};
+    auto moments = [&]() {  // read at once: one wait for the six
+      if (sp < 0) return;
+      const double* f = now + a.cforce0 + 6 * (cmark[i] - 1);
+#pragma unroll
+      for (int q = 0; q < 6; q++) terms[q] = f[q];
+    };
+    auto m = [&](int q) { return terms[q]; };
     auto xy = [&](T(&f)[8], T(&g)[8]) {
 #pragma unroll
       for (int k = 0; k < 8; k++) {
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
       for (int q = 0; q < 21; q++) c0[q] = row0[q];
       strain_rates(xy, z, sd, d);
       own();
-      moments(i, sp, m);
+      moments();
       if (__all(mat == m0)) {
         voigt_update(sa.dt, c0, d, m, sp, s);
       } else {  // one pass per distinct material of the wavefront
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
       set_spacing(sz, sd[2]);
       strain_rates(xy, z, sd, d);
       own();
-      moments(i, sp, m);
+      moments();
       voigt_update(sa.dt, cc, d, m, sp, s);
     }
 #pragma unroll
@@ -624,12 +624,9 @@ __global__ __launch_bounds__(1024) void resident_alone_kernel(ResidentArgs<T> a)
           }
           cell_constants(sa, e, cc);
         }
-        double m[6] = {0, 0, 0, 0, 0, 0};
+        auto m = [&](int q) { return now[a.cforce0 + 6 * a.ccls[sp] + q]; };
 #pragma unroll
-        for (int q = 0; q < 6; q++) {
-          if (sp >= 0) m[q] = now[a.cforce0 + 6 * a.ccls[sp] + q];
-          s[q] = Sg[q][e];
-        }
+        for (int q = 0; q < 6; q++) s[q] = Sg[q][e];
         strain_rates<T>(
             [&](T(&f)[8], T(&g)[8]) {
 #pragma unroll
