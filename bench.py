@@ -47,8 +47,10 @@ REFERENCE_MODEL_BYTES = {"stress": {"f64": 344, "f32": 188}, "velocity": {"f64":
 # samples per kernel in a 2000-step run): events between every launch slowed the stream by 4 %
 # (FP64) to 8 % (FP32).
 TIMING_STRIDE = 32
-# the sources the counter traffic in profiles/ was measured with
-KERNEL_SOURCES = ("pannde_amd/csrc/rsg_kernels.hip", "pannde_amd/csrc/rsg_internal.h")
+# the sources the counter traffic in profiles/ was measured with: the per-step kernels and every
+# header they are built from
+KERNEL_SOURCES = ("pannde_amd/csrc/rsg_kernels.hip", "pannde_amd/csrc/rsg_device.h",
+                  "pannde_amd/csrc/rsg_internal.h")
 # Untimed first steps of the drop-in driver leg (code-object loading on first launch).
 DROPIN_UNTIMED = 10
 # The CPU baseline uses at most this many MPI ranks: the host's CPU share for one GPU.
