@@ -35,7 +35,6 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <unordered_map>
@@ -400,7 +399,7 @@ struct rsg_instance {
 
   size_t elt() const { return precision == RSG_FP64 ? 8 : 4; }
 
-  std::mutex alloc_mu;  // set-up allocates from two threads
+  std::mutex alloc_mu;  // set-up allocates from several threads
 
   // host sources of the copies queued on `stream` since it was last synchronized; a set-up
   // queues all its uploads and waits once (finish_uploads)
@@ -530,7 +529,7 @@ void parallel_tasks(int t, F&& fn) {
   int started = 1;
   try {
     for (; started < t; started++) workers.emplace_back(task, started);
-  } catch (const std::system_error&) {  // no thread to be had: the caller takes the rest
+  } catch (...) {  // no thread, or no memory for one: the caller takes the rest
   }
   task(0);
   for (int w = started; w < t; w++) task(w);
@@ -1982,21 +1981,16 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
       }
     });
     double clo[3] = {lo[0] + 0.5 * hmin[0], lo[1] + 0.5 * hmin[1], lo[2] + 0.5 * hmin[2]};
-    bool cells_ok = true, nodes_ok = true;
-    std::thread cell_sort([&]() {  // the two orders are independent
-      try {
-        h->cell_of = locality_order(nc, cx.data(), cy.data(), cz.data(), hmin, clo, h->tile);
-      } catch (const std::bad_alloc&) {
-        cells_ok = false;
-      }
-    });
     try {
-      h->node_of = locality_order(nn, X[0], X[1], X[2], hmin, lo, h->tile);
+      parallel_tasks(2, [&](int w) {  // the two orders are independent
+        if (w == 0)
+          h->node_of = locality_order(nn, X[0], X[1], X[2], hmin, lo, h->tile);
+        else
+          h->cell_of = locality_order(nc, cx.data(), cy.data(), cz.data(), hmin, clo, h->tile);
+      });
     } catch (const std::bad_alloc&) {
-      nodes_ok = false;
+      return fail(RSG_ERR_NOMEM, "host allocation failed");
     }
-    cell_sort.join();
-    if (!cells_ok || !nodes_ok) return fail(RSG_ERR_NOMEM, "host allocation failed");
   }
   h->cell_at.resize(nc);
   h->node_at.resize(nn);
@@ -2019,7 +2013,7 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
   }
 
   CREATE_PHASE("stream");
-  // node arrays and cell arrays are independent: built on two threads
+  // node arrays, cell arrays and the resident plan are independent: each built on a thread
   auto node_part = [&]() -> int {
     int rc;
     std::vector<double> idt(nn), w(nn), dn[3];
@@ -2316,46 +2310,27 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     return RSG_OK;
   };
   {
-    int rc_cells = RSG_OK, rc_res = RSG_OK;
-    std::string err_cells, err_res;
-    int dev = 0;
+    int dev = 0, rcs[3] = {RSG_OK, RSG_OK, RSG_OK};
+    std::string errs[3];
     HIP_TRY(hipGetDevice(&dev));
-    std::thread resident([&]() {
-      try {
-        const hipError_t e = hipSetDevice(dev);
-        rc_res = e != hipSuccess ? fail(RSG_ERR_DEVICE, "hipSetDevice: %s", hipGetErrorString(e)) : resident_part();
-      } catch (const std::bad_alloc&) {
-        rc_res = fail(RSG_ERR_NOMEM, "host allocation failed");
-      }
-      if (rc_res) err_res = g_last_error;
-    });
-    std::thread worker([&]() {
-      try {
+    try {
+      parallel_tasks(3, [&](int w) {
         // a new thread starts on device 0: work on the caller's device
         const hipError_t e = hipSetDevice(dev);
-        rc_cells = e != hipSuccess ? fail(RSG_ERR_DEVICE, "hipSetDevice: %s", hipGetErrorString(e)) : cell_part();
-      } catch (const std::bad_alloc&) {
-        rc_cells = fail(RSG_ERR_NOMEM, "host allocation failed");
-      }
-      if (rc_cells) err_cells = g_last_error;
-    });
-    int rc_nodes;
-    try {
-      rc_nodes = node_part();
+        rcs[w] = e != hipSuccess ? fail(RSG_ERR_DEVICE, "hipSetDevice: %s", hipGetErrorString(e))
+                 : w == 0        ? node_part()
+                 : w == 1        ? cell_part()
+                                 : resident_part();
+        if (rcs[w]) errs[w] = g_last_error;
+      });
     } catch (const std::bad_alloc&) {
-      rc_nodes = fail(RSG_ERR_NOMEM, "host allocation failed");
+      return fail(RSG_ERR_NOMEM, "host allocation failed");
     }
-    worker.join();
-    resident.join();
-    if (rc_nodes) return rc_nodes;
-    if (rc_cells) {
-      g_last_error = err_cells;
-      return rc_cells;
-    }
-    if (rc_res) {
-      g_last_error = err_res;
-      return rc_res;
-    }
+    for (int w = 0; w < 3; w++)
+      if (rcs[w]) {
+        g_last_error = errs[w];
+        return rcs[w];
+      }
   }
   // What each kernel reads once a step (links, keys, lists, per-entity coefficients) stays in the
   // 256 MiB memory-side cache from step to step where it fits beside the state with a tenth to
