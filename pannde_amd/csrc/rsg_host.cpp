@@ -349,6 +349,11 @@ struct rsg_instance {
   uint32_t res_seq = 0;            // launches so far
   hipEvent_t res_event = nullptr;  // behind the last one
   int32_t* res_status = nullptr;  // pinned, from the first resident launch on
+  // the last launch of several tiles, until its decision is known: its steps (0: it is), first
+  // step's amplitudes and trace row
+  int32_t res_pending = 0;
+  const double* res_amp = nullptr;
+  int64_t res_row = 0;
 
   // state transfers: the caller -> internal maps on the device (from the first transfer on) and
   // each transfer thread's chunk of pinned memory
@@ -1458,10 +1463,6 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
     HIP_TRY(hipHostMalloc((void**)&h->res_status, rsg::kResidentStatus * sizeof(int32_t), hipHostMallocDefault));
     memset(h->res_status, 0, rsg::kResidentStatus * sizeof(int32_t));
   }
-  if (__atomic_load_n(h->res_status + rsg::kResidentAlone, __ATOMIC_RELAXED)) {
-    h->res_tiles = 0;  // the GPU is shared with work that keeps the tiles apart
-    return RSG_OK;
-  }
   rsg::ResidentArgs<T> a;
   a.v = va;
   a.s = sa;
@@ -1515,26 +1516,14 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   return RSG_OK;
 }
 
+// kb steps, two launches each; every stride-th step's launches are timed (0: none).
 template <typename T>
-int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* force_dev) {
-  rsg::VelocityArgs<T> va;
-  rsg::StressArgs<T> sa;
-  fill_args<T>(h, va, sa);
+int run_steps(rsg_instance* h, int kb, rsg::VelocityArgs<T>& va, rsg::StressArgs<T>& sa, const double* amp_dev,
+              int64_t trace_row, int stride) {
   const size_t nch = std::max<size_t>(1, h->channels.size());
   const size_t row = h->sensors.size() * 3;
-  if (h->res_tiles > 0 && h->res_nclasses >= 0 && kb >= (h->res_tiles == 1 ? 2 : kResidentMinSteps) && h->timing == 0) {
-    va.trace = h->trace.p ? h->trace.p + (size_t)h->trace_dev_steps * row : nullptr;
-    bool done = false;
-    const int rc = run_resident<T>(h, kb, va, sa, force_dev, row, &done);
-    if (rc) return rc;
-    if (done) {
-      h->trace_dev_steps += row ? kb : 0;
-      return RSG_OK;
-    }
-  }
   // timed steps get three events: before the velocity launch, between the two, after the
   // stress launch (events between every launch slow the stream down, so a stride samples)
-  const int stride = h->timing;
   const int nt = stride > 0 ? (kb + stride - 1) / stride : 0;
   if (nt) {
     int rc = ensure_events(h, (size_t)3 * nt);
@@ -1545,7 +1534,7 @@ int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* forc
     hipEvent_t* ev = timed ? &h->tev[(size_t)3 * (k / stride)] : nullptr;
     va.amp = amp_dev + (size_t)k * nch;
     sa.amp = va.amp;
-    va.trace = h->trace.p ? h->trace.p + (size_t)(h->trace_dev_steps + k) * row : nullptr;
+    va.trace = h->trace.p ? h->trace.p + (size_t)(trace_row + k) * row : nullptr;
     hipError_t e;
     if (timed) HIP_TRY(hipEventRecord(ev[0], h->stream));
     if (sizeof(T) == 8)
@@ -1572,6 +1561,56 @@ int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* forc
     }
     h->t_launches += nt;
   }
+  return RSG_OK;
+}
+
+// Once this returns, the steps of the handle's last resident launch are made or queued: it waits for
+// the launch's decision, which comes as the launch begins, and queues the per-step kernels when that
+// was against the steps.  Called before anything else that uses the handle's state, tables or
+// amplitudes goes on its stream.
+int settle_resident(rsg_instance* h) {
+  if (h->res_pending == 0) return RSG_OK;
+  auto decision = [&]() { return (uint32_t)__atomic_load_n(h->res_status + rsg::kResidentDecision, __ATOMIC_ACQUIRE); };
+  uint32_t d = decision();
+  for (uint32_t spin = 1; d >> 1 != (h->res_seq & 0x7FFFFFFFu); spin++, d = decision()) {
+    if (spin % 64) continue;
+    const hipError_t e = hipEventQuery(h->res_event);
+    if (e == hipSuccess) break;  // (a launch that has ended has decided)
+    if (e != hipErrorNotReady) return fail(RSG_ERR_DEVICE, "resident launch: %s", hipGetErrorString(e));
+    std::this_thread::yield();
+  }
+  const int kb = h->res_pending;
+  h->res_pending = 0;
+  if (decision() != 2 * h->res_seq) return RSG_OK;
+  h->res_tiles = 0;  // the GPU is shared with work that keeps the tiles apart
+  auto steps = [&](auto zero) {
+    using T = decltype(zero);
+    rsg::VelocityArgs<T> va;
+    rsg::StressArgs<T> sa;
+    fill_args<T>(h, va, sa);
+    return run_steps<T>(h, kb, va, sa, h->res_amp, h->res_row, 0);
+  };
+  return h->precision == RSG_FP64 ? steps(0.0) : steps(0.0f);
+}
+
+template <typename T>
+int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* force_dev) {
+  rsg::VelocityArgs<T> va;
+  rsg::StressArgs<T> sa;
+  fill_args<T>(h, va, sa);
+  const size_t row = h->sensors.size() * 3;
+  bool done = false;
+  int rc;
+  if (h->res_tiles > 0 && h->res_nclasses >= 0 && kb >= (h->res_tiles == 1 ? 2 : kResidentMinSteps) && h->timing == 0) {
+    va.trace = h->trace.p ? h->trace.p + (size_t)h->trace_dev_steps * row : nullptr;
+    if ((rc = run_resident<T>(h, kb, va, sa, force_dev, row, &done))) return rc;
+    if (done && h->res_tiles > 1) {
+      h->res_pending = kb;
+      h->res_amp = amp_dev;
+      h->res_row = h->trace_dev_steps;
+    }
+  }
+  if (!done && (rc = run_steps<T>(h, kb, va, sa, amp_dev, h->trace_dev_steps, h->timing))) return rc;
   h->trace_dev_steps += row ? kb : 0;
   return RSG_OK;
 }
@@ -1595,6 +1634,7 @@ void fill_energy_args(rsg_instance* h, rsg::EnergyArgs<T>& a, double* work) {
 
 int energy_on_stream(rsg_instance* h, double* work, double* kinetic, double* strain) {
   Range range_("rsg_energy");
+  if (int rc = settle_resident(h)) return rc;
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
   if (h->tables_dirty) {
     int rc = build_tables(h);  // the special-cell keys the kernel resolves
@@ -2399,6 +2439,7 @@ int rsg_set_channels(rsg_handle h, int32_t n, const rsg_channel_desc* ch) {
       c.sig.build(d.n_signal, d.signal_t, d.signal_v);
     }
   }
+  if (int rc = settle_resident(h)) return rc;
   if (h->stream) HIP_TRY(hipStreamSynchronize(h->stream));
   h->channels.swap(list);
   h->tables_dirty = true;
@@ -2416,11 +2457,13 @@ int rsg_set_sensors(rsg_handle h, int32_t n, const int32_t* nodes) {
     if (seen[nodes[s]]) return fail(RSG_ERR_ARG, "sensor node %d listed twice", nodes[s]);
     seen[nodes[s]] = 1;
   }
+  int rc = settle_resident(h);
+  if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
   h->sensors.assign(nodes, nodes + n);
   h->trace_host.clear();
   h->trace_dev_steps = 0;
-  int rc = h->trace.alloc((size_t)std::max(1, n) * 3 * kTraceCapSteps, h->stream);
+  rc = h->trace.alloc((size_t)std::max(1, n) * 3 * kTraceCapSteps, h->stream);
   if (rc) return rc;
   h->tables_dirty = true;
   return build_tables(h);
@@ -2431,7 +2474,8 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   if (h->in_batch) return fail(RSG_ERR_STATE, "the handle is stepped by a batch; remove it first");
   if (nsteps < 0) return fail(RSG_ERR_ARG, "nsteps < 0");
-  int rc;
+  int rc = settle_resident(h);
+  if (rc) return rc;
   if (h->tables_dirty && (rc = build_tables(h))) return rc;
   const size_t nch = h->channels.size();
   if (!amplitudes)
@@ -2442,6 +2486,7 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
   // the resident kernel's summed source terms follow the amplitudes of an upload
   const size_t nf = h->res_nclasses >= 0 ? h->res_force.size() : 0;
   for (int32_t done = 0; done < nsteps;) {
+    if ((rc = settle_resident(h))) return rc;
     int kb = std::min(kBlockSteps, nsteps - done);
     // no channels: a buffer no term reads, and zero sums (of special nodes that are sensors only)
     const bool none = nch == 0 && nf == 0;
@@ -2517,19 +2562,22 @@ int rsg_get_state(rsg_handle h, double* V, double* S) {
   Range range_("rsg_get_state");
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
-  const int rc = transfer_state(h, V, S, false);
+  int rc = settle_resident(h);
+  if (!rc) rc = transfer_state(h, V, S, false);
   return rc ? rc : check_resident(h);
 }
 
 int rsg_set_state(rsg_handle h, const double* V, const double* S) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   if (h->in_batch) return fail(RSG_ERR_STATE, "the handle is in a batch; remove it first");
-  return transfer_state(h, const_cast<double*>(V), const_cast<double*>(S), true);
+  const int rc = settle_resident(h);
+  return rc ? rc : transfer_state(h, const_cast<double*>(V), const_cast<double*>(S), true);
 }
 
 int rsg_get_traces(rsg_handle h, int64_t first, int64_t n, double* out) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
-  int rc = flush_traces(h);
+  int rc = settle_resident(h);
+  if (!rc) rc = flush_traces(h);
   if (rc) return rc;
   const size_t row = h->sensors.size() * 3;
   const int64_t have = row ? (int64_t)(h->trace_host.size() / row) : 0;
@@ -2543,6 +2591,7 @@ int rsg_get_traces(rsg_handle h, int64_t first, int64_t n, double* out) {
 
 int rsg_synchronize(rsg_handle h) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
+  if (int rc = settle_resident(h)) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
   return check_resident(h);
@@ -3168,7 +3217,8 @@ int rsg_batch_add(rsg_batch b, rsg_handle h, int64_t nsteps, int32_t* slot) {
   if (h->precision != b->precision) return fail(RSG_ERR_ARG, "precision differs from the batch's");
   for (auto& c : h->channels)
     if (!c.has_signal) return fail(RSG_ERR_ARG, "batched instances need signal tables on every channel");
-  int rc;
+  int rc = settle_resident(h);
+  if (rc) return rc;
   if (h->tables_dirty && (rc = build_tables(h))) return rc;
   // the handle's own uploads must be complete; blocks already enqueued do not involve it
   HIP_TRY(hipStreamSynchronize(h->stream));

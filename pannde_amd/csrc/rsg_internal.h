@@ -224,9 +224,10 @@ constexpr uint32_t kResidentOwner = 0x80000000u;  // node record: this tile writ
 constexpr int kResidentForces = 256;  // largest row
 constexpr uint8_t kResidentSensor = 0x80;  // node mark: a sensor this tile records
 
-// Status words, 1 when: a launch's tiles did not get onto the GPU together and one workgroup made
-// its steps (later launches should not try); a wait between tiles ran out (the state is lost).
-constexpr int kResidentAlone = 0, kResidentLost = 1, kResidentStatus = 2;
+// Status words: the last launch's decision (several tiles), 2 seq + 1 when its steps are made and
+// 2 seq when its tiles did not get onto the GPU together and nothing is written; 1 when a wait
+// between tiles ran out (the state is lost).
+constexpr int kResidentDecision = 0, kResidentLost = 1, kResidentStatus = 2;
 
 template <typename T>
 struct ResidentArgs {

@@ -41,10 +41,11 @@
 // of them than compute units, and the host lets one resident launch run at a time, but another
 // process or stream may hold part of the GPU.  So a launch first agrees: the last workgroup to
 // start decides that the steps are made; one that has waited long decides that they are not, and
-// all leave with nothing written.  A kernel of one workgroup follows each launch and makes the
-// steps of such a one by itself, slowly, and tells the host not to try again.  (A cooperative
-// launch would see to it too, but costs 20 us and the host's wait for it, and on ROCm 7 its queue
-// slows the streams created after it: a batch's two lanes took 5.4 ms for 2.0 ms of work.)
+// all leave with nothing written.  The host reads the decision before it puts anything else of the
+// handle on the stream, and makes the steps of a launch that decided against them with the per-step
+// kernels.  (A cooperative launch would see to it too, but costs 20 us and the host's wait for it,
+// and on ROCm 7 its queue slows the streams created after it: a batch's two lanes took 5.4 ms for
+// 2.0 ms of work.)
 #include <type_traits>
 
 #include "rsg_device.h"
@@ -61,17 +62,19 @@ constexpr uint64_t kStartTicks = 2000000ull;
 __device__ __forceinline__ bool decided(uint32_t d, uint32_t seq) { return (d >> 1) == (seq & 0x7FFFFFFFu); }
 
 // Whether the launch's steps are made, once decided.  Called by one thread of each workgroup, which
-// was the last to start or not.
-__device__ __forceinline__ bool agree(uint32_t* decision, uint32_t seq, bool last) {
+// was the last to start or not; the one that decides tells the host.
+__device__ __forceinline__ bool agree(uint32_t* decision, int32_t* status, uint32_t seq, bool last) {
   uint64_t t0 = 0;
   for (;;) {
     uint32_t d = __hip_atomic_load(decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (decided(d, seq)) return d & 1;
     const uint64_t t = wall_clock64();
     if (t0 == 0) t0 = t;
-    if (last || t - t0 > kStartTicks)  // the first decision stands
-      __hip_atomic_compare_exchange_strong(decision, &d, 2 * seq + (last ? 1u : 0u), __ATOMIC_RELAXED,
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t mine = 2 * seq + (last ? 1u : 0u);
+    if ((last || t - t0 > kStartTicks) &&  // the first decision stands
+        __hip_atomic_compare_exchange_strong(decision, &d, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+      __hip_atomic_store(status + kResidentDecision, (int32_t)mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -442,7 +445,7 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
   };
 
   if (a.ntiles > 1) {
-    if (t == 0) go = agree(a.ctrl + 1, a.seq, last);
+    if (t == 0) go = agree(a.ctrl + 1, a.status, a.seq, last);
     __syncthreads();
     if (!go) return;
   }
@@ -539,117 +542,6 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
   }
 }
 
-// The steps of a launch whose tiles did not get onto the GPU together, by one workgroup from
-// memory: all nodes, then all cells, tile after tile.  Ends at once after any other launch.
-template <typename T>
-__global__ __launch_bounds__(1024) void resident_alone_kernel(ResidentArgs<T> a) {
-  if (__hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * a.seq + 1) return;
-  const int t = threadIdx.x, threads = blockDim.x;
-  T* const Sg[6] = {a.s.S0, a.s.S1, a.s.S2, a.s.S3, a.s.S4, a.s.S5};
-  T* const Vg[3] = {a.v.V0, a.v.V1, a.v.V2};
-  const VelocityArgs<T>& va = a.v;
-  const StressArgs<T>& sa = a.s;
-  for (int k = 0; k < a.nsteps; k++) {
-    const double* now = a.force + (size_t)k * a.nforce;
-    for (int b = 0; b < a.ntiles; b++) {
-      const ResidentTile tl = a.tiles[b];
-      for (int i = t; i < tl.nnode; i += threads) {
-        const v4u rec = reinterpret_cast<const v4u*>(a.nrec)[tl.node0 + i];
-        if (!(rec.w & kResidentOwner)) continue;
-        const int n = (int)(rec.w & ~kResidentOwner);
-        int c[8];
-        unpack12(rec, c);
-#pragma unroll
-        for (int q = 0; q < 8; q++)  // slots to cells
-          c[q] = c[q] < tl.ncell                ? (int)a.crec[4 * (size_t)(tl.cell0 + c[q]) + 3]
-                 : c[q] < tl.ncell + tl.nhalo ? a.hcell[tl.halo0 + c[q] - tl.ncell]
-                                              : -1;
-        T idt, sx, sy, sz, r[3];
-        int sp = -1;
-        if (va.key || va.lkey) {
-          const uint32_t key = resolve_key(va, va.lkey ? va.lkey[4 * (size_t)n + 3] : va.key[n], sp);
-          idt = va.cls[key >> kMatShift];
-          axis_spacings(va.axis, key, sx, sy, sz);
-        } else {
-          idt = va.idt[n];
-          sx = va.dnx[n];
-          sy = va.dny[n];
-          sz = va.dnz[n];
-          if (is_boxed(idt)) {
-            sp = unbox(idt);
-            idt = va.sp_idt[sp];
-          }
-        }
-        node_rates(
-            [&](int p, T(&f)[8], T(&g)[8]) {
-#pragma unroll
-              for (int q = 0; q < 8; q++) {
-                f[q] = c[q] >= 0 ? Sg[slot_comp(2 * p)][c[q]] : T(0);
-                g[q] = c[q] >= 0 ? Sg[slot_comp(2 * p + 1)][c[q]] : T(0);
-              }
-            },
-            sx, sy, sz, r);
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-          if (sp >= 0) r[d] = r[d] + (T)now[3 * a.ncls[sp] + d];
-          Vg[d][n] = Vg[d][n] + idt * r[d];
-          if (sp >= 0 && va.sp_sens[sp] >= 0) va.trace[(size_t)k * a.row + 3 * va.sp_sens[sp] + d] = (double)Vg[d][n];
-        }
-      }
-    }
-    __syncthreads();
-    for (int b = 0; b < a.ntiles; b++) {
-      const ResidentTile tl = a.tiles[b];
-      for (int i = t; i < tl.ncell; i += threads) {
-        const v4u rec = reinterpret_cast<const v4u*>(a.crec)[tl.cell0 + i];
-        const int e = (int)rec.w;
-        int c[8];
-        unpack12(rec, c);
-#pragma unroll
-        for (int q = 0; q < 8; q++) c[q] = (int)(a.nrec[4 * (size_t)(tl.node0 + c[q]) + 3] & ~kResidentOwner);
-        T sx, sy, sz, cc[21], d[6], s[6];
-        int sp = -1;
-        if (sa.key || sa.lkey) {
-          const uint32_t key = resolve_key(sa, sa.lkey ? sa.lkey[4 * (size_t)e + 3] : sa.key[e], sp);
-          axis_spacings(sa.axis, key, sx, sy, sz);
-#pragma unroll
-          for (int q = 0; q < 21; q++) cc[q] = sa.cls[(size_t)(key >> kMatShift) * kMatRow + q];
-        } else {
-          sx = sa.dcx[e];
-          sy = sa.dcy[e];
-          sz = sa.dcz[e];
-          if (is_boxed(sx)) {
-            sp = unbox(sx);
-            sx = sa.sp_dcx[sp];
-          }
-          cell_constants(sa, e, cc);
-        }
-        auto m = [&](int q) { return now[a.cforce0 + 6 * a.ccls[sp] + q]; };
-#pragma unroll
-        for (int q = 0; q < 6; q++) s[q] = Sg[q][e];
-        strain_rates<T>(
-            [&](T(&f)[8], T(&g)[8]) {
-#pragma unroll
-              for (int q = 0; q < 8; q++) {
-                f[q] = Vg[0][c[q]];
-                g[q] = Vg[1][c[q]];
-              }
-            },
-            [&](T(&f)[8]) {
-#pragma unroll
-              for (int q = 0; q < 8; q++) f[q] = Vg[2][c[q]];
-            },
-            sx, sy, sz, d);
-        voigt_update(sa.dt, cc, d, m, sp, s);
-#pragma unroll
-        for (int q = 0; q < 6; q++) Sg[q][e] = s[q];
-      }
-    }
-    __syncthreads();
-  }
-  if (t == 0) __hip_atomic_store(a.status + kResidentAlone, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 template <typename T, int THREADS, bool NKEY, bool CKEY>
 const void* resident_fn(bool rec) {
   return rec ? reinterpret_cast<const void*>(&resident_kernel<T, THREADS, NKEY, CKEY, true>)
@@ -673,10 +565,7 @@ hipError_t launch_resident(const ResidentArgs<T>& a, int threads, hipStream_t st
   const size_t lds = resident_lds_bytes(a.max_set, a.max_node, a.max_cell, sizeof(T), rec) +
                      (a.tables ? resident_table_bytes(sizeof(T)) : 0);
   void* args[1] = {const_cast<void*>(static_cast<const void*>(&a))};
-  const hipError_t e = hipLaunchKernel(fn, dim3(a.ntiles), dim3(threads), args, lds, st);
-  if (e != hipSuccess || a.ntiles == 1) return e;
-  hipLaunchKernelGGL(resident_alone_kernel<T>, dim3(1), dim3(1024), 0, st, a);
-  return hipGetLastError();
+  return hipLaunchKernel(fn, dim3(a.ntiles), dim3(threads), args, lds, st);
 }
 
 }  // namespace

@@ -1,8 +1,12 @@
 // faults.cpp -- failures on demand for the host code over its CPU stand-ins (hip_host_stub.cpp,
 // resident_stub.cpp).  TEST INFRASTRUCTURE ONLY: linked with --wrap, so that the calls named below
 // pass through here; a test sets the counters through ctypes.
+#include <hip/hip_runtime_api.h>
+
 #include <system_error>
 #include <thread>
+
+#include "../../pannde_amd/csrc/rsg_internal.h"
 
 extern "C" {
 
@@ -18,6 +22,79 @@ void NAME(__wrap_, START_THREAD)(std::thread* self, void* state, void (*depend)(
   if (fault_threads == 0) throw std::system_error(std::make_error_code(std::errc::resource_unavailable_try_again));
   if (fault_threads > 0) fault_threads--;
   NAME(__real_, START_THREAD)(self, state, depend);
+}
+
+// Resident launches that decide against their steps (and say so when the host has asked the event
+// that often), launches so far, and what the per-step kernels were launched with: the first
+// channel's amplitude and the trace row's address.
+int fault_refuse = 0, fault_late = 0;
+int fault_resident = 0, fault_velocity = 0, fault_stress = 0;
+double fault_amp[4096], fault_stress_amp[4096];
+const double* fault_trace[4096];
+}  // extern "C"
+
+namespace {
+int32_t* late_word = nullptr;
+int32_t late_value = 0;
+
+template <typename A, typename F>
+hipError_t resident(const A& a, F&& real) {
+  fault_resident++;
+  if (a.ntiles == 1) return real();
+  late_word = a.status + rsg::kResidentDecision;
+  if (fault_refuse == 0) {
+    *late_word = (int32_t)(2 * a.seq + 1);
+    return real();
+  }
+  fault_refuse--;
+  late_value = (int32_t)(2 * a.seq);
+  if (fault_late == 0) *late_word = late_value;
+  return hipSuccess;
+}
+template <typename A>
+void velocity(const A& a) {
+  fault_amp[fault_velocity % 4096] = a.amp[0];
+  fault_trace[fault_velocity++ % 4096] = a.trace;
+}
+template <typename A>
+void stress(const A& a) {
+  fault_stress_amp[fault_stress++ % 4096] = a.amp[0];
+}
+}  // namespace
+
+extern "C" {
+
+hipError_t __real_hipEventQuery(hipEvent_t e);
+hipError_t __wrap_hipEventQuery(hipEvent_t e) {
+  if (fault_late > 0) {
+    if (--fault_late == 0) *late_word = late_value;
+    return hipErrorNotReady;
+  }
+  return __real_hipEventQuery(e);
+}
+
+#define RESIDENT_F64 _ZN3rsg19launch_resident_f64ERKNS_12ResidentArgsIdEEiP12ihipStream_t
+#define RESIDENT_F32 _ZN3rsg19launch_resident_f32ERKNS_12ResidentArgsIfEEiP12ihipStream_t
+hipError_t NAME(__real_, RESIDENT_F64)(const rsg::ResidentArgs<double>& a, int threads, hipStream_t s);
+hipError_t NAME(__wrap_, RESIDENT_F64)(const rsg::ResidentArgs<double>& a, int threads, hipStream_t s) {
+  return resident(a, [&]() { return NAME(__real_, RESIDENT_F64)(a, threads, s); });
+}
+hipError_t NAME(__real_, RESIDENT_F32)(const rsg::ResidentArgs<float>& a, int threads, hipStream_t s);
+hipError_t NAME(__wrap_, RESIDENT_F32)(const rsg::ResidentArgs<float>& a, int threads, hipStream_t s) {
+  return resident(a, [&]() { return NAME(__real_, RESIDENT_F32)(a, threads, s); });
+}
+
+#define VELOCITY_F64 _ZN3rsg19launch_velocity_f64ERKNS_12VelocityArgsIdEEiP12ihipStream_t
+#define STRESS_F64 _ZN3rsg17launch_stress_f64ERKNS_10StressArgsIdEEiP12ihipStream_t
+hipError_t NAME(__real_, VELOCITY_F64)(const rsg::VelocityArgs<double>& a, int block, hipStream_t s);
+hipError_t NAME(__wrap_, VELOCITY_F64)(const rsg::VelocityArgs<double>& a, int block, hipStream_t s) {
+  velocity(a);
+  return NAME(__real_, VELOCITY_F64)(a, block, s);
+}
+hipError_t NAME(__real_, STRESS_F64)(const rsg::StressArgs<double>& a, int block, hipStream_t s);
+hipError_t NAME(__wrap_, STRESS_F64)(const rsg::StressArgs<double>& a, int block, hipStream_t s) {
+  stress(a);
+  return NAME(__real_, STRESS_F64)(a, block, s);
 }
 
 }  // extern "C"

@@ -65,3 +65,62 @@ for n in (0, 1, 2, 3, 5):
     assert same(s.get_state() + (s.traces(),), case), n
     s.close()
 ''')
+
+
+def test_refused_launch_is_made_by_the_per_step_kernels(lib):
+    """Whatever comes after a launch that decided against its steps first queues those steps, each
+    with its own amplitudes and trace row; no launch is put behind an undecided one."""
+    run(lib, r'''
+case = cases.al_block(seed=1, nx=20, ny=19, nz=18, nsteps=400, n_sensors=4)
+sig = case.force[0]
+def amplitude(k):
+    t = 0.0
+    for _ in range(k):
+        t += case.dt
+    return 0.125 * rsg.signal_eval(sig.signal_t, sig.signal_v, [t])[0]
+row = 8 * 3 * 4
+def check(n, first, base):
+    assert knob("fault_velocity").value == n and knob("fault_stress").value == n
+    amps = (ctypes.c_double * 4096).in_dll(rsg.lib(), "fault_amp")
+    samps = (ctypes.c_double * 4096).in_dll(rsg.lib(), "fault_stress_amp")
+    rows = (ctypes.c_size_t * 4096).in_dll(rsg.lib(), "fault_trace")
+    for k in range(n):
+        assert amps[k] == samps[k] == amplitude(first + k), k
+        assert rows[k] - rows[0] == row * k
+def reset(refuse, late):
+    for name, v in (("refuse", refuse), ("late", late), ("resident", 0), ("velocity", 0), ("stress", 0)):
+        knob("fault_" + name).value = v
+reads = dict(state=lambda s: s.get_state(), traces=lambda s: s.traces(), energy=lambda s: s.energy(),
+             sync=lambda s: s.synchronize(), step=lambda s: s.solve(1), zero=lambda s: s.solve(0),
+             set_state=lambda s: s.set_state(np.zeros((3, case.n_nodes)), None),
+             sources=lambda s: s.set_sources(case.force, []), sensors=lambda s: s.set_sensors(case.sensors))
+for name, read in reads.items():
+    for late in (0, 3):
+        s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+        reset(0, 0)
+        s.solve(7)  # made
+        reset(1, late)
+        s.solve(9)  # not made
+        assert knob("fault_resident").value == 1 and knob("fault_velocity").value == 0
+        read(s)
+        assert knob("fault_late").value == 0
+        check(9 + (name == "step"), 7, 0)
+        s.close()
+# a batch takes the handle with its steps queued
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+reset(1, 2)
+s.solve(9)
+b = rsg.Batch(rsg.RSG_FP64)
+b.remove(b.add(s, 0))
+check(9, 0, 0)
+b.close()
+s.close()
+# blocks of 256 steps: the second one is not launched resident once the first has refused
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+reset(99, 0)
+s.solve(400)
+assert knob("fault_resident").value == 1
+check(400, 0, 0)
+assert s.traces().shape[0] == 400
+s.close()
+''')
