@@ -347,7 +347,8 @@ struct rsg_instance {
   DevBuf<uint8_t> res_ncls, res_ccls;
   void* res_ctrl = nullptr;
   uint32_t res_seq = 0;            // launches so far
-  hipEvent_t res_event = nullptr;  // behind the last one
+  hipEvent_t res_event = nullptr;  // behind the last one, where it could be recorded
+  bool res_recorded = false;
   int32_t* res_status = nullptr;  // pinned, from the first resident launch on
   // the last launch of several tiles, until its decision is known: its steps (0: it is), first
   // step's amplitudes and trace row
@@ -1498,6 +1499,7 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
       return rsg::launch_resident_f32(a, h->res_threads, h->stream);
   };
   hipError_t e;
+  h->res_recorded = false;
   if (h->res_tiles == 1) {
     e = launch();
   } else {
@@ -1505,12 +1507,19 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
     ResidentOrder& o = resident_order();
     std::lock_guard<std::mutex> lock(o.mu);
     rsg_instance*& last = o.last[h->device];
-    if (last && last != h) HIP_TRY(rsg::resident_after(h->stream, last->res_event));
-    e = launch();
-    if (e == hipSuccess) e = hipEventRecord(h->res_event, h->stream);
-    if (e == hipSuccess) last = h;
+    e = last && last != h ? rsg::resident_after(h->stream, last->res_event) : hipSuccess;
+    if (e == hipSuccess) e = launch();
+    // without its record the launch is waited for by its stream, and a launch of another handle may
+    // meet it on the GPU and be refused
+    if (e == hipSuccess && hipEventRecord(h->res_event, h->stream) == hipSuccess) {
+      h->res_recorded = true;
+      last = h;
+    }
   }
-  if (e != hipSuccess) return fail(RSG_ERR_DEVICE, "resident launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {  // nothing was launched: the per-step kernels say whether the device works
+    h->res_tiles = 0;
+    return RSG_OK;
+  }
   h->res_seq++;
   *done = true;
   return RSG_OK;
@@ -1574,7 +1583,7 @@ int settle_resident(rsg_instance* h) {
   uint32_t d = decision();
   for (uint32_t spin = 1; d >> 1 != (h->res_seq & 0x7FFFFFFFu); spin++, d = decision()) {
     if (spin % 64) continue;
-    const hipError_t e = hipEventQuery(h->res_event);
+    const hipError_t e = h->res_recorded ? hipEventQuery(h->res_event) : hipStreamSynchronize(h->stream);
     if (e == hipSuccess) break;  // (a launch that has ended has decided)
     if (e != hipErrorNotReady) return fail(RSG_ERR_DEVICE, "resident launch: %s", hipGetErrorString(e));
     std::this_thread::yield();

@@ -29,6 +29,8 @@ void NAME(__wrap_, START_THREAD)(std::thread* self, void* state, void (*depend)(
 // channel's amplitude and the trace row's address.
 int fault_refuse = 0, fault_late = 0;
 int fault_resident = 0, fault_velocity = 0, fault_stress = 0;
+// resident launches that fail, and which of the event records from now on does (1: the next)
+int fault_launch = 0, fault_record = 0;
 double fault_amp[4096], fault_stress_amp[4096];
 const double* fault_trace[4096];
 }  // extern "C"
@@ -39,6 +41,7 @@ int32_t late_value = 0;
 
 template <typename A, typename F>
 hipError_t resident(const A& a, F&& real) {
+  if (fault_launch > 0 && fault_launch--) return hipErrorLaunchFailure;
   fault_resident++;
   if (a.ntiles == 1) return real();
   late_word = a.status + rsg::kResidentDecision;
@@ -71,6 +74,12 @@ hipError_t __wrap_hipEventQuery(hipEvent_t e) {
     return hipErrorNotReady;
   }
   return __real_hipEventQuery(e);
+}
+
+hipError_t __real_hipEventRecord(hipEvent_t e, hipStream_t s);
+hipError_t __wrap_hipEventRecord(hipEvent_t e, hipStream_t s) {
+  if (fault_record > 0 && --fault_record == 0) return hipErrorUnknown;
+  return __real_hipEventRecord(e, s);
 }
 
 #define RESIDENT_F64 _ZN3rsg19launch_resident_f64ERKNS_12ResidentArgsIdEEiP12ihipStream_t

@@ -124,3 +124,37 @@ check(400, 0, 0)
 assert s.traces().shape[0] == 400
 s.close()
 ''')
+
+
+def test_launch_without_its_event(lib):
+    """A resident launch whose event could not be recorded has been made all the same: its steps and
+    their time count once."""
+    run(lib, r'''
+case = cases.al_block(seed=1, nx=20, ny=19, nz=18, nsteps=24, n_sensors=4)
+t = 0.0
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+for n, record in ((7, 2), (8, 0), (9, 1)):  # the first call's amplitude upload records an event too
+    knob("fault_record").value = record
+    s.solve(n)
+    assert knob("fault_record").value == 0
+    for _ in range(n):
+        t += case.dt
+    assert s.time == t
+assert knob("fault_resident").value == 3 and knob("fault_velocity").value == 0
+assert same(s.get_state() + (s.traces(),), case)
+s.close()
+''')
+
+
+def test_failed_launch(lib):
+    """Steps that could not be launched resident are made by the per-step kernels."""
+    run(lib, r'''
+case = cases.al_block(seed=1, nx=20, ny=19, nz=18, nsteps=24, n_sensors=4)
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+knob("fault_launch").value = 1
+s.solve(7)
+s.solve(9)
+s.synchronize()
+assert knob("fault_resident").value == 0 and knob("fault_velocity").value == knob("fault_stress").value == 16
+s.close()
+''')
