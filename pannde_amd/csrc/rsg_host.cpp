@@ -254,6 +254,7 @@ void leave_resident_order(const rsg_instance* h) {
 }
 
 constexpr int64_t kCacheBytes = (int64_t)256 << 20;  // the GPU's memory-side cache
+constexpr int kLostV = 1, kLostS = 2, kLostTraces = 4;  // what a resident launch has lost
 constexpr int kBlockSteps = 256;   // steps whose amplitudes are staged per upload
 constexpr int kTraceCapSteps = 4096;
 
@@ -350,6 +351,7 @@ struct rsg_instance {
   hipEvent_t res_event = nullptr;  // behind the last one, where it could be recorded
   bool res_recorded = false;
   int32_t* res_status = nullptr;  // pinned, from the first resident launch on
+  int32_t res_lost = 0;  // kLost... of a launch whose tiles lost each other, until written again
   // the last launch of several tiles, until its decision is known: its steps (0: it is), first
   // step's amplitudes and trace row
   int32_t res_pending = 0;
@@ -1351,10 +1353,18 @@ int build_tables(rsg_instance* h) {
   return RSG_OK;
 }
 
-// Fails when a wait of the resident kernel ran out in work that has been synchronized.
-int check_resident(rsg_instance* h) {
-  if (h->res_status && __atomic_load_n(h->res_status + rsg::kResidentLost, __ATOMIC_RELAXED))
-    return fail(RSG_ERR_DEVICE, "the resident step kernel's workgroups lost each other");
+// Fails when a wait of the resident kernel ran out in work that has been synchronized and `part`
+// (kLostV, kLostS, kLostTraces) has not been replaced since.
+int check_resident(rsg_instance* h, int part) {
+  if (h->res_status && __atomic_load_n(h->res_status + rsg::kResidentLost, __ATOMIC_RELAXED)) {
+    __atomic_store_n(h->res_status + rsg::kResidentLost, 0, __ATOMIC_RELAXED);
+    h->res_lost = kLostV | kLostS | (h->sensors.empty() ? 0 : kLostTraces);
+    h->res_tiles = 0;
+  }
+  if (h->res_lost & part)
+    return fail(RSG_ERR_DEVICE, "the resident step kernel's workgroups lost each other: %s",
+                h->res_lost & part & kLostTraces ? "the recorded traces are lost until the sensors are set again"
+                                                 : "the state is lost until both its parts are written again");
   return RSG_OK;
 }
 
@@ -1368,7 +1378,7 @@ int flush_traces(rsg_instance* h) {
   HIP_TRY(copy_on(h->trace_host.data() + old, h->trace.p, (size_t)h->trace_dev_steps * row * sizeof(double),
                   hipMemcpyDeviceToHost, h->stream));
   h->trace_dev_steps = 0;
-  return check_resident(h);
+  return RSG_OK;
 }
 
 template <typename T>
@@ -1665,7 +1675,7 @@ int energy_on_stream(rsg_instance* h, double* work, double* kinetic, double* str
   double tot[2] = {0.0, 0.0};
   HIP_TRY(hipMemcpyAsync(tot, out, sizeof(tot), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
-  if (int rc = check_resident(h)) return rc;
+  if (int rc = check_resident(h, kLostV | kLostS)) return rc;
   if (kinetic) *kinetic = tot[0];
   if (strain) *strain = tot[1];
   return RSG_OK;
@@ -2469,6 +2479,8 @@ int rsg_set_sensors(rsg_handle h, int32_t n, const int32_t* nodes) {
   int rc = settle_resident(h);
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
+  (void)check_resident(h, 0);
+  h->res_lost &= ~kLostTraces;
   h->sensors.assign(nodes, nodes + n);
   h->trace_host.clear();
   h->trace_dev_steps = 0;
@@ -2573,20 +2585,25 @@ int rsg_get_state(rsg_handle h, double* V, double* S) {
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
   int rc = settle_resident(h);
   if (!rc) rc = transfer_state(h, V, S, false);
-  return rc ? rc : check_resident(h);
+  return rc ? rc : check_resident(h, kLostV | kLostS);
 }
 
 int rsg_set_state(rsg_handle h, const double* V, const double* S) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   if (h->in_batch) return fail(RSG_ERR_STATE, "the handle is in a batch; remove it first");
-  const int rc = settle_resident(h);
-  return rc ? rc : transfer_state(h, const_cast<double*>(V), const_cast<double*>(S), true);
+  int rc = settle_resident(h);
+  if (!rc) rc = transfer_state(h, const_cast<double*>(V), const_cast<double*>(S), true);
+  if (rc) return rc;
+  (void)check_resident(h, 0);  // what was lost before the write
+  h->res_lost &= ~((V ? kLostV : 0) | (S ? kLostS : 0));
+  return RSG_OK;
 }
 
 int rsg_get_traces(rsg_handle h, int64_t first, int64_t n, double* out) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   int rc = settle_resident(h);
   if (!rc) rc = flush_traces(h);
+  if (!rc) rc = check_resident(h, kLostTraces);
   if (rc) return rc;
   const size_t row = h->sensors.size() * 3;
   const int64_t have = row ? (int64_t)(h->trace_host.size() / row) : 0;
@@ -2603,7 +2620,7 @@ int rsg_synchronize(rsg_handle h) {
   if (int rc = settle_resident(h)) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
-  return check_resident(h);
+  return check_resident(h, kLostV | kLostS);
 }
 
 int rsg_get_time(rsg_handle h, double* time, int64_t* steps) {

@@ -31,6 +31,8 @@ int fault_refuse = 0, fault_late = 0;
 int fault_resident = 0, fault_velocity = 0, fault_stress = 0;
 // resident launches that fail, and which of the event records from now on does (1: the next)
 int fault_launch = 0, fault_record = 0;
+// resident launches whose tiles lose each other
+int fault_lost = 0;
 double fault_amp[4096], fault_stress_amp[4096];
 const double* fault_trace[4096];
 }  // extern "C"
@@ -43,6 +45,7 @@ template <typename A, typename F>
 hipError_t resident(const A& a, F&& real) {
   if (fault_launch > 0 && fault_launch--) return hipErrorLaunchFailure;
   fault_resident++;
+  if (fault_lost > 0 && fault_lost--) a.status[rsg::kResidentLost] = 1;
   if (a.ntiles == 1) return real();
   late_word = a.status + rsg::kResidentDecision;
   if (fault_refuse == 0) {

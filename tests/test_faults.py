@@ -158,3 +158,45 @@ s.synchronize()
 assert knob("fault_resident").value == 0 and knob("fault_velocity").value == knob("fault_stress").value == 16
 s.close()
 ''')
+
+
+def test_lost_state_is_replaced(lib):
+    """A state that a launch lost is refused until both its parts have been written again, the traces
+    until the sensors are set again."""
+    run(lib, r'''
+case = cases.al_block(seed=1, nx=20, ny=19, nz=18, nsteps=24, n_sensors=4)
+rng = np.random.default_rng(3)
+V, S = rng.standard_normal((3, case.n_nodes)), rng.standard_normal((6, case.n_cells))
+def refused(call):
+    try:
+        call()
+    except rsg.RSGError as e:
+        return "lost" in str(e)
+    return False
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+s.solve(7)
+knob("fault_lost").value = 1
+s.solve(8)
+s.solve(1)
+assert refused(s.synchronize) and refused(s.get_state) and refused(s.energy) and refused(s.traces)
+s.set_state(V, None)
+assert refused(s.get_state)
+s.set_state(None, S)
+assert all(np.array_equal(a, b) for a, b in zip(s.get_state(), (V, S)))
+s.synchronize()
+s.energy()
+assert refused(s.traces)
+s.set_sensors(case.sensors)
+assert s.traces(0, 0).shape[0] == 0
+assert knob("fault_resident").value == 2
+s.solve(9)
+assert knob("fault_resident").value == 2 and s.traces(0, 9).shape[0] == 9
+# the write that replaces the state may be the first call after the loss
+r = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+knob("fault_lost").value = 1
+r.solve(8)
+r.set_state(V, S)
+assert all(np.array_equal(a, b) for a, b in zip(r.get_state(), (V, S)))
+r.close()
+s.close()
+''')
