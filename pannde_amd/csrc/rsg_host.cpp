@@ -350,6 +350,7 @@ struct rsg_instance {
   uint32_t res_seq = 0;            // launches so far
   hipEvent_t res_event = nullptr;  // behind the last one, where it could be recorded
   bool res_recorded = false;
+  std::chrono::steady_clock::time_point res_not_before;  // after a refused launch
   int32_t* res_status = nullptr;  // pinned, from the first resident launch on
   int32_t res_lost = 0;  // kLost... of a launch whose tiles lost each other, until written again
   // the last launch of several tiles, until its decision is known: its steps (0: it is), first
@@ -1465,6 +1466,18 @@ int ensure_events(rsg_instance* h, size_t n) {
 // 58; 259,000 cells FP32 4 steps 49 / 46, 6 steps 63 / 68).
 constexpr int kResidentMinSteps = 5;
 
+// A handle steps with the per-step kernels for this long after a refused launch, which cost it 20 ms
+// of waiting: 2 % of its time while the GPU stays crowded, and the work that crowds it may end.
+constexpr std::chrono::seconds kResidentRetry(1);
+
+// Whether kb steps go into a resident launch.
+bool steps_resident(const rsg_instance* h, int kb) {
+  return h->res_tiles > 0 && h->res_nclasses >= 0 && kb >= (h->res_tiles == 1 ? 2 : kResidentMinSteps) &&
+         h->timing == 0 &&
+         (h->res_not_before == std::chrono::steady_clock::time_point() ||
+          std::chrono::steady_clock::now() >= h->res_not_before);
+}
+
 // kb steps in one launch of the resident kernel; *done says whether it was launched.
 template <typename T>
 int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const rsg::StressArgs<T>& sa,
@@ -1601,7 +1614,8 @@ int settle_resident(rsg_instance* h) {
   const int kb = h->res_pending;
   h->res_pending = 0;
   if (decision() != 2 * h->res_seq) return RSG_OK;
-  h->res_tiles = 0;  // the GPU is shared with work that keeps the tiles apart
+  // the GPU is shared with work that keeps the tiles apart: not again soon
+  h->res_not_before = std::chrono::steady_clock::now() + kResidentRetry;
   auto steps = [&](auto zero) {
     using T = decltype(zero);
     rsg::VelocityArgs<T> va;
@@ -1620,7 +1634,7 @@ int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* forc
   const size_t row = h->sensors.size() * 3;
   bool done = false;
   int rc;
-  if (h->res_tiles > 0 && h->res_nclasses >= 0 && kb >= (h->res_tiles == 1 ? 2 : kResidentMinSteps) && h->timing == 0) {
+  if (steps_resident(h, kb)) {
     va.trace = h->trace.p ? h->trace.p + (size_t)h->trace_dev_steps * row : nullptr;
     if ((rc = run_resident<T>(h, kb, va, sa, force_dev, row, &done))) return rc;
     if (done && h->res_tiles > 1) {

@@ -200,3 +200,25 @@ assert all(np.array_equal(a, b) for a, b in zip(r.get_state(), (V, S)))
 r.close()
 s.close()
 ''')
+
+
+def test_refused_launch_is_tried_again(lib):
+    """A refused launch keeps a handle off the resident kernel for a second, not for good."""
+    run(lib, r'''
+import time
+case = cases.al_block(seed=1, nx=20, ny=19, nz=18, nsteps=24, n_sensors=4)
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+knob("fault_refuse").value = 1
+t = time.monotonic()
+s.solve(7)
+s.solve(7)
+s.synchronize()
+if time.monotonic() - t < 0.9:
+    assert knob("fault_resident").value == 1 and knob("fault_velocity").value == 14
+time.sleep(1.1)
+n = knob("fault_velocity").value
+s.solve(7)
+s.synchronize()
+assert knob("fault_resident").value >= 2 and knob("fault_velocity").value == n
+s.close()
+''')
