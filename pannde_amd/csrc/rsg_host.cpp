@@ -30,7 +30,6 @@
 #include <ctime>
 #include <exception>
 #include <iterator>
-#include <map>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -330,23 +329,21 @@ struct rsg_instance {
   double* node_m = nullptr;    // node masses rho_n*dxn*dyn*dzn (energy)
   double* cell_vol = nullptr;  // cell volumes dxc*dyc*dzc (energy)
 
-  // resident stepping (res_tiles 0: the mesh has no plan)
-  int32_t res_tiles = 0, res_threads = 0, res_nexp = 0, res_set = 0, res_node = 0, res_cell = 0;
-  void* res_tile = nullptr;
-  void* res_crec = nullptr;
-  void* res_nrec = nullptr;
-  void* res_halo = nullptr;
-  void* res_hcell = nullptr;
-  void* res_xbuf = nullptr;
+  // resident stepping: the plan (ntiles 0: none, or none any more), its arrays on the host until the
+  // first resident launch puts them on the device, in front of the exchange buffers and of the
+  // kernel's records where these do not fit LDS
+  rsg::ResidentPlan res;
+  int32_t res_threads = 0;
+  bool res_records = false;  // in LDS
   size_t res_lds_room = 0;   // LDS a tile leaves free
-  void* res_work = nullptr;  // the kernel's records where they do not fit LDS
+  void* res_mem = nullptr;
   // source terms as the resident kernel takes them: one list of channels per class and component
   // (res_force: the node classes, 3 lists each, then the cell classes, 6 each); -1 node classes:
   // more classes than the kernel holds
   int32_t res_nclasses = -1;
   std::vector<std::vector<int32_t>> res_force;
-  DevBuf<uint8_t> res_ncls, res_ccls;
-  void* res_ctrl = nullptr;
+  std::vector<uint8_t> res_cls_h;  // class of each special node, then of each special cell
+  DevBuf<uint8_t> res_cls;         // released: not on the device since the last table build
   uint32_t res_seq = 0;            // launches so far
   hipEvent_t res_event = nullptr;  // behind the last one, where it could be recorded
   bool res_recorded = false;
@@ -414,6 +411,10 @@ struct rsg_instance {
   // queues all its uploads and waits once (finish_uploads)
   std::mutex hold_mu;
   std::vector<std::shared_ptr<const void>> held;
+  void hold(std::shared_ptr<const void> p) {
+    std::lock_guard<std::mutex> lock(hold_mu);
+    held.push_back(std::move(p));
+  }
 
   // device memory from the pool on the handle's stream, released with the handle
   int dalloc(void** p, size_t bytes) {
@@ -447,8 +448,7 @@ struct rsg_instance {
     amp[1].release();
     trace.release();
     partial.release();
-    res_ncls.release();
-    res_ccls.release();
+    res_cls.release();
     if (stream) (void)hipStreamSynchronize(stream);
     for (int i = 0; i < 2; i++) {
       if (stage[i]) (void)hipHostFree(stage[i]);
@@ -848,8 +848,7 @@ int queue_upload(rsg_instance* h, void* dst, std::vector<T>&& src) {
   if (src.empty()) return RSG_OK;
   auto keep = std::make_shared<std::vector<T>>(std::move(src));
   HIP_TRY(hipMemcpyAsync(dst, keep->data(), keep->size() * sizeof(T), hipMemcpyHostToDevice, h->stream));
-  std::lock_guard<std::mutex> lock(h->hold_mu);
-  h->held.push_back(std::move(keep));
+  h->hold(std::move(keep));
   return RSG_OK;
 }
 
@@ -1147,8 +1146,7 @@ int patch_keys(rsg_instance* h, uint32_t* dst, bool packed, const std::vector<ui
                            hipMemcpyHostToDevice, h->stream));
     a = e;
   }
-  std::lock_guard<std::mutex> lock(h->hold_mu);
-  h->held.push_back(std::move(rec));
+  h->hold(std::move(rec));
   return RSG_OK;
 }
 
@@ -1262,29 +1260,43 @@ int build_tables(rsg_instance* h) {
   // classes of equal term lists, for the resident kernel
   h->res_nclasses = -1;
   h->res_force.clear();
-  std::vector<uint8_t> ncls, ccls;
-  if (h->res_tiles > 0) {
-    std::map<std::vector<std::vector<int32_t>>, int32_t> seen;
-    auto classify = [&](const std::vector<int32_t>& off, const std::vector<int32_t>& term, int lists,
-                        std::vector<uint8_t>& cls) {
-      seen.clear();
-      cls.resize(off.size() / (lists + 1));
-      for (size_t s = 0; s < cls.size(); s++) {
-        std::vector<std::vector<int32_t>> key((size_t)lists);
-        for (int q = 0; q < lists; q++)
-          key[q].assign(term.begin() + off[s * (lists + 1) + q], term.begin() + off[s * (lists + 1) + q + 1]);
-        auto it = seen.emplace(std::move(key), (int32_t)seen.size()).first;
-        if ((size_t)it->second * lists == h->res_force.size() - (lists == 6 ? 3 * (size_t)h->res_nclasses : 0))
-          h->res_force.insert(h->res_force.end(), it->first.begin(), it->first.end());
-        if (it->second >= 127 || h->res_force.size() > (size_t)rsg::kResidentForces) return false;
-        cls[s] = (uint8_t)it->second;
+  h->res_cls_h.clear();
+  h->res_cls.release();
+  if (h->res.ntiles > 0) {
+    // appends the classes of `off`'s entities, numbered by first appearance, to res_cls_h and their
+    // lists to res_force; their number, or -1 when the kernel does not hold that many
+    auto classify = [&](const std::vector<int32_t>& off, const std::vector<int32_t>& term, int lists) -> int32_t {
+      std::unordered_map<uint64_t, std::vector<std::pair<const int32_t*, uint8_t>>> seen;
+      int32_t classes = 0;
+      for (const int32_t* o = off.data(); o < off.data() + off.size(); o += lists + 1) {
+        uint64_t hash = 0x9E3779B97F4A7C15ull;
+        auto mix = [&](uint32_t w) {
+          hash = (hash ^ w) * 0xFF51AFD7ED558CCDull;
+          hash ^= hash >> 29;
+        };
+        for (int q = 1; q <= lists; q++) mix((uint32_t)(o[q] - o[0]));
+        for (int32_t k = o[0]; k < o[lists]; k++) mix((uint32_t)term[k]);
+        auto equal = [&](const int32_t* r) {
+          for (int q = 1; q <= lists; q++)
+            if (r[q] - r[0] != o[q] - o[0]) return false;
+          return std::equal(term.begin() + o[0], term.begin() + o[lists], term.begin() + r[0]);
+        };
+        auto& list = seen[hash];
+        int32_t cls = -1;
+        for (auto& e : list)
+          if (equal(e.first)) cls = e.second;
+        if (cls < 0) {
+          cls = classes++;
+          if (cls >= 127 || h->res_force.size() + lists > (size_t)rsg::kResidentForces) return -1;
+          for (int q = 0; q < lists; q++) h->res_force.emplace_back(term.begin() + o[q], term.begin() + o[q + 1]);
+          list.push_back({o, (uint8_t)cls});
+        }
+        h->res_cls_h.push_back((uint8_t)cls);
       }
-      return true;
+      return classes;
     };
-    if (classify(sp_off, terms, 3, ncls)) {
-      h->res_nclasses = (int32_t)seen.size();
-      if (!classify(csp_off, cterms, 6, ccls)) h->res_nclasses = -1;
-    }
+    const int32_t nodes = classify(sp_off, terms, 3);
+    if (nodes >= 0 && classify(csp_off, cterms, 6) >= 0) h->res_nclasses = nodes;
     if (h->res_nclasses < 0) h->res_force.clear();
   }
   // class-table form: keys carry the special flag; the special tables carry the class
@@ -1301,10 +1313,10 @@ int build_tables(rsg_instance* h) {
     if (h->precision == RSG_FP64) return queue_upload(h, buf.p, std::vector<double>(v));
     return queue_upload(h, buf.p, std::vector<float>(v.begin(), v.end()));
   };
-  auto put_int = [&](auto& buf, const auto& v) -> int {
+  auto put_int = [&](DevBuf<int32_t>& buf, const std::vector<int32_t>& v) -> int {
     int rc = buf.alloc(std::max<size_t>(1, v.size()), h->stream);
     if (rc) return rc;
-    return queue_upload(h, buf.p, std::decay_t<decltype(v)>(v));
+    return queue_upload(h, buf.p, std::vector<int32_t>(v));
   };
   int rc;
   if ((rc = put_real(h->sp_node_val, sp_idt))) return rc;
@@ -1316,10 +1328,6 @@ int build_tables(rsg_instance* h) {
   if ((rc = put_int(h->cell_terms, cterms))) return rc;
   if ((rc = put_int(h->sp_node_key, sp_nkey))) return rc;
   if ((rc = put_int(h->sp_cell_key, sp_ckey))) return rc;
-  if (h->res_nclasses >= 0) {
-    if ((rc = put_int(h->res_ncls, ncls))) return rc;
-    if ((rc = put_int(h->res_ccls, ccls))) return rc;
-  }
   if (h->v_lkey || h->nkey) {
     if ((rc = patch_keys(h, h->v_lkey ? h->v_lkey : h->nkey, h->v_lkey != nullptr, h->v_lconn_h, h->nkey_h,
                          node_boxes, h->v_flagged)))
@@ -1349,6 +1357,8 @@ int build_tables(rsg_instance* h) {
     }
     if (!h->stage_ev[b]) HIP_TRY(hipEventCreateWithFlags(&h->stage_ev[b], hipEventDisableTiming));
   }
+  // no channels: the resident kernel's sums (of nodes that are sensors only) are zero
+  if (h->channels.empty()) HIP_TRY(hipMemsetAsync(h->amp[0].p, 0, h->amp[0].bytes(), h->stream));
   if ((rc = finish_uploads(h))) return rc;
   h->tables_dirty = false;
   return RSG_OK;
@@ -1360,7 +1370,7 @@ int check_resident(rsg_instance* h, int part) {
   if (h->res_status && __atomic_load_n(h->res_status + rsg::kResidentLost, __ATOMIC_RELAXED)) {
     __atomic_store_n(h->res_status + rsg::kResidentLost, 0, __ATOMIC_RELAXED);
     h->res_lost = kLostV | kLostS | (h->sensors.empty() ? 0 : kLostTraces);
-    h->res_tiles = 0;
+    h->res.ntiles = 0;
   }
   if (h->res_lost & part)
     return fail(RSG_ERR_DEVICE, "the resident step kernel's workgroups lost each other: %s",
@@ -1472,10 +1482,42 @@ constexpr std::chrono::seconds kResidentRetry(1);
 
 // Whether kb steps go into a resident launch.
 bool steps_resident(const rsg_instance* h, int kb) {
-  return h->res_tiles > 0 && h->res_nclasses >= 0 && kb >= (h->res_tiles == 1 ? 2 : kResidentMinSteps) &&
+  return h->res.ntiles > 0 && h->res_nclasses >= 0 && kb >= (h->res.ntiles == 1 ? 2 : kResidentMinSteps) &&
          h->timing == 0 &&
          (h->res_not_before == std::chrono::steady_clock::time_point() ||
           std::chrono::steady_clock::now() >= h->res_not_before);
+}
+
+// Bytes of the exchange buffers, as many as a multiple of 16 that the records follow.
+size_t resident_exchange_bytes(const rsg_instance* h) { return ((size_t)24 * h->res.nexp * h->elt() + 15) / 16 * 16; }
+
+// Puts the plan on the device with the first resident launch, and the classes of the source terms
+// with the first after a table build: a handle that is never stepped resident (in a batch, step by
+// step) holds no device memory for it.  False when there is no memory: for now the per-step kernels
+// do without.
+bool resident_on_device(rsg_instance* h) {
+  rsg::ResidentPlan& p = h->res;
+  bool ok = true;
+  if (!h->res_mem) {
+    const size_t work = h->res_records ? 0 : (size_t)16 * p.ntiles * (p.max_node + p.max_cell);
+    ok = h->dalloc(&h->res_mem, p.bytes + resident_exchange_bytes(h) + work) == RSG_OK;
+    if (ok) {
+      const hipError_t e = hipMemcpyAsync(h->res_mem, p.block.get(), p.bytes, hipMemcpyHostToDevice, h->stream);
+      h->hold(std::shared_ptr<const void>(p.block.release(), [](const void* b) { delete[] (const char*)b; }));
+      if (e != hipSuccess) {
+        p.ntiles = 0;
+        return false;
+      }
+    }
+  }
+  if (ok && !h->res_cls.p)
+    ok = h->res_cls.alloc(std::max<size_t>(1, h->res_cls_h.size()), h->stream) == RSG_OK &&
+         queue_upload(h, h->res_cls.p, std::vector<uint8_t>(h->res_cls_h)) == RSG_OK;
+  if (!ok) {
+    h->res_cls.release();
+    h->res_not_before = std::chrono::steady_clock::now() + kResidentRetry;
+  }
+  return ok;
 }
 
 // kb steps in one launch of the resident kernel; *done says whether it was launched.
@@ -1487,29 +1529,32 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
     HIP_TRY(hipHostMalloc((void**)&h->res_status, rsg::kResidentStatus * sizeof(int32_t), hipHostMallocDefault));
     memset(h->res_status, 0, rsg::kResidentStatus * sizeof(int32_t));
   }
+  if (!resident_on_device(h)) return RSG_OK;
+  const rsg::ResidentPlan& p = h->res;
+  char* const mem = (char*)h->res_mem;
   rsg::ResidentArgs<T> a;
   a.v = va;
   a.s = sa;
-  a.tiles = (const rsg::ResidentTile*)h->res_tile;
-  a.crec = (const uint32_t*)h->res_crec;
-  a.nrec = (const uint32_t*)h->res_nrec;
-  a.halo = (const int32_t*)h->res_halo;
-  a.hcell = (const int32_t*)h->res_hcell;
-  a.xbuf = (unsigned long long*)h->res_xbuf;
-  a.ctrl = (uint32_t*)h->res_ctrl;
+  a.tiles = (const rsg::ResidentTile*)(mem + p.tiles);
+  a.crec = (const uint32_t*)(mem + p.crec);
+  a.nrec = (const uint32_t*)(mem + p.nrec);
+  a.halo = (const int32_t*)(mem + p.halo);
+  a.hcell = (const int32_t*)(mem + p.hcell);
+  a.xbuf = (unsigned long long*)(mem + p.bytes);
+  a.ctrl = (uint32_t*)(mem + p.ctrl);
   a.seq = h->res_seq + 1;
   a.status = h->res_status;
   a.nsteps = kb;
-  a.ntiles = h->res_tiles;
-  a.nexp = h->res_nexp;
-  a.max_set = h->res_set;
-  a.max_node = h->res_node;
-  a.max_cell = h->res_cell;
-  a.work = (uint32_t*)h->res_work;
+  a.ntiles = p.ntiles;
+  a.nexp = p.nexp;
+  a.max_set = p.max_set;
+  a.max_node = p.max_node;
+  a.max_cell = p.max_cell;
+  a.work = h->res_records ? nullptr : (uint32_t*)(mem + p.bytes + resident_exchange_bytes(h));
   a.force = force;
   a.nforce = (int32_t)h->res_force.size();
-  a.ncls = h->res_ncls.p;
-  a.ccls = h->res_ccls.p;
+  a.ncls = h->res_cls.p;
+  a.ccls = h->res_cls.p + h->n_sp_node;
   a.cforce0 = 3 * h->res_nclasses;
   a.row = (int32_t)row;
   a.nmat = std::max(0, h->n_nmat);
@@ -1523,7 +1568,7 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   };
   hipError_t e;
   h->res_recorded = false;
-  if (h->res_tiles == 1) {
+  if (p.ntiles == 1) {
     e = launch();
   } else {
     if (!h->res_event) HIP_TRY(hipEventCreateWithFlags(&h->res_event, hipEventDisableTiming));
@@ -1540,7 +1585,7 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
     }
   }
   if (e != hipSuccess) {  // nothing was launched: the per-step kernels say whether the device works
-    h->res_tiles = 0;
+    h->res.ntiles = 0;
     return RSG_OK;
   }
   h->res_seq++;
@@ -1613,6 +1658,10 @@ int settle_resident(rsg_instance* h) {
   }
   const int kb = h->res_pending;
   h->res_pending = 0;
+  {  // what was copied before the launch has arrived
+    std::lock_guard<std::mutex> lock(h->hold_mu);
+    h->held.clear();
+  }
   if (decision() != 2 * h->res_seq) return RSG_OK;
   // the GPU is shared with work that keeps the tiles apart: not again soon
   h->res_not_before = std::chrono::steady_clock::now() + kResidentRetry;
@@ -1637,7 +1686,7 @@ int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* forc
   if (steps_resident(h, kb)) {
     va.trace = h->trace.p ? h->trace.p + (size_t)h->trace_dev_steps * row : nullptr;
     if ((rc = run_resident<T>(h, kb, va, sa, force_dev, row, &done))) return rc;
-    if (done && h->res_tiles > 1) {
+    if (done && h->res.ntiles > 1) {
       h->res_pending = kb;
       h->res_amp = amp_dev;
       h->res_row = h->trace_dev_steps;
@@ -2349,37 +2398,28 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     const int32_t max_tiles = nc <= 500 ? 1 : std::min<int32_t>(cus, nc / 64);
     rsg::ResidentMesh m{nn, nc, h->cells.data(), h->node_cells.data(), h->cell_of.data(), h->cell_at.data(),
                         h->node_at.data(), {X[0], X[1], X[2]}, {lo[0], lo[1], lo[2]}, {hmin[0], hmin[1], hmin[2]}};
-    rsg::ResidentPlan p;
+    rsg::ResidentPlan& p = h->res;
     auto run = [](int n, auto&& fn) { parallel_each(n, fn); };
-    if (!rsg::build_resident_plan(m, max_tiles, lds, e, run, p)) return RSG_OK;
+    try {
+      if (!rsg::build_resident_plan(m, max_tiles, lds, e, run, p)) return RSG_OK;
+    } catch (const std::bad_alloc&) {  // no memory for it: the handle does without
+      p = rsg::ResidentPlan();
+      return RSG_OK;
+    }
     // Threads past a tile's nodes still pay: other waves read the halo and take the cells (32,000
     // cells in tiles of 125, 216 nodes: FP64 5.0 us a step with 256 threads, 4.4 with 512, FP32 4.0
     // and 3.5; tiles of 512, 729 nodes: 7.7 with 512, 6.4 with 1024, FP32 5.6 and 4.5; tiles of 64,
     // 125 nodes: no difference).
     h->res_threads = p.max_node <= 128 ? 256 : p.max_node <= 512 ? 512 : 1024;
-    h->res_nexp = p.nexp;
-    h->res_set = p.max_set;
-    h->res_node = p.max_node;
-    h->res_cell = p.max_cell;
-    const int32_t tiles = (int32_t)p.tiles.size();
-    int rc;
-    if ((rc = upload(h.get(), &h->res_tile, std::move(p.tiles)))) return rc;
-    if ((rc = upload(h.get(), &h->res_crec, std::move(p.crec)))) return rc;
-    if ((rc = upload(h.get(), &h->res_nrec, std::move(p.nrec)))) return rc;
-    if ((rc = upload(h.get(), &h->res_halo, std::move(p.halo)))) return rc;
-    if ((rc = upload(h.get(), &h->res_hcell, std::move(p.hcell)))) return rc;
-    if ((rc = h->dalloc(&h->res_xbuf, (size_t)24 * p.nexp * e))) return rc;
+    h->res_records = rsg::resident_lds_bytes(p.max_set, p.max_node, p.max_cell, e, true) +
+                         rsg::kResidentStaticLds <= lds;
+    h->res_lds_room = lds - rsg::kResidentStaticLds -
+                      rsg::resident_lds_bytes(p.max_set, p.max_node, p.max_cell, e, h->res_records);
     // PANNDE_RSG_RESIDENT=alone (tests): the count of started tiles begins where it never meets a
     // launch's total, so every launch decides against its steps
     const char* alone = std::getenv("PANNDE_RSG_RESIDENT");
     const uint32_t started = alone && !strcmp(alone, "alone") ? 1u << 31 : 0;
-    if ((rc = upload(h.get(), &h->res_ctrl, std::vector<uint32_t>{started, 0}))) return rc;
-    const bool records = rsg::resident_lds_bytes(h->res_set, h->res_node, h->res_cell, e, true) +
-                             rsg::kResidentStaticLds <= lds;
-    if (!records && (rc = h->dalloc(&h->res_work, (size_t)16 * tiles * (h->res_node + h->res_cell)))) return rc;
-    h->res_lds_room = lds - rsg::kResidentStaticLds -
-                      rsg::resident_lds_bytes(h->res_set, h->res_node, h->res_cell, e, records);
-    h->res_tiles = tiles;
+    memcpy(p.block.get() + p.ctrl, &started, sizeof(started));
     return RSG_OK;
   };
   {
@@ -2523,8 +2563,7 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
   for (int32_t done = 0; done < nsteps;) {
     if ((rc = settle_resident(h))) return rc;
     int kb = std::min(kBlockSteps, nsteps - done);
-    // no channels: a buffer no term reads, and zero sums (of special nodes that are sensors only)
-    const bool none = nch == 0 && nf == 0;
+    const bool none = nch == 0;  // a buffer that no term reads, and zero sums
     const double* amp = none ? h->amp[0].p : nullptr;
     const double* force = h->amp[0].p;
     if (!none && !amplitudes && h->win_first >= 0 && h->steps >= h->win_first &&
@@ -2685,7 +2724,8 @@ int rsg_device_bytes(rsg_handle h, int64_t* bytes) {
   *bytes = h->dev_bytes + (int64_t)(h->sp_node_val.bytes() + h->sp_node_off.bytes() +
                                     h->sp_node_sens.bytes() + h->node_terms.bytes() +
                                     h->sp_cell_val.bytes() + h->sp_cell_off.bytes() +
-                                    h->cell_terms.bytes() + h->amp[0].bytes() + h->amp[1].bytes() +
+                                    h->cell_terms.bytes() + h->res_cls.bytes() + h->amp[0].bytes() +
+                                    h->amp[1].bytes() +
                                     h->trace.bytes() + h->partial.bytes());
   return RSG_OK;
 }

@@ -35,6 +35,8 @@ int fault_launch = 0, fault_record = 0;
 int fault_lost = 0;
 double fault_amp[4096], fault_stress_amp[4096];
 const double* fault_trace[4096];
+// device allocations so far, and whether there is no memory for more
+int fault_allocs = 0, fault_no_memory = 0;
 }  // extern "C"
 
 namespace {
@@ -77,6 +79,13 @@ hipError_t __wrap_hipEventQuery(hipEvent_t e) {
     return hipErrorNotReady;
   }
   return __real_hipEventQuery(e);
+}
+
+hipError_t __real_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s);
+hipError_t __wrap_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s) {
+  if (fault_no_memory) return hipErrorOutOfMemory;
+  fault_allocs++;
+  return __real_hipMallocFromPoolAsync(p, bytes, pool, s);
 }
 
 hipError_t __real_hipEventRecord(hipEvent_t e, hipStream_t s);
