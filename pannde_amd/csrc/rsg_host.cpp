@@ -194,6 +194,23 @@ hipError_t device_alloc(void** p, size_t bytes, hipStream_t s) {
 // other stream still uses it.
 void device_free(void* p, hipStream_t s) { (void)hipFreeAsync(p, s); }
 
+// Makes `device` the thread's current device while it lives: an entry point may be called with
+// another one current, and what it creates must be on the handle's.
+struct DeviceScope {
+  int before = -1;
+  hipError_t status;
+  explicit DeviceScope(int device) {
+    int now = device;
+    status = hipGetDevice(&now);
+    if (status == hipSuccess && now != device && (status = hipSetDevice(device)) == hipSuccess) before = now;
+  }
+  ~DeviceScope() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+  DeviceScope(const DeviceScope&) = delete;
+  DeviceScope& operator=(const DeviceScope&) = delete;
+};
+
 // A copy ordered on s (a non-blocking stream) that has finished when this returns.  hipMemcpy
 // runs on the null stream and waits for the work queued on every stream, so while batches keep
 // other streams busy a handle's uploads would wait behind them.
@@ -1525,6 +1542,8 @@ template <typename T>
 int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const rsg::StressArgs<T>& sa,
                  const double* force, size_t row, bool* done) {
   *done = false;
+  DeviceScope scope(h->device);
+  HIP_TRY(scope.status);
   if (!h->res_status) {
     HIP_TRY(hipHostMalloc((void**)&h->res_status, rsg::kResidentStatus * sizeof(int32_t), hipHostMallocDefault));
     memset(h->res_status, 0, rsg::kResidentStatus * sizeof(int32_t));
@@ -1850,6 +1869,8 @@ int transfer_chunks(rsg_instance* h, double* V, double* S, bool write) {
 
 int transfer_state(rsg_instance* h, double* V, double* S, bool write) {
   if (!V && !S) return RSG_OK;
+  DeviceScope scope(h->device);
+  HIP_TRY(scope.status);
   try {
     if (!rsg::launch_state_f64) return transfer_state_on_host(h, V, S, write);
     int rc;

@@ -3,8 +3,10 @@
 // pass through here; a test sets the counters through ctypes.
 #include <hip/hip_runtime_api.h>
 
+#include <mutex>
 #include <system_error>
 #include <thread>
+#include <unordered_map>
 
 #include "../../pannde_amd/csrc/rsg_internal.h"
 
@@ -40,6 +42,18 @@ int fault_allocs = 0, fault_no_memory = 0;
 }  // extern "C"
 
 namespace {
+thread_local int current = 0;
+std::mutex devices_mu;
+std::unordered_map<const void*, int> devices;
+void put_device(const void* p) {
+  std::lock_guard<std::mutex> lock(devices_mu);
+  devices[p] = current;
+}
+int device_of(const void* p) {
+  std::lock_guard<std::mutex> lock(devices_mu);
+  return devices.count(p) ? devices[p] : 0;
+}
+
 int32_t* late_word = nullptr;
 int32_t late_value = 0;
 
@@ -83,13 +97,42 @@ hipError_t __wrap_hipEventQuery(hipEvent_t e) {
 
 hipError_t __real_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s);
 hipError_t __wrap_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s) {
+  if (device_of(s) != current) return hipErrorInvalidValue;
   if (fault_no_memory) return hipErrorOutOfMemory;
   fault_allocs++;
   return __real_hipMallocFromPoolAsync(p, bytes, pool, s);
 }
 
+// Two devices: a stream or event is on the device current where it was made, memory is taken from
+// the current device's pool, and mixing them is an error.
+void fault_set_device(int d) { current = d; }
+void fault_get_device(int* d) { *d = current; }
+hipError_t __real_hipGetDevice(int* d);
+hipError_t __wrap_hipGetDevice(int* d) {
+  *d = current;
+  return hipSuccess;
+}
+hipError_t __real_hipSetDevice(int d);
+hipError_t __wrap_hipSetDevice(int d) {
+  current = d;
+  return hipSuccess;
+}
+hipError_t __real_hipStreamCreateWithFlags(hipStream_t* s, unsigned int flags);
+hipError_t __wrap_hipStreamCreateWithFlags(hipStream_t* s, unsigned int flags) {
+  const hipError_t e = __real_hipStreamCreateWithFlags(s, flags);
+  put_device(*s);
+  return e;
+}
+hipError_t __real_hipEventCreateWithFlags(hipEvent_t* v, unsigned flags);
+hipError_t __wrap_hipEventCreateWithFlags(hipEvent_t* v, unsigned flags) {
+  const hipError_t e = __real_hipEventCreateWithFlags(v, flags);
+  put_device(*v);
+  return e;
+}
+
 hipError_t __real_hipEventRecord(hipEvent_t e, hipStream_t s);
 hipError_t __wrap_hipEventRecord(hipEvent_t e, hipStream_t s) {
+  if (device_of(e) != device_of(s)) return hipErrorInvalidHandle;
   if (fault_record > 0 && --fault_record == 0) return hipErrorUnknown;
   return __real_hipEventRecord(e, s);
 }

@@ -259,3 +259,24 @@ for late in (0, 1):  # none for the plan; none for the classes of a new table bu
     assert knob("fault_velocity").value - v == 9 and knob("fault_resident").value == r
     s.close()
 ''')
+
+
+def test_calls_with_another_device_current(lib):
+    """Steps and state transfers use the handle's device, whichever is current, and leave that one
+    current: with one transfer thread and with several."""
+    run(lib, r'''
+for dims in ((20, 19, 18), (46, 40, 40)):
+    case = cases.al_block(seed=1, nx=dims[0], ny=dims[1], nz=dims[2], nsteps=16, n_sensors=4)
+    s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+    for device in (1, 0):
+        rsg.lib().fault_set_device(device)
+        s.set_state(np.zeros((3, case.n_nodes)), np.zeros((6, case.n_cells)))
+        s.solve(8)
+        now = ctypes.c_int(-1)
+        state = s.get_state()
+        rsg.lib().fault_get_device(ctypes.byref(now))
+        assert now.value == device
+        s.synchronize()
+    assert knob("fault_velocity").value == 0
+    s.close()
+''')
