@@ -1868,6 +1868,7 @@ int transfer_chunks(rsg_instance* h, double* V, double* S, bool write) {
 }
 
 int transfer_state(rsg_instance* h, double* V, double* S, bool write) {
+  HIP_TRY(hipStreamSynchronize(h->stream));
   if (!V && !S) return RSG_OK;
   DeviceScope scope(h->device);
   HIP_TRY(scope.status);

@@ -95,6 +95,14 @@ hipError_t __wrap_hipEventQuery(hipEvent_t e) {
   return __real_hipEventQuery(e);
 }
 
+// waits for a stream so far
+int fault_waits = 0;
+hipError_t __real_hipStreamSynchronize(hipStream_t s);
+hipError_t __wrap_hipStreamSynchronize(hipStream_t s) {
+  __atomic_fetch_add(&fault_waits, 1, __ATOMIC_RELAXED);
+  return __real_hipStreamSynchronize(s);
+}
+
 hipError_t __real_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s);
 hipError_t __wrap_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s) {
   if (device_of(s) != current) return hipErrorInvalidValue;

@@ -280,3 +280,18 @@ for dims in ((20, 19, 18), (46, 40, 40)):
     assert knob("fault_velocity").value == 0
     s.close()
 ''')
+
+
+def test_state_calls_wait_for_the_stream(lib):
+    """rsg_get_state and rsg_set_state return with the handle's queued steps finished, also when no
+    array is asked for."""
+    run(lib, r'''
+case = cases.al_block(seed=1, nx=9, ny=8, nz=7, nsteps=9, n_sensors=4)
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+for call in (rsg.lib().rsg_get_state, rsg.lib().rsg_set_state):
+    s.solve(9)
+    n = knob("fault_waits").value
+    assert call(s._h, None, None) == rsg.RSG_OK
+    assert knob("fault_waits").value > n
+s.close()
+''')
