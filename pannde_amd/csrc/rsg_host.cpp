@@ -22,6 +22,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -220,6 +221,82 @@ hipError_t copy_on(void* dst, const void* src, size_t bytes, hipMemcpyKind kind,
   return e;
 }
 
+// Pinned memory for state transfers, which hipHostFree would give back only once every stream of the
+// device is idle.  A chunk and its event belong to a device's pool and serve one transfer at a time;
+// a transfer that finds none free makes one, up to kPinnedChunks for the device (32 MiB), and past
+// that shares what there is: it goes on with fewer, or waits for its first.  They are kept for the
+// transfers to come until the process ends, like the device pool's memory.
+struct PinnedChunk {
+  void* p = nullptr;
+  hipEvent_t ev = nullptr;
+};
+constexpr int kPinnedChunks = 16;
+struct PinnedPool {
+  std::mutex mu;
+  std::condition_variable given;
+  struct Device {
+    std::vector<PinnedChunk> idle;
+    int made = 0;
+  };
+  std::unordered_map<int, Device> devices;
+};
+PinnedPool& pinned_pool() {
+  static PinnedPool* const o = new PinnedPool();  // (handles may go after static objects)
+  return *o;
+}
+
+// Up to `want` chunks of the device, which is current; at least one, unless there is no pinned
+// memory at all.
+std::vector<PinnedChunk> take_chunks(int device, int want) {
+  PinnedPool& o = pinned_pool();
+  std::vector<PinnedChunk> got;
+  got.reserve((size_t)want);
+  std::unique_lock<std::mutex> lock(o.mu);
+  PinnedPool::Device& d = o.devices[device];
+  d.idle.reserve(kPinnedChunks);  // giving back takes no memory
+  while ((int)got.size() < want) {
+    if (!d.idle.empty()) {
+      got.push_back(d.idle.back());
+      d.idle.pop_back();
+      continue;
+    }
+    bool made = false;
+    if (d.made < kPinnedChunks) {
+      d.made++;
+      lock.unlock();
+      PinnedChunk c;
+      made = hipHostMalloc(&c.p, rsg::kStateChunk * sizeof(double), hipHostMallocDefault) == hipSuccess;
+      if (made && hipEventCreateWithFlags(&c.ev, hipEventDisableTiming) != hipSuccess) {
+        (void)hipHostFree(c.p);
+        made = false;
+      }
+      lock.lock();
+      if (made)
+        got.push_back(c);
+      else
+        d.made--;
+    }
+    if (made) continue;
+    if (!got.empty() || d.made == 0) break;
+    o.given.wait(lock, [&]() { return !d.idle.empty() || d.made == 0; });
+  }
+  return got;
+}
+
+// Gives a chunk back that no work uses any more, or drops one that work may still use.
+void give_chunk(int device, const PinnedChunk& c, bool idle) {
+  PinnedPool& o = pinned_pool();
+  {
+    std::lock_guard<std::mutex> lock(o.mu);
+    PinnedPool::Device& d = o.devices[device];
+    if (idle)
+      d.idle.push_back(c);
+    else
+      d.made--;
+  }
+  o.given.notify_all();
+}
+
 // A device buffer owned by its handle, from the device pool on the handle's stream: released
 // on reallocation, and by the handle before it destroys that stream.
 template <typename T>
@@ -373,12 +450,9 @@ struct rsg_instance {
   const double* res_amp = nullptr;
   int64_t res_row = 0;
 
-  // state transfers: the caller -> internal maps on the device (from the first transfer on) and
-  // each transfer thread's chunk of pinned memory
+  // state transfers: the caller -> internal maps on the device, from the first transfer on
   void* node_at_d = nullptr;
   void* cell_at_d = nullptr;
-  std::vector<void*> chunk;
-  std::vector<hipEvent_t> chunk_ev;
 
   // source / sensor tables
   std::vector<Channel> channels;
@@ -474,10 +548,6 @@ struct rsg_instance {
     leave_resident_order(this);
     if (res_event) (void)hipEventDestroy(res_event);
     if (res_status) (void)hipHostFree(res_status);
-    for (void* c : chunk)
-      if (c) (void)hipHostFree(c);
-    for (hipEvent_t e : chunk_ev)
-      if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : tev) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -1799,17 +1869,18 @@ int transfer_state_on_host(rsg_instance* h, double* V, double* S, bool write) {
 // between the state and pinned memory, reordered, and a host thread copies it.  A state of more
 // than 128 Ki values takes up to setup_threads() threads, each with a chunk of its own, so
 // launches, bus and host copies overlap (one thread's copy of fresh pages is far below the bus).
+// *done: false when there is no pinned memory and nothing was moved.
 template <typename T>
-int transfer_chunks(rsg_instance* h, double* V, double* S, bool write) {
+int transfer_chunks(rsg_instance* h, double* V, double* S, bool write, bool* done) {
   const int64_t nv = (int64_t)3 * h->nn, g0 = V ? 0 : nv, g1 = S ? nv + (int64_t)6 * h->nc : nv;
   const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
-  const int threads = (int)std::max<int64_t>(1, std::min<int64_t>({(g1 - g0) >> 17, setup_threads(), hw}));
+  const int most = (int)std::max<int64_t>(1, std::min<int64_t>({(g1 - g0) >> 17, setup_threads(), hw, kPinnedChunks}));
+  const std::vector<PinnedChunk> pinned = take_chunks(h->device, most);
+  const int threads = (int)pinned.size();
+  *done = threads > 0;
+  if (threads == 0) return RSG_OK;
   const int64_t size = std::min<int64_t>(rsg::kStateChunk, (g1 - g0 + threads - 1) / threads);
   const int64_t chunks = (g1 - g0 + size - 1) / size;
-  if ((int)h->chunk.size() < threads) {
-    h->chunk.resize(threads, nullptr);
-    h->chunk_ev.resize(threads, nullptr);
-  }
   rsg::StateArgs<T> a;
   for (int d = 0; d < 3; d++) a.V[d] = (T*)h->V[d];
   for (int s = 0; s < 6; s++) a.S[s] = (T*)h->S[s];
@@ -1832,13 +1903,7 @@ int transfer_chunks(rsg_instance* h, double* V, double* S, bool write) {
   };
   auto work = [&](int w) -> int {
     if (w > 0) HIP_TRY(hipSetDevice(h->device));
-    if (!h->chunk[w]) {
-      // sized for this handle's largest transfer
-      const size_t most = std::min<int64_t>(rsg::kStateChunk, nv + (int64_t)6 * h->nc) * sizeof(T);
-      HIP_TRY(hipHostMalloc(&h->chunk[w], most, hipHostMallocDefault));
-    }
-    if (!h->chunk_ev[w]) HIP_TRY(hipEventCreateWithFlags(&h->chunk_ev[w], hipEventDisableTiming));
-    T* c = (T*)h->chunk[w];
+    T* const c = (T*)pinned[w].p;
     for (int64_t k = w; k < chunks; k += threads) {
       const int64_t g = g0 + k * size;
       const int n = (int)std::min<int64_t>(size, g1 - g);
@@ -1847,21 +1912,31 @@ int transfer_chunks(rsg_instance* h, double* V, double* S, bool write) {
         HIP_TRY(rsg::launch_state_f64(a, g, n, c, write, h->stream));
       else
         HIP_TRY(rsg::launch_state_f32(a, g, n, c, write, h->stream));
-      HIP_TRY(hipEventRecord(h->chunk_ev[w], h->stream));
-      HIP_TRY(hipEventSynchronize(h->chunk_ev[w]));  // the chunk is the thread's again
+      HIP_TRY(hipEventRecord(pinned[w].ev, h->stream));
+      HIP_TRY(hipEventSynchronize(pinned[w].ev));  // the chunk is the thread's again
       if (!write) copy(g, n, c);
     }
     return RSG_OK;
   };
-  std::vector<int> rcs((size_t)threads, RSG_OK);
-  std::vector<std::string> errs((size_t)threads);
-  parallel_tasks(threads, [&](int w) {
-    rcs[w] = work(w);
-    if (rcs[w]) errs[w] = g_last_error;
-  });
+  std::array<int, kPinnedChunks> rcs;
+  std::array<std::string, kPinnedChunks> errs;
+  rcs.fill(RSG_ERR_NOMEM);
+  bool idle = true;
+  try {
+    parallel_tasks(threads, [&](int w) {
+      rcs[w] = work(w);
+      if (rcs[w]) errs[w] = g_last_error;
+    });
+  } catch (...) {
+    idle = false;
+  }
+  // after a failure a launch that uses a chunk may be on the stream still
+  for (int w = 0; w < threads; w++) idle = idle && rcs[w] == RSG_OK;
+  idle = idle || hipStreamSynchronize(h->stream) == hipSuccess;
+  for (auto& c : pinned) give_chunk(h->device, c, idle);
   for (int w = 0; w < threads; w++)
     if (rcs[w]) {
-      g_last_error = errs[w];
+      g_last_error = errs[w].empty() ? "host allocation failed" : errs[w];
       return rcs[w];
     }
   return RSG_OK;
@@ -1874,13 +1949,16 @@ int transfer_state(rsg_instance* h, double* V, double* S, bool write) {
   HIP_TRY(scope.status);
   try {
     if (!rsg::launch_state_f64) return transfer_state_on_host(h, V, S, write);
+    bool done = false;
     int rc;
     if (!h->node_at_d) {
       if (!h->cell_at_d && (rc = upload(h, &h->cell_at_d, std::vector<int32_t>(h->cell_at)))) return rc;
       if ((rc = upload(h, &h->node_at_d, std::vector<int32_t>(h->node_at)))) return rc;
       if ((rc = finish_uploads(h))) return rc;
     }
-    return h->precision == RSG_FP64 ? transfer_chunks<double>(h, V, S, write) : transfer_chunks<float>(h, V, S, write);
+    rc = h->precision == RSG_FP64 ? transfer_chunks<double>(h, V, S, write, &done)
+                                  : transfer_chunks<float>(h, V, S, write, &done);
+    return rc || done ? rc : fail(RSG_ERR_NOMEM, "no pinned memory for the transfer");
   } catch (const std::bad_alloc&) {
     return fail(RSG_ERR_NOMEM, "host allocation failed");
   }

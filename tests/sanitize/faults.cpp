@@ -95,6 +95,19 @@ hipError_t __wrap_hipEventQuery(hipEvent_t e) {
   return __real_hipEventQuery(e);
 }
 
+// pinned allocations made and freed so far
+int fault_pinned = 0, fault_unpinned = 0;
+hipError_t __real_hipHostMalloc(void** p, size_t bytes, unsigned int flags);
+hipError_t __wrap_hipHostMalloc(void** p, size_t bytes, unsigned int flags) {
+  __atomic_fetch_add(&fault_pinned, 1, __ATOMIC_RELAXED);
+  return __real_hipHostMalloc(p, bytes, flags);
+}
+hipError_t __real_hipHostFree(void* p);
+hipError_t __wrap_hipHostFree(void* p) {
+  __atomic_fetch_add(&fault_unpinned, 1, __ATOMIC_RELAXED);
+  return __real_hipHostFree(p);
+}
+
 // waits for a stream so far
 int fault_waits = 0;
 hipError_t __real_hipStreamSynchronize(hipStream_t s);
@@ -107,7 +120,7 @@ hipError_t __real_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t po
 hipError_t __wrap_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s) {
   if (device_of(s) != current) return hipErrorInvalidValue;
   if (fault_no_memory) return hipErrorOutOfMemory;
-  fault_allocs++;
+  __atomic_fetch_add(&fault_allocs, 1, __ATOMIC_RELAXED);
   return __real_hipMallocFromPoolAsync(p, bytes, pool, s);
 }
 

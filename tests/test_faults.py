@@ -295,3 +295,31 @@ for call in (rsg.lib().rsg_get_state, rsg.lib().rsg_set_state):
     assert knob("fault_waits").value > n
 s.close()
 ''')
+
+
+def test_transfers_share_pinned_memory(lib):
+    """State transfers take their pinned chunks from a pool of the process: destroying a handle frees
+    none (which would wait for every stream of the device), many handles make no more than the pool
+    holds, and transfers of several threads at once move the right values."""
+    run(lib, r'''
+import threading
+case = cases.al_block(seed=1, nx=46, ny=40, nz=40, nsteps=1, n_sensors=0)
+solvers = [rsg.DeviceSolver.from_case(case, p) for p in (rsg.RSG_FP64, rsg.RSG_FP32) * 4]
+bad = []
+def work(i):
+    rng = np.random.default_rng(i)
+    for _ in range(3):
+        V, S = (rng.integers(-99, 99, (k, n)).astype(float) for k, n in ((3, case.n_nodes), (6, case.n_cells)))
+        solvers[i].set_state(V, S)
+        if not all(np.array_equal(a, b) for a, b in zip(solvers[i].get_state(), (V, S))):
+            bad.append(i)
+threads = [threading.Thread(target=work, args=(i,)) for i in range(len(solvers))]
+for t in threads:
+    t.start()
+for t in threads:
+    t.join()
+assert not bad and 1 <= knob("fault_pinned").value <= 16
+for s in solvers:
+    s.close()
+assert knob("fault_unpinned").value == 0
+''')
