@@ -297,6 +297,48 @@ void give_chunk(int device, const PinnedChunk& c, bool idle) {
   o.given.notify_all();
 }
 
+// The status words of handles that step resident, in pinned pages shared by the handles of a device:
+// a handle gives its words back when it goes (its stream is idle), the pages stay.
+union StatusWords {
+  int32_t words[16];
+  StatusWords* next;  // idle ones, in a list
+};
+constexpr int kStatusPage = 64;
+struct StatusPool {
+  std::mutex mu;
+  std::unordered_map<int, StatusWords*> idle;  // by device
+};
+StatusPool& status_pool() {
+  static StatusPool* const o = new StatusPool();
+  return *o;
+}
+// Zeroed words for a handle of the device, which is current; null when there is no memory.
+int32_t* take_status(int device) {
+  StatusPool& o = status_pool();
+  std::lock_guard<std::mutex> lock(o.mu);
+  StatusWords*& idle = o.idle[device];
+  if (!idle) {
+    StatusWords* page = nullptr;
+    if (hipHostMalloc((void**)&page, kStatusPage * sizeof(*page), hipHostMallocDefault) != hipSuccess) return nullptr;
+    for (int i = 0; i < kStatusPage; i++) {
+      page[i].next = idle;
+      idle = &page[i];
+    }
+  }
+  StatusWords* const s = idle;
+  idle = s->next;
+  memset(s, 0, sizeof(*s));
+  return s->words;
+}
+void give_status(int device, int32_t* words) {
+  StatusPool& o = status_pool();
+  std::lock_guard<std::mutex> lock(o.mu);
+  StatusWords*& idle = o.idle[device];
+  StatusWords* const s = reinterpret_cast<StatusWords*>(words);
+  s->next = idle;
+  idle = s;
+}
+
 // A device buffer owned by its handle, from the device pool on the handle's stream: released
 // on reallocation, and by the handle before it destroys that stream.
 template <typename T>
@@ -547,7 +589,7 @@ struct rsg_instance {
     }
     leave_resident_order(this);
     if (res_event) (void)hipEventDestroy(res_event);
-    if (res_status) (void)hipHostFree(res_status);
+    if (res_status) give_status(device, res_status);
     for (hipEvent_t e : tev) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -1579,13 +1621,13 @@ bool steps_resident(const rsg_instance* h, int kb) {
 size_t resident_exchange_bytes(const rsg_instance* h) { return ((size_t)24 * h->res.nexp * h->elt() + 15) / 16 * 16; }
 
 // Puts the plan on the device with the first resident launch, and the classes of the source terms
-// with the first after a table build: a handle that is never stepped resident (in a batch, step by
+// with the first after a table build, and takes the status words: a handle that is never stepped resident (in a batch, step by
 // step) holds no device memory for it.  False when there is no memory: for now the per-step kernels
 // do without.
 bool resident_on_device(rsg_instance* h) {
   rsg::ResidentPlan& p = h->res;
-  bool ok = true;
-  if (!h->res_mem) {
+  bool ok = h->res_status || (h->res_status = take_status(h->device));
+  if (ok && !h->res_mem) {
     const size_t work = h->res_records ? 0 : (size_t)16 * p.ntiles * (p.max_node + p.max_cell);
     ok = h->dalloc(&h->res_mem, p.bytes + resident_exchange_bytes(h) + work) == RSG_OK;
     if (ok) {
@@ -1596,6 +1638,10 @@ bool resident_on_device(rsg_instance* h) {
         return false;
       }
     }
+  }
+  if (ok && p.ntiles > 1 && !h->res_event) {
+    ok = hipEventCreateWithFlags(&h->res_event, hipEventDisableTiming) == hipSuccess;
+    if (!ok) h->res_event = nullptr;
   }
   if (ok && !h->res_cls.p)
     ok = h->res_cls.alloc(std::max<size_t>(1, h->res_cls_h.size()), h->stream) == RSG_OK &&
@@ -1614,10 +1660,6 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   *done = false;
   DeviceScope scope(h->device);
   HIP_TRY(scope.status);
-  if (!h->res_status) {
-    HIP_TRY(hipHostMalloc((void**)&h->res_status, rsg::kResidentStatus * sizeof(int32_t), hipHostMallocDefault));
-    memset(h->res_status, 0, rsg::kResidentStatus * sizeof(int32_t));
-  }
   if (!resident_on_device(h)) return RSG_OK;
   const rsg::ResidentPlan& p = h->res;
   char* const mem = (char*)h->res_mem;
@@ -1660,7 +1702,6 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   if (p.ntiles == 1) {
     e = launch();
   } else {
-    if (!h->res_event) HIP_TRY(hipEventCreateWithFlags(&h->res_event, hipEventDisableTiming));
     ResidentOrder& o = resident_order();
     std::lock_guard<std::mutex> lock(o.mu);
     rsg_instance*& last = o.last[h->device];

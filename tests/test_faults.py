@@ -323,3 +323,29 @@ for s in solvers:
     s.close()
 assert knob("fault_unpinned").value == 0
 ''')
+
+
+def test_status_words_are_shared(lib):
+    """Handles that step resident take their status words from pages of the process: destroying one
+    frees no pinned memory, and the words serve the next handle, zeroed."""
+    run(lib, r'''
+case = cases.al_block(seed=1, nx=9, ny=8, nz=7, nsteps=9, n_sensors=4)
+case.force = []  # no sources: no pinned staging of amplitudes either
+def stepped():
+    s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+    s.solve(9)
+    s.synchronize()
+    return s
+solvers = [stepped() for _ in range(100)]
+assert knob("fault_resident").value == 100 and knob("fault_pinned").value == 2
+knob("fault_lost").value = 1
+lost = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+lost.solve(9)
+for s in solvers + [lost]:
+    s.close()
+solvers = [stepped() for _ in range(128)]
+assert knob("fault_pinned").value == 2
+for s in solvers:
+    s.close()
+assert knob("fault_unpinned").value == 0
+''')
