@@ -42,12 +42,12 @@ template <typename T>
 hipError_t launch(const StateArgs<T>& a, int64_t g0, int n, T* chunk, bool write, hipStream_t s) {
   if (n <= 0 || n > kStateChunk || g0 < 0 || g0 + n > (int64_t)3 * a.nn + (int64_t)6 * a.nc || !chunk)
     return hipErrorInvalidValue;
-  const int grid = (n + 255) / 256;
-  if (write)
-    hipLaunchKernelGGL(state_write_kernel<T>, dim3(grid), dim3(256), 0, s, a, g0, n, (const T*)chunk);
-  else
-    hipLaunchKernelGGL(state_read_kernel<T>, dim3(grid), dim3(256), 0, s, a, g0, n, chunk);
-  return hipGetLastError();
+  // (hipLaunchKernel's own result: the thread's last error may be another call's)
+  const void* const fn = write ? reinterpret_cast<const void*>(&state_write_kernel<T>)
+                               : reinterpret_cast<const void*>(&state_read_kernel<T>);
+  StateArgs<T> arg = a;
+  void* args[4] = {&arg, &g0, &n, &chunk};
+  return hipLaunchKernel(fn, dim3((n + 255) / 256), dim3(256), args, 0, s);
 }
 
 }  // namespace
