@@ -195,6 +195,11 @@ hipError_t device_alloc(void** p, size_t bytes, hipStream_t s) {
 // other stream still uses it.
 void device_free(void* p, hipStream_t s) { (void)hipFreeAsync(p, s); }
 
+// (see rsg::forget_error; host code without the kernel library has no launchers that ask)
+void forget_error() {
+  if (rsg::forget_error) rsg::forget_error();
+}
+
 // Makes `device` the thread's current device while it lives: an entry point may be called with
 // another one current, and what it creates must be on the handle's.
 struct DeviceScope {
@@ -270,6 +275,7 @@ std::vector<PinnedChunk> take_chunks(int device, int want) {
         (void)hipHostFree(c.p);
         made = false;
       }
+      if (!made) forget_error();
       lock.lock();
       if (made)
         got.push_back(c);
@@ -492,9 +498,7 @@ struct rsg_instance {
   const double* res_amp = nullptr;
   int64_t res_row = 0;
 
-  // state transfers: the caller -> internal maps on the device, from the first transfer on
-  void* node_at_d = nullptr;
-  void* cell_at_d = nullptr;
+  int32_t* order = nullptr;  // node_at, then cell_at, on the device: from the first state transfer on
 
   // source / sensor tables
   std::vector<Channel> channels;
@@ -1647,6 +1651,7 @@ bool resident_on_device(rsg_instance* h) {
     ok = h->res_cls.alloc(std::max<size_t>(1, h->res_cls_h.size()), h->stream) == RSG_OK &&
          queue_upload(h, h->res_cls.p, std::vector<uint8_t>(h->res_cls_h)) == RSG_OK;
   if (!ok) {
+    forget_error();
     h->res_cls.release();
     h->res_not_before = std::chrono::steady_clock::now() + kResidentRetry;
   }
@@ -1712,9 +1717,12 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
     if (e == hipSuccess && hipEventRecord(h->res_event, h->stream) == hipSuccess) {
       h->res_recorded = true;
       last = h;
+    } else if (e == hipSuccess) {
+      forget_error();
     }
   }
   if (e != hipSuccess) {  // nothing was launched: the per-step kernels say whether the device works
+    forget_error();
     h->res.ntiles = 0;
     return RSG_OK;
   }
@@ -1874,10 +1882,10 @@ int energy_on_stream(rsg_instance* h, double* work, double* kinetic, double* str
   return RSG_OK;
 }
 
-// The state as host arrays through whole-array copies, reordered here: for builds of the host
-// code without the kernels of rsg_state.hip.
+// The state as host arrays through whole-array copies, reordered here: where there is no device
+// memory for the maps or no pinned memory for the chunks (a state can always be read), and in builds
+// of the host code without the kernels of rsg_state.hip.
 int transfer_state_on_host(rsg_instance* h, double* V, double* S, bool write) {
-  HIP_TRY(hipStreamSynchronize(h->stream));
   const size_t e = h->elt();
   std::vector<char> buf((size_t)std::max(h->nn, h->nc) * e);
   auto move = [&](void* dev, int32_t n, const std::vector<int32_t>& of, double* host) -> int {
@@ -1925,8 +1933,8 @@ int transfer_chunks(rsg_instance* h, double* V, double* S, bool write, bool* don
   rsg::StateArgs<T> a;
   for (int d = 0; d < 3; d++) a.V[d] = (T*)h->V[d];
   for (int s = 0; s < 6; s++) a.S[s] = (T*)h->S[s];
-  a.node_at = (const int32_t*)h->node_at_d;
-  a.cell_at = (const int32_t*)h->cell_at_d;
+  a.node_at = h->order;
+  a.cell_at = h->order + h->nn;
   a.nn = h->nn;
   a.nc = h->nc;
   // values [g, g + n) between a chunk and the caller's arrays
@@ -1990,16 +1998,22 @@ int transfer_state(rsg_instance* h, double* V, double* S, bool write) {
   HIP_TRY(scope.status);
   try {
     if (!rsg::launch_state_f64) return transfer_state_on_host(h, V, S, write);
-    bool done = false;
-    int rc;
-    if (!h->node_at_d) {
-      if (!h->cell_at_d && (rc = upload(h, &h->cell_at_d, std::vector<int32_t>(h->cell_at)))) return rc;
-      if ((rc = upload(h, &h->node_at_d, std::vector<int32_t>(h->node_at)))) return rc;
-      if ((rc = finish_uploads(h))) return rc;
+    if (!h->order) {
+      const size_t nodes = (size_t)h->nn * sizeof(int32_t), cells = (size_t)h->nc * sizeof(int32_t);
+      void* p = nullptr;
+      if (h->dalloc(&p, nodes + cells) != RSG_OK) {
+        forget_error();
+        return transfer_state_on_host(h, V, S, write);
+      }
+      int32_t* const o = (int32_t*)p;  // (the transfers wait for the copies: same stream)
+      HIP_TRY(hipMemcpyAsync(o, h->node_at.data(), nodes, hipMemcpyHostToDevice, h->stream));
+      HIP_TRY(hipMemcpyAsync(o + h->nn, h->cell_at.data(), cells, hipMemcpyHostToDevice, h->stream));
+      h->order = o;
     }
-    rc = h->precision == RSG_FP64 ? transfer_chunks<double>(h, V, S, write, &done)
-                                  : transfer_chunks<float>(h, V, S, write, &done);
-    return rc || done ? rc : fail(RSG_ERR_NOMEM, "no pinned memory for the transfer");
+    bool done = false;
+    const int rc = h->precision == RSG_FP64 ? transfer_chunks<double>(h, V, S, write, &done)
+                                            : transfer_chunks<float>(h, V, S, write, &done);
+    return rc || done ? rc : transfer_state_on_host(h, V, S, write);
   } catch (const std::bad_alloc&) {
     return fail(RSG_ERR_NOMEM, "host allocation failed");
   }

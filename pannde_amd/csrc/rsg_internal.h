@@ -282,6 +282,9 @@ constexpr size_t kResidentStaticLds = 2 * kResidentForces * 8 + 192;  // and wha
 RSG_WEAK hipError_t resident_limits(int* cus, size_t* lds);
 // Work queued on s from now on waits for the event.
 RSG_WEAK hipError_t resident_after(hipStream_t s, hipEvent_t e);
+// Drops the thread's last HIP error, where what failed is done without: the launchers that ask for
+// the last error would report it as theirs.
+RSG_WEAK void forget_error();
 // threads: 256, 512 or 1024 per workgroup.
 RSG_WEAK hipError_t launch_resident_f64(const ResidentArgs<double>& a, int threads, hipStream_t s);
 RSG_WEAK hipError_t launch_resident_f32(const ResidentArgs<float>& a, int threads, hipStream_t s);

@@ -565,9 +565,7 @@ hipError_t launch_resident(const ResidentArgs<T>& a, int threads, hipStream_t st
   const size_t lds = resident_lds_bytes(a.max_set, a.max_node, a.max_cell, sizeof(T), rec) +
                      (a.tables ? resident_table_bytes(sizeof(T)) : 0);
   void* args[1] = {const_cast<void*>(static_cast<const void*>(&a))};
-  const hipError_t e = hipLaunchKernel(fn, dim3(a.ntiles), dim3(threads), args, lds, st);
-  if (e != hipSuccess) (void)hipGetLastError();  // not the next launch's error
-  return e;
+  return hipLaunchKernel(fn, dim3(a.ntiles), dim3(threads), args, lds, st);
 }
 
 }  // namespace
@@ -581,6 +579,8 @@ hipError_t resident_limits(int* cus, size_t* lds) {
   *lds = (size_t)bytes;
   return hipSuccess;
 }
+
+void forget_error() { (void)hipGetLastError(); }
 
 hipError_t resident_after(hipStream_t s, hipEvent_t e) { return hipStreamWaitEvent(s, e, 0); }
 

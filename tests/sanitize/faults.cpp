@@ -95,10 +95,11 @@ hipError_t __wrap_hipEventQuery(hipEvent_t e) {
   return __real_hipEventQuery(e);
 }
 
-// pinned allocations made and freed so far
-int fault_pinned = 0, fault_unpinned = 0;
+// pinned allocations made and freed so far, and whether there is no pinned memory for more
+int fault_pinned = 0, fault_unpinned = 0, fault_no_pinned = 0;
 hipError_t __real_hipHostMalloc(void** p, size_t bytes, unsigned int flags);
 hipError_t __wrap_hipHostMalloc(void** p, size_t bytes, unsigned int flags) {
+  if (fault_no_pinned) return hipErrorOutOfMemory;
   __atomic_fetch_add(&fault_pinned, 1, __ATOMIC_RELAXED);
   return __real_hipHostMalloc(p, bytes, flags);
 }

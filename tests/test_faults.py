@@ -349,3 +349,22 @@ for s in solvers:
     s.close()
 assert knob("fault_unpinned").value == 0
 ''')
+
+
+def test_state_without_memory_for_the_transfer(lib):
+    """A state can be read and written when the device is full or no memory can be pinned, and goes
+    through the device again once there is some."""
+    run(lib, r'''
+rng = np.random.default_rng(3)
+for precision in (rsg.RSG_FP64, rsg.RSG_FP32):
+    for lack in ("fault_no_memory", "fault_no_pinned"):
+        case = cases.al_block(seed=1, nx=46, ny=40, nz=40, nsteps=1, n_sensors=0)
+        s = rsg.DeviceSolver.from_case(case, precision)
+        for n in (1, 0, 0):
+            knob(lack).value = n
+            V, S = (rng.integers(-99, 99, (k, n)).astype(float) for k, n in ((3, case.n_nodes), (6, case.n_cells)))
+            s.set_state(V, S)
+            assert all(np.array_equal(a, b) for a, b in zip(s.get_state(), (V, S))), lack
+        s.close()
+assert knob("fault_pinned").value > 0
+''')
