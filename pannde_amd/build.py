@@ -16,7 +16,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 DEVICE_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 HOST_FLAGS = ["-x", "c++", "-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
-              "-I/opt/rocm/include", "-Wall", "-Wno-unused-function"]
+              "-I/opt/rocm/include", "-Wall", "-Wno-unused-function", "-DRSG_LIBRARY"]
 
 
 def _run(cmd, verbose):
@@ -61,7 +61,7 @@ def build(verbose=False):
         raise RuntimeError("\n".join(failed))
     tmp = OUT + ".tmp"
     _run([HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950"] + objs +
-         ["-L/opt/rocm/lib", "-lrocprofiler-sdk-roctx", "-Wl,-rpath,/opt/rocm/lib", "-o", tmp], verbose)
+         ["-L/opt/rocm/lib", "-lrocprofiler-sdk-roctx", "-Wl,-rpath,/opt/rocm/lib", "-Wl,--no-undefined", "-o", tmp], verbose)
     os.replace(tmp, OUT)
     # the native mesh builder of the case generator (host code only)
     _run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-Wall", "-shared", "-fPIC",

@@ -197,7 +197,7 @@ void device_free(void* p, hipStream_t s) { (void)hipFreeAsync(p, s); }
 
 // (see rsg::forget_error; host code without the kernel library has no launchers that ask)
 void forget_error() {
-  if (rsg::forget_error) rsg::forget_error();
+  if (rsg::linked(rsg::forget_error)) rsg::forget_error();
 }
 
 // Makes `device` the thread's current device while it lives: an entry point may be called with
@@ -1997,7 +1997,7 @@ int transfer_state(rsg_instance* h, double* V, double* S, bool write) {
   DeviceScope scope(h->device);
   HIP_TRY(scope.status);
   try {
-    if (!rsg::launch_state_f64) return transfer_state_on_host(h, V, S, write);
+    if (!rsg::linked(rsg::launch_state_f64)) return transfer_state_on_host(h, V, S, write);
     if (!h->order) {
       const size_t nodes = (size_t)h->nn * sizeof(int32_t), cells = (size_t)h->nc * sizeof(int32_t);
       void* p = nullptr;
@@ -2541,7 +2541,7 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
   const bool chosen = tuning && (tuning->block_velocity || tuning->block_stress || tuning->per_thread_velocity ||
                                  tuning->per_thread_stress || tuning->lds_velocity || tuning->lds_stress);
   auto resident_part = [&]() -> int {
-    if (!rsg::resident_limits || chosen || !h->incidence_exact) return RSG_OK;
+    if (!rsg::linked(rsg::resident_limits) || chosen || !h->incidence_exact) return RSG_OK;
     int cus = 0;
     size_t lds = 0;
     HIP_TRY(rsg::resident_limits(&cus, &lds));

@@ -275,9 +275,18 @@ inline size_t resident_lds_bytes(int max_set, int max_node, int max_cell, size_t
 }
 constexpr size_t kResidentStaticLds = 2 * kResidentForces * 8 + 192;  // and what it declares itself
 
-// These launchers, and those of the state transfers, live in the kernel library only: builds of
-// the host code without it step with the per-step kernels and reorder states on the host.
+// These launchers, and those of the state transfers, may be left out of builds of the host code alone
+// (the sanitizers'), which step with the per-step kernels and reorder states on the host.  The
+// library is built with RSG_LIBRARY, where one that is missing fails the link.
+#ifdef RSG_LIBRARY
+#define RSG_WEAK
+#else
 #define RSG_WEAK __attribute__((weak))
+#endif
+template <typename F>
+bool linked(F* launcher) {
+  return launcher != nullptr;
+}
 // Compute units of the current device, and LDS bytes a workgroup may take.
 RSG_WEAK hipError_t resident_limits(int* cus, size_t* lds);
 // Work queued on s from now on waits for the event.
