@@ -384,8 +384,8 @@ struct ResidentOrder {
   std::unordered_map<int, rsg_instance*> last;  // by device
 };
 ResidentOrder& resident_order() {
-  static ResidentOrder o;
-  return o;
+  static ResidentOrder* const o = new ResidentOrder();  // (handles may go after static objects)
+  return *o;
 }
 // Before the handle's event goes (its stream is idle).
 void leave_resident_order(const rsg_instance* h) {
