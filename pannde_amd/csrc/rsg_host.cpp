@@ -2547,9 +2547,13 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     HIP_TRY(rsg::resident_limits(&cus, &lds));
     const size_t e = h->elt();
     if ((size_t)nc * (9 * e + 32) > (size_t)cus * lds) return RSG_OK;
-    // One tile up to 500 cells (480 cells on one compute unit: FP32 2.8 us a step against 3.5 on
-    // 7, FP64 4.4 against 4.2), then a tile per compute unit but no tile below 64 cells, where
-    // the exchange is all of a step (4800 cells: 4.4 us with tiles of 64, 5.6 with 125).
+    // One tile up to 500 cells, then a tile per compute unit but no tile below 64 cells, where the
+    // exchange is all of a step (4800 cells: 4.4 us with tiles of 64, 5.6 with 125).  One tile has no
+    // exchange and agrees with nobody, several share its work.  us a step, one / several, in calls
+    // of 5 steps and of 250: FP64 180 cells 3.8 / 5.7 and 2.7 / 3.7, 384 4.9 / 5.6 and 3.76 / 3.83,
+    // 500 5.3 / 5.8 and 4.08 / 3.99, 560 6.0 / 5.9 and 4.75 / 4.03; FP32 500 cells 3.8 / 4.9 and 2.8 /
+    // 3.3, and one tile stays ahead to about 700 (648 4.2 / 4.9 and 3.1 / 3.3, 800 4.7 / 4.9 and 3.5 /
+    // 3.3).
     const int32_t max_tiles = nc <= 500 ? 1 : std::min<int32_t>(cus, nc / 64);
     rsg::ResidentMesh m{nn, nc, h->cells.data(), h->node_cells.data(), h->cell_of.data(), h->cell_at.data(),
                         h->node_at.data(), {X[0], X[1], X[2]}, {lo[0], lo[1], lo[2]}, {hmin[0], hmin[1], hmin[2]}};
