@@ -114,7 +114,13 @@ int rsg_create(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_t p
                rsg_handle* out);
 
 /* Kernel and layout choices of a handle (they never change results: every choice is
- * bit-identical).  A zero field takes the default shown. */
+ * bit-identical).  A zero field takes the default shown.
+ *
+ * With the first six fields (workgroups, entities per thread, LDS staging) all zero, a mesh whose
+ * state fits the LDS of the whole GPU (FP64 to about 350,000 cells, FP32 to about 600,000) takes
+ * the steps of an rsg_step call of five steps or more (two on meshes of at most 500 cells) in one
+ * launch that keeps the state on the chip, at about half the time a step.  Naming any of the six,
+ * also at its default, asks for the two kernels a step that they describe. */
 typedef struct {
   int32_t block_velocity;      /* workgroup size of the velocity kernel, 64..512 step 64 (256;
                                   512 for meshes of 3 x 2^20 nodes or more when
@@ -128,7 +134,9 @@ typedef struct {
   int32_t lds_velocity;        /* 1: stage each workgroup's gathers in LDS, -1: gather from HBM (1) */
   int32_t lds_stress;          /* the same for the stress kernel (1) */
   int32_t tile[3];             /* locality brick in cells along x, y, z (8, 8, 4) */
-  int32_t c_layout;            /* 1: C in 64-cell blocks [n/64][21][64], -1: [21][n] (1) */
+  int32_t c_layout;            /* per-cell C in 64-cell blocks, 1: [n/64][w][64], -1: [w][n] (1); w is 21,
+                                  or 9 (C11, C12, C13, C22, C23, C33, C44, C55, C66) where each other
+                                  entry is the same for all cells */
   int32_t xcd_remap;           /* 1: XCD-contiguous workgroup order, -1: hardware order (1) */
   int32_t coeff_classes;       /* 1: each entity carries a 4-byte key into small tables of
                                   materials (a cell's 21 C, a node's dt/rho) and of spacings
@@ -214,13 +222,15 @@ int rsg_energy_noalloc(rsg_handle h, double* kinetic, double* strain);
  * step (the first of each n) are bracketed by HIP events on the handle's stream (1: every
  * step; events between launches slow the stream, so a stride keeps the timed run close to
  * an untimed one); 0 turns timing off.  Totals and the number of timed steps accumulate
- * until read (and reset). */
+ * until read (and reset).  While timing is on every step is made by the two kernels, also where
+ * an untimed handle takes the steps of a call in one launch (see rsg_tuning). */
 int rsg_set_timing(rsg_handle h, int32_t enabled);
 int rsg_get_kernel_times(rsg_handle h, double* velocity_ms, double* stress_ms,
                          int64_t* launches);
 
 /* Bytes of device memory the handle holds (state, coefficients, the links of each kernel:
- * connectivity, or the LDS plan of a staged kernel, and the source and trace buffers). */
+ * connectivity, or the LDS plan of a staged kernel, the source and trace buffers, from the first
+ * state transfer on the caller's numbering, and from the first one-launch call on its tiles). */
 int rsg_device_bytes(rsg_handle h, int64_t* bytes);
 
 /* Releases the handle and returns its device memory to the library's pool (one per device,

@@ -8,6 +8,12 @@ choice only affects speed.  Members of a batch may differ in their tuning (each 
 covers the members of one kernel configuration), but members of one configuration share
 launches, so tune once on a representative instance and create the batch's members with
 the result.
+
+What is tuned is the two kernels a step.  A handle without a tuning takes the steps of a call of
+five or more in one launch where its mesh fits the GPU's LDS (FP64 to about 350,000 cells, FP32 to
+about 600,000), at about half the time a step; one with the result of ``tune`` does not.  So tune
+larger meshes, batches' members and handles that are stepped once a call, and leave the others
+without.
 """
 from __future__ import annotations
 

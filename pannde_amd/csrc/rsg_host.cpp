@@ -1624,10 +1624,10 @@ bool steps_resident(const rsg_instance* h, int kb) {
 // Bytes of the exchange buffers, as many as a multiple of 16 that the records follow.
 size_t resident_exchange_bytes(const rsg_instance* h) { return ((size_t)24 * h->res.nexp * h->elt() + 15) / 16 * 16; }
 
-// Puts the plan on the device with the first resident launch, and the classes of the source terms
-// with the first after a table build, and takes the status words: a handle that is never stepped resident (in a batch, step by
-// step) holds no device memory for it.  False when there is no memory: for now the per-step kernels
-// do without.
+// Takes the status words and puts the plan on the device with the first resident launch, and the
+// classes of the source terms with the first after a table build: a handle that is never stepped
+// resident (in a batch, step by step) holds no device memory for it.  False when there is no memory:
+// for now the per-step kernels do without.
 bool resident_on_device(rsg_instance* h) {
   rsg::ResidentPlan& p = h->res;
   bool ok = h->res_status || (h->res_status = take_status(h->device));
@@ -1785,7 +1785,8 @@ int run_steps(rsg_instance* h, int kb, rsg::VelocityArgs<T>& va, rsg::StressArgs
 // amplitudes goes on its stream.
 int settle_resident(rsg_instance* h) {
   if (h->res_pending == 0) return RSG_OK;
-  auto decision = [&]() { return (uint32_t)__atomic_load_n(h->res_status + rsg::kResidentDecision, __ATOMIC_ACQUIRE); };
+  const int32_t* const word = h->res_status + rsg::kResidentDecision;
+  auto decision = [word]() { return (uint32_t)__atomic_load_n(word, __ATOMIC_ACQUIRE); };
   uint32_t d = decision();
   for (uint32_t spin = 1; d >> 1 != (h->res_seq & 0x7FFFFFFFu); spin++, d = decision()) {
     if (spin % 64) continue;
@@ -2538,6 +2539,7 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
   // step against the two per-step kernels (us, aluminium blocks): 480 cells 8.9 -> 4.1 in FP64 and
   // 8.3 -> 2.7 in FP32, 32,000 cells 9.7 -> 4.4 and 8.9 -> 3.5, 131,000 cells 12.8 -> 6.4 and
   // 10.0 -> 4.5, 259,000 cells 18.2 -> 11.0 and 12.0 -> 6.9, 531,000 cells in FP32 20.4 -> 11.5.
+  // (Also a named default is a choice: tests and tuners compare the two forms that way.)
   const bool chosen = tuning && (tuning->block_velocity || tuning->block_stress || tuning->per_thread_velocity ||
                                  tuning->per_thread_stress || tuning->lds_velocity || tuning->lds_stress);
   auto resident_part = [&]() -> int {
@@ -2615,9 +2617,9 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     const int64_t e = (int64_t)h->elt(), cache = kCacheBytes - kCacheBytes / 10;
     const int64_t state = e * (3 * (int64_t)nn + 6 * (int64_t)nc);
     h->once_v = (int64_t)nn * ((h->v_lkey || h->v_lconn ? 16 : 32) + (h->nkey ? 4 : 0)) + h->v_list_bytes +
-                           (h->n_nmat < 0 ? 4 * e * nn : 0);
+                (h->n_nmat < 0 ? 4 * e * nn : 0);
     h->once_s = (int64_t)nc * ((h->s_lkey || h->s_lconn ? 16 : 32) + (h->ckey ? 4 : 0)) + h->s_list_bytes +
-                           (h->n_cmat < 0 ? (h->crow ? 3 + rsg::kAxialEntries : 24) * e * nc : 0);
+                (h->n_cmat < 0 ? (h->crow ? 3 + rsg::kAxialEntries : 24) * e * nc : 0);
     h->stream_v = state + h->once_v > cache;
     h->stream_s = state + h->once_v + h->once_s > cache;
   }
@@ -3293,8 +3295,8 @@ int batch_block(rsg_batch_s* b, int l, int32_t* unfinished) {
   // configuration, each group within the state budget (an instance larger than the budget
   // forms a group of its own)
   auto config = [](const rsg_instance* h) -> std::array<int32_t, 8> {
-    return {h->v_lkey ? 3 : h->nkey ? 1 : 0, h->s_lkey ? 3 : h->ckey ? 1 : h->crow ? 2 : 0, h->block_v, h->block_s, h->cpt_v,
-            h->cpt_s, (h->v_lconn || h->v_lkey) ? 1 : 0, (h->s_lconn || h->s_lkey) ? 1 : 0};
+    return {h->v_lkey ? 3 : h->nkey ? 1 : 0, h->s_lkey ? 3 : h->ckey ? 1 : h->crow ? 2 : 0, h->block_v, h->block_s,
+            h->cpt_v, h->cpt_s, (h->v_lconn || h->v_lkey) ? 1 : 0, (h->s_lconn || h->s_lkey) ? 1 : 0};
   };
   std::vector<std::array<int32_t, 8>> configs;  // distinct configurations, first seen first
   for (size_t i = 0; i < b->slots.size(); i++)

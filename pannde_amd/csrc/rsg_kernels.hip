@@ -119,7 +119,8 @@ __device__ __forceinline__ void load8_nodes(const T* __restrict__ f, const int (
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 // Coefficient form of a kernel instance: KM = 0 per-entity arrays, 2 per-cell arrays of the axial
-// entries (stress kernels), 1 class-table keys, 3 keys packed with the LDS links (a batch launches each form for its own members).
+// entries (stress kernels), 1 class-table keys, 3 keys packed with the LDS links (a batch launches
+// each form for its own members).
 template <int KM, typename A>
 __device__ __forceinline__ constexpr bool packed(const A&) {
   return KM == 3;
@@ -716,7 +717,8 @@ constexpr bool cacheable(bool lds, int u, int cpt) { return lds && u > 0 && cpt 
 template <typename T>
 hipError_t launch_velocity(const VelocityArgs<T>& a, int block, hipStream_t s) {
   const bool lds = a.lconn != nullptr || a.lkey != nullptr;
-  return with_variant<false>(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : 0, [&](auto L, auto U, auto C, auto K) {
+  const int km = a.lkey ? 3 : a.key ? 1 : 0;
+  return with_variant<false>(lds, a.max_u, block, a.cpt, km, [&](auto L, auto U, auto C, auto K) {
     constexpr bool l = decltype(L)::value;
     constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
     const size_t bytes = lds ? velocity_lds_bytes(a.max_u, sizeof(T)) : 0;
@@ -729,7 +731,8 @@ hipError_t launch_velocity(const VelocityArgs<T>& a, int block, hipStream_t s) {
 template <typename T>
 hipError_t launch_stress(const StressArgs<T>& a, int block, hipStream_t s) {
   const bool lds = a.lconn != nullptr || a.lkey != nullptr;
-  return with_variant<true>(lds, a.max_u, block, a.cpt, a.lkey ? 3 : a.key ? 1 : a.crow ? 2 : 0, [&](auto L, auto U, auto C, auto K) {
+  const int km = a.lkey ? 3 : a.key ? 1 : a.crow ? 2 : 0;
+  return with_variant<true>(lds, a.max_u, block, a.cpt, km, [&](auto L, auto U, auto C, auto K) {
     constexpr bool l = decltype(L)::value;
     constexpr int u = decltype(U)::value, c = decltype(C)::value, m = decltype(K)::value;
     const size_t bytes = lds ? (size_t)3 * a.max_u * sizeof(T) : 0;

@@ -50,7 +50,8 @@ def same(got, case):
 
 def run(lib, script, **env):
     r = subprocess.run([sys.executable, "-c", PRELUDE + script + '\nprint("ok")\n', ROOT], stdout=subprocess.PIPE,
-                       stderr=subprocess.STDOUT, text=True, timeout=300, env=dict(os.environ, PANNDE_RSG_LIB=lib, **env))
+                       stderr=subprocess.STDOUT, text=True, timeout=300,
+                       env=dict(os.environ, PANNDE_RSG_LIB=lib, **env))
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout[-4000:]
 
 
