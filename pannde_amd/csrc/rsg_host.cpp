@@ -29,6 +29,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <ctime>
+#include <deque>
 #include <exception>
 #include <iterator>
 #include <memory>
@@ -251,14 +252,16 @@ PinnedPool& pinned_pool() {
 }
 
 // Up to `want` chunks of the device, which is current; at least one, unless there is no pinned
-// memory at all.
-std::vector<PinnedChunk> take_chunks(int device, int want) {
+// memory at all.  `ahead`: the transfer will wait behind steps queued before it, so it takes chunks
+// only while half the pool is left to transfers that will not, else none.
+std::vector<PinnedChunk> take_chunks(int device, int want, bool ahead) {
   PinnedPool& o = pinned_pool();
   std::vector<PinnedChunk> got;
   got.reserve((size_t)want);
   std::unique_lock<std::mutex> lock(o.mu);
   PinnedPool::Device& d = o.devices[device];
   d.idle.reserve(kPinnedChunks);  // giving back takes no memory
+  if (ahead && (int)d.idle.size() + kPinnedChunks - d.made < want + kPinnedChunks / 2) return got;
   while ((int)got.size() < want) {
     if (!d.idle.empty()) {
       got.push_back(d.idle.back());
@@ -492,11 +495,15 @@ struct rsg_instance {
   std::chrono::steady_clock::time_point res_not_before;  // after a refused launch
   int32_t* res_status = nullptr;  // pinned, from the first resident launch on
   int32_t res_lost = 0;  // kLost... of a launch whose tiles lost each other, until written again
-  // the last launch of several tiles, until its decision is known: its steps (0: it is), first
-  // step's amplitudes and trace row
-  int32_t res_pending = 0;
-  const double* res_amp = nullptr;
-  int64_t res_row = 0;
+  // the last launches of several tiles (up to number res_seq), until their decisions are known: their
+  // steps, the first step's amplitudes, the buffer these are in, and the first trace row
+  struct Launch {
+    int32_t steps;
+    int32_t buffer;
+    const double* amp;
+    int64_t row;
+  };
+  std::deque<Launch> res_pending;
 
   int32_t* order = nullptr;  // node_at, then cell_at, on the device: from the first state transfer on
 
@@ -1512,12 +1519,14 @@ int check_resident(rsg_instance* h, int part) {
   return RSG_OK;
 }
 
+int finish_steps(rsg_instance* h);
+
 int flush_traces(rsg_instance* h) {
   const size_t row = h->sensors.size() * 3;
   if (h->trace_dev_steps == 0 || row == 0) return RSG_OK;
+  if (int rc = finish_steps(h)) return rc;
   const size_t old = h->trace_host.size();
   h->trace_host.resize(old + (size_t)h->trace_dev_steps * row);
-  HIP_TRY(hipStreamSynchronize(h->stream));
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
   HIP_TRY(copy_on(h->trace_host.data() + old, h->trace.p, (size_t)h->trace_dev_steps * row * sizeof(double),
                   hipMemcpyDeviceToHost, h->stream));
@@ -1661,7 +1670,7 @@ bool resident_on_device(rsg_instance* h) {
 // kb steps in one launch of the resident kernel; *done says whether it was launched.
 template <typename T>
 int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const rsg::StressArgs<T>& sa,
-                 const double* force, size_t row, bool* done) {
+                 const double* force, size_t row, bool chained, bool* done) {
   *done = false;
   DeviceScope scope(h->device);
   HIP_TRY(scope.status);
@@ -1679,6 +1688,7 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   a.xbuf = (unsigned long long*)(mem + p.bytes);
   a.ctrl = (uint32_t*)(mem + p.ctrl);
   a.seq = h->res_seq + 1;
+  a.chained = chained;
   a.status = h->res_status;
   a.nsteps = kb;
   a.ntiles = p.ntiles;
@@ -1779,43 +1789,76 @@ int run_steps(rsg_instance* h, int kb, rsg::VelocityArgs<T>& va, rsg::StressArgs
   return RSG_OK;
 }
 
-// Once this returns, the steps of the handle's last resident launch are made or queued: it waits for
-// the launch's decision, which comes as the launch begins, and queues the per-step kernels when that
-// was against the steps.  Called before anything else that uses the handle's state, tables or
-// amplitudes goes on its stream.
-int settle_resident(rsg_instance* h) {
-  if (h->res_pending == 0) return RSG_OK;
-  const int32_t* const word = h->res_status + rsg::kResidentDecision;
-  auto decision = [word]() { return (uint32_t)__atomic_load_n(word, __ATOMIC_ACQUIRE); };
-  uint32_t d = decision();
-  for (uint32_t spin = 1; d >> 1 != (h->res_seq & 0x7FFFFFFFu); spin++, d = decision()) {
+// Takes note of the decisions of the handle's resident launches: of those that are known, and of
+// what it waits for, every launch (`all`) or those whose amplitudes are in `buffer`.  When one was
+// refused so were those queued behind it, and the per-step kernels make the steps of all of them
+// (*again, where given: what was queued after them has run on the wrong state).  A launch decides as
+// it begins, so after a wait for the stream this does not wait.
+int settle_resident(rsg_instance* h, bool all = true, int buffer = -1, bool* again = nullptr) {
+  if (again) *again = false;
+  std::deque<rsg_instance::Launch>& q = h->res_pending;
+  if (q.empty()) return RSG_OK;
+  const uint64_t* const word = reinterpret_cast<const uint64_t*>(h->res_status + rsg::kResidentDecision);
+  bool ended = false;  // all launches have, so they have decided
+  for (uint32_t spin = 1; !q.empty(); spin++) {
+    const uint64_t w = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    const uint32_t d = (uint32_t)w, first_refused = (uint32_t)(w >> 32);
+    const uint32_t head = h->res_seq + 1 - (uint32_t)q.size();  // the oldest's number
+    const int64_t size = (int64_t)q.size();
+    const int64_t last = (int32_t)(((d >> 1) - head) << 1) >> 1;  // the last one decided, counted from there
+    const int64_t known = ended ? size : std::max<int64_t>(0, std::min(size, last + 1));
+    const bool refused = last >= 0 && !(d & 1);
+    if (!refused) {
+      q.erase(q.begin(), q.begin() + known);
+    } else if (known < size) {
+      all = true;  // the others refuse as soon as they begin
+    } else {
+      // the GPU is shared with work that keeps the tiles apart: not again soon
+      h->res_not_before = std::chrono::steady_clock::now() + kResidentRetry;
+      q.erase(q.begin(), q.begin() + std::max<int64_t>(0, std::min<int64_t>(size, (int32_t)(first_refused - head))));
+      if (again) *again = true;
+      auto steps = [&](auto zero, const rsg_instance::Launch& l) {
+        using T = decltype(zero);
+        rsg::VelocityArgs<T> va;
+        rsg::StressArgs<T> sa;
+        fill_args<T>(h, va, sa);
+        return run_steps<T>(h, l.steps, va, sa, l.amp, l.row, 0);
+      };
+      while (!q.empty()) {
+        const rsg_instance::Launch l = q.front();
+        q.pop_front();
+        const int rc = h->precision == RSG_FP64 ? steps(0.0, l) : steps(0.0f, l);
+        if (rc) return rc;
+      }
+    }
+    if (q.empty()) break;
+    if (!all && std::none_of(q.begin(), q.end(), [&](auto& l) { return l.buffer == buffer; })) return RSG_OK;
     if (spin % 64) continue;
     const hipError_t e = h->res_recorded ? hipEventQuery(h->res_event) : hipStreamSynchronize(h->stream);
-    if (e == hipSuccess) break;  // (a launch that has ended has decided)
-    if (e != hipErrorNotReady) return fail(RSG_ERR_DEVICE, "resident launch: %s", hipGetErrorString(e));
-    std::this_thread::yield();
+    if (e == hipSuccess)
+      ended = true;
+    else if (e != hipErrorNotReady)
+      return fail(RSG_ERR_DEVICE, "resident launch: %s", hipGetErrorString(e));
+    else
+      std::this_thread::yield();
   }
-  const int kb = h->res_pending;
-  h->res_pending = 0;
-  {  // what was copied before the launch has arrived
-    std::lock_guard<std::mutex> lock(h->hold_mu);
-    h->held.clear();
-  }
-  if (decision() != 2 * h->res_seq) return RSG_OK;
-  // the GPU is shared with work that keeps the tiles apart: not again soon
-  h->res_not_before = std::chrono::steady_clock::now() + kResidentRetry;
-  auto steps = [&](auto zero) {
-    using T = decltype(zero);
-    rsg::VelocityArgs<T> va;
-    rsg::StressArgs<T> sa;
-    fill_args<T>(h, va, sa);
-    return run_steps<T>(h, kb, va, sa, h->res_amp, h->res_row, 0);
-  };
-  return h->precision == RSG_FP64 ? steps(0.0) : steps(0.0f);
+  std::lock_guard<std::mutex> lock(h->hold_mu);
+  h->held.clear();  // what was copied before the launches has arrived
+  return RSG_OK;
 }
 
+// Waits for the handle's queued steps, those of refused launches included.
+int finish_steps(rsg_instance* h) {
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  bool again = false;
+  if (int rc = settle_resident(h, true, -1, &again)) return rc;
+  if (again) HIP_TRY(hipStreamSynchronize(h->stream));
+  return RSG_OK;
+}
+
+// kb steps with the amplitudes at amp_dev, which are in amp[buffer] (2: in neither, no amplitudes).
 template <typename T>
-int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* force_dev) {
+int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* force_dev, int buffer) {
   rsg::VelocityArgs<T> va;
   rsg::StressArgs<T> sa;
   fill_args<T>(h, va, sa);
@@ -1824,14 +1867,16 @@ int run_block(rsg_instance* h, int kb, const double* amp_dev, const double* forc
   int rc;
   if (steps_resident(h, kb)) {
     va.trace = h->trace.p ? h->trace.p + (size_t)h->trace_dev_steps * row : nullptr;
-    if ((rc = run_resident<T>(h, kb, va, sa, force_dev, row, &done))) return rc;
-    if (done && h->res.ntiles > 1) {
-      h->res_pending = kb;
-      h->res_amp = amp_dev;
-      h->res_row = h->trace_dev_steps;
-    }
+    const bool chained = !h->res_pending.empty();
+    h->res_pending.push_back({kb, buffer, amp_dev, h->trace_dev_steps});
+    rc = run_resident<T>(h, kb, va, sa, force_dev, row, chained, &done);
+    if (!done || h->res.ntiles == 1) h->res_pending.pop_back();
+    if (rc) return rc;
   }
-  if (!done && (rc = run_steps<T>(h, kb, va, sa, amp_dev, h->trace_dev_steps, h->timing))) return rc;
+  if (!done) {
+    if ((rc = settle_resident(h))) return rc;
+    if ((rc = run_steps<T>(h, kb, va, sa, amp_dev, h->trace_dev_steps, h->timing))) return rc;
+  }
   h->trace_dev_steps += row ? kb : 0;
   return RSG_OK;
 }
@@ -1855,29 +1900,32 @@ void fill_energy_args(rsg_instance* h, rsg::EnergyArgs<T>& a, double* work) {
 
 int energy_on_stream(rsg_instance* h, double* work, double* kinetic, double* strain) {
   Range range_("rsg_energy");
-  if (int rc = settle_resident(h)) return rc;
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
+  int rc;
   if (h->tables_dirty) {
-    int rc = build_tables(h);  // the special-cell keys the kernel resolves
-    if (rc) return rc;
+    if ((rc = settle_resident(h))) return rc;
+    if ((rc = build_tables(h))) return rc;  // the special-cell keys the kernel resolves
   }
   const int nb = rsg::kEnergyMaxBlocks;
   double* out = work + 2 * nb;
-  hipError_t e;
-  if (h->precision == RSG_FP64) {
-    rsg::EnergyArgs<double> a;
-    fill_energy_args<double>(h, a, work);
-    e = rsg::launch_energy_f64(a, nb, out, h->stream);
-  } else {
-    rsg::EnergyArgs<float> a;
-    fill_energy_args<float>(h, a, work);
-    e = rsg::launch_energy_f32(a, nb, out, h->stream);
-  }
-  if (e != hipSuccess) return fail(RSG_ERR_DEVICE, "energy launch: %s", hipGetErrorString(e));
   double tot[2] = {0.0, 0.0};
-  HIP_TRY(hipMemcpyAsync(tot, out, sizeof(tot), hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  if (int rc = check_resident(h, kLostV | kLostS)) return rc;
+  for (bool again = true; again;) {  // a second time when refused steps were made only now
+    hipError_t e;
+    if (h->precision == RSG_FP64) {
+      rsg::EnergyArgs<double> a;
+      fill_energy_args<double>(h, a, work);
+      e = rsg::launch_energy_f64(a, nb, out, h->stream);
+    } else {
+      rsg::EnergyArgs<float> a;
+      fill_energy_args<float>(h, a, work);
+      e = rsg::launch_energy_f32(a, nb, out, h->stream);
+    }
+    if (e != hipSuccess) return fail(RSG_ERR_DEVICE, "energy launch: %s", hipGetErrorString(e));
+    HIP_TRY(hipMemcpyAsync(tot, out, sizeof(tot), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    if ((rc = settle_resident(h, true, -1, &again))) return rc;
+  }
+  if ((rc = check_resident(h, kLostV | kLostS))) return rc;
   if (kinetic) *kinetic = tot[0];
   if (strain) *strain = tot[1];
   return RSG_OK;
@@ -1887,6 +1935,7 @@ int energy_on_stream(rsg_instance* h, double* work, double* kinetic, double* str
 // memory for the maps or no pinned memory for the chunks (a state can always be read), and in builds
 // of the host code without the kernels of rsg_state.hip.
 int transfer_state_on_host(rsg_instance* h, double* V, double* S, bool write) {
+  HIP_TRY(hipStreamSynchronize(h->stream));
   const size_t e = h->elt();
   std::vector<char> buf((size_t)std::max(h->nn, h->nc) * e);
   auto move = [&](void* dev, int32_t n, const std::vector<int32_t>& of, double* host) -> int {
@@ -1925,7 +1974,11 @@ int transfer_chunks(rsg_instance* h, double* V, double* S, bool write, bool* don
   const int64_t nv = (int64_t)3 * h->nn, g0 = V ? 0 : nv, g1 = S ? nv + (int64_t)6 * h->nc : nv;
   const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
   const int most = (int)std::max<int64_t>(1, std::min<int64_t>({(g1 - g0) >> 17, setup_threads(), hw, kPinnedChunks}));
-  const std::vector<PinnedChunk> pinned = take_chunks(h->device, most);
+  std::vector<PinnedChunk> pinned = take_chunks(h->device, most, true);
+  if (pinned.empty()) {
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    pinned = take_chunks(h->device, most, false);
+  }
   const int threads = (int)pinned.size();
   *done = threads > 0;
   if (threads == 0) return RSG_OK;
@@ -1993,8 +2046,10 @@ int transfer_chunks(rsg_instance* h, double* V, double* S, bool write, bool* don
 }
 
 int transfer_state(rsg_instance* h, double* V, double* S, bool write) {
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  if (!V && !S) return RSG_OK;
+  if (!V && !S) {
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    return RSG_OK;
+  }
   DeviceScope scope(h->device);
   HIP_TRY(scope.status);
   try {
@@ -2710,7 +2765,7 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   if (h->in_batch) return fail(RSG_ERR_STATE, "the handle is stepped by a batch; remove it first");
   if (nsteps < 0) return fail(RSG_ERR_ARG, "nsteps < 0");
-  int rc = settle_resident(h);
+  int rc = settle_resident(h, h->tables_dirty);
   if (rc) return rc;
   if (h->tables_dirty && (rc = build_tables(h))) return rc;
   const size_t nch = h->channels.size();
@@ -2722,11 +2777,12 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
   // the resident kernel's summed source terms follow the amplitudes of an upload
   const size_t nf = h->res_nclasses >= 0 ? h->res_force.size() : 0;
   for (int32_t done = 0; done < nsteps;) {
-    if ((rc = settle_resident(h))) return rc;
+    if ((rc = settle_resident(h, false))) return rc;
     int kb = std::min(kBlockSteps, nsteps - done);
     const bool none = nch == 0;  // a buffer that no term reads, and zero sums
     const double* amp = none ? h->amp[0].p : nullptr;
     const double* force = h->amp[0].p;
+    int buffer = none ? 2 : h->win_buf;  // of the amplitudes
     if (!none && !amplitudes && h->win_first >= 0 && h->steps >= h->win_first &&
         h->steps < h->win_first + h->win_len) {
       // the next steps' amplitudes are on the device already (the signal tables are the
@@ -2742,6 +2798,7 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
       // a table-driven upload covers a whole block ahead; caller amplitudes cover this call
       const int up = amplitudes ? kb : kBlockSteps;
       if (h->stage_busy[b]) HIP_TRY(hipEventSynchronize(h->stage_ev[b]));
+      if ((rc = settle_resident(h, false, b))) return rc;
       if (!h->stage[b]) {
         HIP_TRY(hipHostMalloc((void**)&h->stage[b], (nch + nf) * kBlockSteps * sizeof(double), hipHostMallocDefault));
         h->stage_len[b] = (nch + nf) * kBlockSteps;
@@ -2775,6 +2832,7 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
       h->cur ^= 1;
       amp = h->amp[b].p;
       force = amp + (size_t)up * nch;
+      buffer = b;
       if (amplitudes) {
         h->win_first = -1;
       } else {
@@ -2783,7 +2841,8 @@ int rsg_step(rsg_handle h, int32_t nsteps, const double* amplitudes, double* tim
         h->win_buf = b;
       }
     }
-    rc = h->precision == RSG_FP64 ? run_block<double>(h, kb, amp, force) : run_block<float>(h, kb, amp, force);
+    rc = h->precision == RSG_FP64 ? run_block<double>(h, kb, amp, force, buffer)
+                                     : run_block<float>(h, kb, amp, force, buffer);
     if (rc) return rc;
     for (int k = 0; k < kb; k++) h->time += h->dt;  // HostRSGTDUT::solve: time += dt
     h->steps += kb;
@@ -2797,8 +2856,11 @@ int rsg_get_state(rsg_handle h, double* V, double* S) {
   Range range_("rsg_get_state");
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
-  int rc = settle_resident(h);
-  if (!rc) rc = transfer_state(h, V, S, false);
+  int rc = RSG_OK;
+  for (bool again = true; again && !rc;) {  // a second time when refused steps were made only now
+    rc = transfer_state(h, V, S, false);
+    if (!rc) rc = settle_resident(h, true, -1, &again);
+  }
   return rc ? rc : check_resident(h, kLostV | kLostS);
 }
 
@@ -2815,8 +2877,7 @@ int rsg_set_state(rsg_handle h, const double* V, const double* S) {
 
 int rsg_get_traces(rsg_handle h, int64_t first, int64_t n, double* out) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
-  int rc = settle_resident(h);
-  if (!rc) rc = flush_traces(h);
+  int rc = flush_traces(h);
   if (!rc) rc = check_resident(h, kLostTraces);
   if (rc) return rc;
   const size_t row = h->sensors.size() * 3;
@@ -2831,8 +2892,7 @@ int rsg_get_traces(rsg_handle h, int64_t first, int64_t n, double* out) {
 
 int rsg_synchronize(rsg_handle h) {
   if (!h) return fail(RSG_ERR_ARG, "handle is null");
-  if (int rc = settle_resident(h)) return rc;
-  HIP_TRY(hipStreamSynchronize(h->stream));
+  if (int rc = finish_steps(h)) return rc;
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
   return check_resident(h, kLostV | kLostS);
 }

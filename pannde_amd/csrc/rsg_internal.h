@@ -225,9 +225,9 @@ constexpr int kResidentForces = 256;  // largest row
 constexpr uint8_t kResidentSensor = 0x80;  // node mark: a sensor this tile records
 
 // Status words: the last launch's decision (several tiles), 2 seq + 1 when its steps are made and
-// 2 seq when its tiles did not get onto the GPU together and nothing is written; 1 when a wait
-// between tiles ran out (the state is lost).
-constexpr int kResidentDecision = 0, kResidentLost = 1, kResidentStatus = 2;
+// 2 seq when nothing is written, with the number of the first launch of those refused last (one
+// 8-byte word); 1 when a wait between tiles ran out (the state is lost).
+constexpr int kResidentDecision = 0, kResidentRefused = 1, kResidentLost = 2, kResidentStatus = 3;
 
 template <typename T>
 struct ResidentArgs {
@@ -240,9 +240,11 @@ struct ResidentArgs {
   const int32_t* halo;   // exchange slot of each halo cell
   const int32_t* hcell;  // internal id of each halo cell
   unsigned long long* xbuf;  // [4][6 * sizeof(T) / 8][nexp]: exported stresses of four steps in turn
-  uint32_t* ctrl;        // [2]: tiles started, over all launches; the last decision (several tiles)
+  uint32_t* ctrl;        // [3] (several tiles): tiles started, over all launches; the last decision; the
+                         // first launch of those refused last
   uint32_t seq;          // number of the launch, from 1
-  int32_t* status;       // [kResidentStatus], pinned
+  int32_t chained;       // 1: refuse the launch if the one before it was
+  int32_t* status;       // [kResidentStatus], pinned, 8-byte aligned
   int32_t nsteps;        // >= 2
   int32_t ntiles;
   int32_t nexp;

@@ -26,8 +26,8 @@ void NAME(__wrap_, START_THREAD)(std::thread* self, void* state, void (*depend)(
   NAME(__real_, START_THREAD)(self, state, depend);
 }
 
-// Resident launches that decide against their steps (and say so when the host has asked the event
-// that often), launches so far, and what the per-step kernels were launched with: the first
+// Resident launches that decide against their steps, when the decisions from now on become known (the
+// host has asked the event that often, or waited for the stream), launches so far, and what the per-step kernels were launched with: the first
 // channel's amplitude and the trace row's address.
 int fault_refuse = 0, fault_late = 0;
 int fault_resident = 0, fault_velocity = 0, fault_stress = 0;
@@ -54,8 +54,14 @@ int device_of(const void* p) {
   return devices.count(p) ? devices[p] : 0;
 }
 
-int32_t* late_word = nullptr;
-int32_t late_value = 0;
+// the status word of the last decision, and what it will hold: late, or at once
+uint64_t* late_word = nullptr;
+uint64_t late_value = 0;
+void decide(int32_t* status, uint32_t decision, uint32_t first_refused) {
+  late_word = reinterpret_cast<uint64_t*>(status + rsg::kResidentDecision);
+  late_value = (uint64_t)first_refused << 32 | decision;
+  if (fault_late == 0) *late_word = late_value;
+}
 
 template <typename A, typename F>
 hipError_t resident(const A& a, F&& real) {
@@ -63,14 +69,19 @@ hipError_t resident(const A& a, F&& real) {
   fault_resident++;
   if (fault_lost > 0 && fault_lost--) a.status[rsg::kResidentLost] = 1;
   if (a.ntiles == 1) return real();
-  late_word = a.status + rsg::kResidentDecision;
-  if (fault_refuse == 0) {
-    *late_word = (int32_t)(2 * a.seq + 1);
+  uint32_t* const decision = a.ctrl + 1;  // as the kernel keeps it
+  const bool barred = a.chained && *decision == 2 * (a.seq - 1);
+  if (!barred && fault_refuse == 0) {
+    *decision = 2 * a.seq + 1;
+    decide(a.status, *decision, 0);
     return real();
   }
-  fault_refuse--;
-  late_value = (int32_t)(2 * a.seq);
-  if (fault_late == 0) *late_word = late_value;
+  *decision = 2 * a.seq;
+  if (!barred) {
+    fault_refuse--;
+    a.ctrl[2] = a.seq;
+  }
+  decide(a.status, *decision, a.ctrl[2]);
   return hipSuccess;
 }
 template <typename A>
@@ -114,6 +125,10 @@ int fault_waits = 0;
 hipError_t __real_hipStreamSynchronize(hipStream_t s);
 hipError_t __wrap_hipStreamSynchronize(hipStream_t s) {
   __atomic_fetch_add(&fault_waits, 1, __ATOMIC_RELAXED);
+  if (fault_late > 0) {
+    fault_late = 0;
+    *late_word = late_value;
+  }
   return __real_hipStreamSynchronize(s);
 }
 

@@ -69,8 +69,8 @@ for n in (0, 1, 2, 3, 5):
 
 
 def test_refused_launch_is_made_by_the_per_step_kernels(lib):
-    """Whatever comes after a launch that decided against its steps first queues those steps, each
-    with its own amplitudes and trace row; no launch is put behind an undecided one."""
+    """Whatever reads or follows a launch that decided against its steps gets those steps, and those of
+    the launches that were queued behind it, each with its own amplitudes and trace row."""
     run(lib, r'''
 case = cases.al_block(seed=1, nx=20, ny=19, nz=18, nsteps=400, n_sensors=4)
 sig = case.force[0]
@@ -103,9 +103,14 @@ for name, read in reads.items():
         reset(1, late)
         s.solve(9)  # not made
         assert knob("fault_resident").value == 1 and knob("fault_velocity").value == 0
+        more = late and name != "zero"
+        if more:  # refused behind it
+            s.solve(6)
+            assert knob("fault_resident").value == 2 and knob("fault_velocity").value == 0
         read(s)
-        assert knob("fault_late").value == 0
-        check(9 + (name == "step"), 7, 0)
+        if name != "zero":  # (which may leave the decision for later)
+            assert knob("fault_late").value == 0
+            check(9 + (6 if more else 0) + (name == "step"), 7, 0)
         s.close()
 # a batch takes the handle with its steps queued
 s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
@@ -123,6 +128,30 @@ s.solve(400)
 assert knob("fault_resident").value == 1
 check(400, 0, 0)
 assert s.traces().shape[0] == 400
+s.close()
+# decisions that come late: blocks are queued behind the refused one, as long as its amplitudes are kept
+case = cases.al_block(seed=1, nx=20, ny=19, nz=18, nsteps=1100, n_sensors=4)
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+reset(0, 0)
+s.solve(20)
+reset(1, 5)
+s.solve(1000)
+# (236 steps are left of the first amplitudes; the third upload overwrites those)
+assert knob("fault_resident").value == 2
+check(1000, 20, 0)
+assert s.traces().shape[0] == 1020
+s.close()
+# many launches in one block of amplitudes: the first ones made, the rest not
+s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
+reset(0, 0)
+for _ in range(10):
+    s.solve(5)
+reset(1, 9)
+for _ in range(30):
+    s.solve(5)
+assert knob("fault_resident").value == 30 and knob("fault_velocity").value == 0
+s.energy()
+check(150, 50, 0)
 s.close()
 ''')
 
