@@ -474,14 +474,15 @@ struct rsg_instance {
   double* node_m = nullptr;    // node masses rho_n*dxn*dyn*dzn (energy)
   double* cell_vol = nullptr;  // cell volumes dxc*dyc*dzc (energy)
 
-  // resident stepping: the plan (ntiles 0: none, or none any more), its arrays on the host until the
-  // first resident launch puts them on the device, in front of the exchange buffers and of the
-  // kernel's records where these do not fit LDS
+  // resident stepping: the plan (ntiles 0: none, or none any more), on the device with the set-up's
+  // uploads, and from the first resident launch on the exchange buffers, followed by the kernel's
+  // records where these do not fit LDS
   rsg::ResidentPlan res;
   int32_t res_threads = 0;
   bool res_records = false;  // in LDS
   size_t res_lds_room = 0;   // LDS a tile leaves free
   void* res_mem = nullptr;
+  void* res_exchange = nullptr;
   // source terms as the resident kernel takes them: one list of channels per class and component
   // (res_force: the node classes, 3 lists each, then the cell classes, 6 each); -1 node classes:
   // more classes than the kernel holds
@@ -1630,27 +1631,34 @@ bool steps_resident(const rsg_instance* h, int kb) {
           std::chrono::steady_clock::now() >= h->res_not_before);
 }
 
-// Bytes of the exchange buffers, as many as a multiple of 16 that the records follow.
-size_t resident_exchange_bytes(const rsg_instance* h) { return ((size_t)24 * h->res.nexp * h->elt() + 15) / 16 * 16; }
+// Bytes of the exchange buffers, up to where the records follow.
+size_t resident_exchange_bytes(const rsg_instance* h) {
+  return ((size_t)24 * h->res.nexp * h->elt() + 255) / 256 * 256;
+}
 
-// Takes the status words and puts the plan on the device with the first resident launch, and the
-// classes of the source terms with the first after a table build: a handle that is never stepped
-// resident (in a batch, step by step) holds no device memory for it.  False when there is no memory:
-// for now the per-step kernels do without.
+// Queues the copy of the plan.  False when there is no memory for it.
+bool upload_plan(rsg_instance* h) {
+  rsg::ResidentPlan& p = h->res;
+  if (h->dalloc(&h->res_mem, p.bytes) != RSG_OK) {
+    forget_error();
+    return false;
+  }
+  const hipError_t e = hipMemcpyAsync(h->res_mem, p.block.get(), p.bytes, hipMemcpyHostToDevice, h->stream);
+  h->hold(std::shared_ptr<const void>(p.block.release(), [](const void* b) { delete[] (const char*)b; }));
+  if (e != hipSuccess) p.ntiles = 0;
+  return e == hipSuccess;
+}
+
+// What resident launches need beyond the plan comes with the first one, and the classes of the source
+// terms with the first after a table build: a handle that is never stepped resident (in a batch, step
+// by step) does without.  False when there is no memory: for now the per-step kernels take over.
 bool resident_on_device(rsg_instance* h) {
   rsg::ResidentPlan& p = h->res;
   bool ok = h->res_status || (h->res_status = take_status(h->device));
-  if (ok && !h->res_mem) {
+  if (ok && !h->res_mem) ok = upload_plan(h);
+  if (ok && !h->res_exchange) {
     const size_t work = h->res_records ? 0 : (size_t)16 * p.ntiles * (p.max_node + p.max_cell);
-    ok = h->dalloc(&h->res_mem, p.bytes + resident_exchange_bytes(h) + work) == RSG_OK;
-    if (ok) {
-      const hipError_t e = hipMemcpyAsync(h->res_mem, p.block.get(), p.bytes, hipMemcpyHostToDevice, h->stream);
-      h->hold(std::shared_ptr<const void>(p.block.release(), [](const void* b) { delete[] (const char*)b; }));
-      if (e != hipSuccess) {
-        p.ntiles = 0;
-        return false;
-      }
-    }
+    ok = h->dalloc(&h->res_exchange, resident_exchange_bytes(h) + work) == RSG_OK;
   }
   if (ok && p.ntiles > 1 && !h->res_event) {
     ok = hipEventCreateWithFlags(&h->res_event, hipEventDisableTiming) == hipSuccess;
@@ -1685,7 +1693,7 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   a.nrec = (const uint32_t*)(mem + p.nrec);
   a.halo = (const int32_t*)(mem + p.halo);
   a.hcell = (const int32_t*)(mem + p.hcell);
-  a.xbuf = (unsigned long long*)(mem + p.bytes);
+  a.xbuf = (unsigned long long*)h->res_exchange;
   a.ctrl = (uint32_t*)(mem + p.ctrl);
   a.seq = h->res_seq + 1;
   a.chained = chained;
@@ -1696,7 +1704,7 @@ int run_resident(rsg_instance* h, int kb, const rsg::VelocityArgs<T>& va, const 
   a.max_set = p.max_set;
   a.max_node = p.max_node;
   a.max_cell = p.max_cell;
-  a.work = h->res_records ? nullptr : (uint32_t*)(mem + p.bytes + resident_exchange_bytes(h));
+  a.work = h->res_records ? nullptr : (uint32_t*)((char*)h->res_exchange + resident_exchange_bytes(h));
   a.force = force;
   a.nforce = (int32_t)h->res_force.size();
   a.ncls = h->res_cls.p;
@@ -1798,24 +1806,20 @@ int settle_resident(rsg_instance* h, bool all = true, int buffer = -1, bool* aga
   if (again) *again = false;
   std::deque<rsg_instance::Launch>& q = h->res_pending;
   if (q.empty()) return RSG_OK;
-  const uint64_t* const word = reinterpret_cast<const uint64_t*>(h->res_status + rsg::kResidentDecision);
+  const int32_t* const word = h->res_status + rsg::kResidentDecision;
   bool ended = false;  // all launches have, so they have decided
   for (uint32_t spin = 1; !q.empty(); spin++) {
-    const uint64_t w = __atomic_load_n(word, __ATOMIC_ACQUIRE);
-    const uint32_t d = (uint32_t)w, first_refused = (uint32_t)(w >> 32);
+    const uint32_t d = (uint32_t)__atomic_load_n(word, __ATOMIC_ACQUIRE);
     const uint32_t head = h->res_seq + 1 - (uint32_t)q.size();  // the oldest's number
-    const int64_t size = (int64_t)q.size();
-    const int64_t last = (int32_t)(((d >> 1) - head) << 1) >> 1;  // the last one decided, counted from there
-    const int64_t known = ended ? size : std::max<int64_t>(0, std::min(size, last + 1));
+    // the launch of the last decision, counted from there (numbers of 31 bits)
+    const int64_t last = (int32_t)(((d >> 1) - head) << 1) >> 1;
     const bool refused = last >= 0 && !(d & 1);
-    if (!refused) {
-      q.erase(q.begin(), q.begin() + known);
-    } else if (known < size) {
-      all = true;  // the others refuse as soon as they begin
-    } else {
+    const int64_t made = refused ? last : ended ? (int64_t)q.size() : last + 1;
+    q.erase(q.begin(), q.begin() + std::max<int64_t>(0, std::min<int64_t>(q.size(), made)));
+    if (refused) all = true;  // those behind it end as soon as they begin
+    if (refused && ended) {
       // the GPU is shared with work that keeps the tiles apart: not again soon
       h->res_not_before = std::chrono::steady_clock::now() + kResidentRetry;
-      q.erase(q.begin(), q.begin() + std::max<int64_t>(0, std::min<int64_t>(size, (int32_t)(first_refused - head))));
       if (again) *again = true;
       auto steps = [&](auto zero, const rsg_instance::Launch& l) {
         using T = decltype(zero);
@@ -2636,6 +2640,7 @@ int rsg_create_ex(const rsg_mesh_desc* mesh, const rsg_model_desc* model, int32_
     const char* alone = std::getenv("PANNDE_RSG_RESIDENT");
     const uint32_t started = alone && !strcmp(alone, "alone") ? 1u << 31 : 0;
     memcpy(p.block.get() + p.ctrl, &started, sizeof(started));
+    (void)upload_plan(h.get());  // or with the first resident launch
     return RSG_OK;
   };
   {

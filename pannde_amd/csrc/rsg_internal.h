@@ -224,10 +224,10 @@ constexpr uint32_t kResidentOwner = 0x80000000u;  // node record: this tile writ
 constexpr int kResidentForces = 256;  // largest row
 constexpr uint8_t kResidentSensor = 0x80;  // node mark: a sensor this tile records
 
-// Status words: the last launch's decision (several tiles), 2 seq + 1 when its steps are made and
-// 2 seq when nothing is written, with the number of the first launch of those refused last (one
-// 8-byte word); 1 when a wait between tiles ran out (the state is lost).
-constexpr int kResidentDecision = 0, kResidentRefused = 1, kResidentLost = 2, kResidentStatus = 3;
+// Status words: the last decision that a launch of several tiles came to, 2 seq + 1 when its steps are
+// made and 2 seq when its tiles did not get onto the GPU together and nothing is written; 1 when a wait
+// between tiles ran out (the state is lost).
+constexpr int kResidentDecision = 0, kResidentLost = 1, kResidentStatus = 2;
 
 template <typename T>
 struct ResidentArgs {
@@ -240,11 +240,9 @@ struct ResidentArgs {
   const int32_t* halo;   // exchange slot of each halo cell
   const int32_t* hcell;  // internal id of each halo cell
   unsigned long long* xbuf;  // [4][6 * sizeof(T) / 8][nexp]: exported stresses of four steps in turn
-  uint32_t* ctrl;        // [3] (several tiles): tiles started, over all launches; the last decision; the
-                         // first launch of those refused last
+  uint32_t* ctrl;        // [2] (several tiles): tiles started, over all launches; the last decision
   uint32_t seq;          // number of the launch, from 1
-  int32_t chained;       // 1: refuse the launch if the one before it was
-  int32_t* status;       // [kResidentStatus], pinned, 8-byte aligned
+  int32_t* status;       // [kResidentStatus], pinned
   int32_t nsteps;        // >= 2
   int32_t ntiles;
   int32_t nexp;
@@ -260,6 +258,8 @@ struct ResidentArgs {
   int32_t row;           // doubles from one step's trace row to the next's
   int32_t nmat;          // values of dt/rho in v.cls
   int32_t tables;        // 1: the class tables' spacings and dt/rho are held in LDS
+  int32_t chained;       // 1: the host does not know the decision on the launch before; if that was
+                         // refused, so is this one (for the launcher)
 };
 
 // The class tables in LDS, for meshes of at most kResidentClasses spacings along each axis and

@@ -41,14 +41,15 @@
 // of them than compute units, and the host lets one resident launch run at a time, but another
 // process or stream may hold part of the GPU.  So a launch first agrees: the last workgroup to
 // start decides that the steps are made; one that has waited long decides that they are not, and
-// all leave with nothing written.  What was queued behind such a launch must not run on its state:
-// a launch whose predecessor was refused (and the host did not know it) refuses itself at once.  The
-// host reads the decisions when it waits for the handle anyway, and makes the steps of refused
-// launches with the per-step kernels.  (A cooperative launch would see to it too, but costs 20 us and
-// the host's wait for it, and on ROCm 7 its queue slows the streams created after it: a batch's two
-// lanes took 5.4 ms for 2.0 ms of work.  Waiting for each decision before queuing more costs nothing
-// on an idle GPU, but beside a busy batch each piece of work then waits for a turn of its own: 100
-// steps of 259,000 cells and their energy 82..136 ms against 55.)
+// all leave with nothing written.  What was queued behind such a launch must not run on its state: a
+// launch that the host queues behind one whose decision it does not know yet gets a kernel of one
+// thread in front, which passes a refusal on.  The host reads the decisions when it waits for the
+// handle anyway, and makes the steps of refused launches with the per-step kernels.
+// (A cooperative launch would see to the start too, but costs 20 us and the host's wait for it, and on
+// ROCm 7 its queue slows the streams created after it: a batch's two lanes took 5.4 ms for 2.0 ms of
+// work.  Waiting for each decision before queuing more costs nothing on an idle GPU, but beside a busy
+// batch each piece of work then waits for a turn of its own: 100 steps of 259,000 cells and their
+// energy 82..136 ms against 55.)
 #include <type_traits>
 
 #include "rsg_device.h"
@@ -66,28 +67,18 @@ __device__ __forceinline__ bool decided(uint32_t d, uint32_t seq) { return (d >>
 
 // Whether the launch's steps are made, once decided.  Called by one thread of each workgroup, which
 // was the last to start or not; the one that decides tells the host.
-template <typename T>
-__device__ __forceinline__ bool agree(const ResidentArgs<T>& a, bool last) {
-  uint32_t* const decision = a.ctrl + 1;
+__device__ __forceinline__ bool agree(uint32_t* decision, int32_t* status, uint32_t seq, bool last) {
   uint64_t t0 = 0;
   for (;;) {
     uint32_t d = __hip_atomic_load(decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (decided(d, a.seq)) return d & 1;
-    const bool barred = a.chained && d == 2 * (a.seq - 1);
+    if (decided(d, seq)) return d & 1;
     const uint64_t t = wall_clock64();
     if (t0 == 0) t0 = t;
-    const uint32_t mine = 2 * a.seq + (last && !barred ? 1u : 0u);
-    if ((last || barred || t - t0 > kStartTicks) &&  // the first decision stands
+    const uint32_t mine = 2 * seq + (last ? 1u : 0u);
+    if ((last || t - t0 > kStartTicks) &&  // the first decision stands
         __hip_atomic_compare_exchange_strong(decision, &d, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT)) {
-      uint32_t first = a.seq;
-      if (barred)
-        first = __hip_atomic_load(a.ctrl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      else if (!last)
-        __hip_atomic_store(a.ctrl + 2, first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(reinterpret_cast<unsigned long long*>(a.status + kResidentDecision),
-                         (unsigned long long)first << 32 | mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+                                             __HIP_MEMORY_SCOPE_AGENT))
+      __hip_atomic_store(status + kResidentDecision, (int32_t)mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -458,7 +449,7 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
   };
 
   if (a.ntiles > 1) {
-    if (t == 0) go = agree(a, last);
+    if (t == 0) go = agree(a.ctrl + 1, a.status, a.seq, last);
     __syncthreads();
     if (!go) return;
   }
@@ -555,6 +546,13 @@ __global__ __launch_bounds__(THREADS) void resident_kernel(ResidentArgs<T> a) {
   }
 }
 
+// In front of launch seq: it is decided against if the launch before it was (the host learns of that
+// one alone).
+__global__ void pass_refusal(uint32_t* decision, uint32_t seq) {
+  if (__hip_atomic_load(decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * (seq - 1))
+    __hip_atomic_store(decision, 2 * seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <typename T, int THREADS, bool NKEY, bool CKEY>
 const void* resident_fn(bool rec) {
   return rec ? reinterpret_cast<const void*>(&resident_kernel<T, THREADS, NKEY, CKEY, true>)
@@ -578,6 +576,13 @@ hipError_t launch_resident(const ResidentArgs<T>& a, int threads, hipStream_t st
   const size_t lds = resident_lds_bytes(a.max_set, a.max_node, a.max_cell, sizeof(T), rec) +
                      (a.tables ? resident_table_bytes(sizeof(T)) : 0);
   void* args[1] = {const_cast<void*>(static_cast<const void*>(&a))};
+  if (a.chained) {
+    uint32_t* decision = a.ctrl + 1;
+    uint32_t seq = a.seq;
+    void* pass[2] = {&decision, &seq};
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(&pass_refusal), dim3(1), dim3(1), pass, 0, st);
+    if (e != hipSuccess) return e;
+  }
   return hipLaunchKernel(fn, dim3(a.ntiles), dim3(threads), args, lds, st);
 }
 

@@ -28,8 +28,8 @@ struct ResidentMesh {
   double lo[3], h[3];  // corner and finest spacing of the mesh
 };
 
-// The plan's arrays as one block of bytes, each 16-byte aligned, so that they go to the device with
-// one allocation and one copy.
+// The plan's arrays as one block of bytes, each on a 256-byte boundary, so that they go to the device
+// with one allocation and one copy.
 struct ResidentPlan {
   int32_t ntiles = 0, nexp = 0, max_set = 0, max_node = 0, max_cell = 0;
   size_t tiles = 0, halo = 0, hcell = 0, nrec = 0, crec = 0, ctrl = 0, bytes = 0;  // offsets, total
@@ -286,7 +286,7 @@ bool build_resident_plan(const ResidentMesh& m, int32_t max_tiles, size_t lds_li
   p.ntiles = nt;
   auto place = [&](size_t bytes) {
     const size_t at = p.bytes;
-    p.bytes += (bytes + 15) / 16 * 16;
+    p.bytes += (bytes + 255) / 256 * 256;
     return at;
   };
   p.tiles = place(sizeof(ResidentTile) * nt);

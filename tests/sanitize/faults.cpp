@@ -37,7 +37,7 @@ int fault_launch = 0, fault_record = 0;
 int fault_lost = 0;
 double fault_amp[4096], fault_stress_amp[4096];
 const double* fault_trace[4096];
-// device allocations so far, and whether there is no memory for more
+// device allocations so far, and the bytes from which on there is no memory for one (0: there is)
 int fault_allocs = 0, fault_no_memory = 0;
 }  // extern "C"
 
@@ -54,12 +54,12 @@ int device_of(const void* p) {
   return devices.count(p) ? devices[p] : 0;
 }
 
-// the status word of the last decision, and what it will hold: late, or at once
-uint64_t* late_word = nullptr;
-uint64_t late_value = 0;
-void decide(int32_t* status, uint32_t decision, uint32_t first_refused) {
-  late_word = reinterpret_cast<uint64_t*>(status + rsg::kResidentDecision);
-  late_value = (uint64_t)first_refused << 32 | decision;
+// the status word, and what it will hold: late, or at once
+int32_t* late_word = nullptr;
+int32_t late_value = 0;
+void decide(int32_t* status, uint32_t decision) {
+  late_word = status + rsg::kResidentDecision;
+  late_value = (int32_t)decision;
   if (fault_late == 0) *late_word = late_value;
 }
 
@@ -70,18 +70,14 @@ hipError_t resident(const A& a, F&& real) {
   if (fault_lost > 0 && fault_lost--) a.status[rsg::kResidentLost] = 1;
   if (a.ntiles == 1) return real();
   uint32_t* const decision = a.ctrl + 1;  // as the kernel keeps it
-  const bool barred = a.chained && *decision == 2 * (a.seq - 1);
-  if (!barred && fault_refuse == 0) {
-    *decision = 2 * a.seq + 1;
-    decide(a.status, *decision, 0);
-    return real();
+  if (a.chained && *decision == 2 * (a.seq - 1)) {
+    *decision = 2 * a.seq;
+    return hipSuccess;
   }
-  *decision = 2 * a.seq;
-  if (!barred) {
-    fault_refuse--;
-    a.ctrl[2] = a.seq;
-  }
-  decide(a.status, *decision, a.ctrl[2]);
+  *decision = 2 * a.seq + !fault_refuse;
+  decide(a.status, *decision);
+  if (fault_refuse == 0) return real();
+  fault_refuse--;
   return hipSuccess;
 }
 template <typename A>
@@ -135,7 +131,7 @@ hipError_t __wrap_hipStreamSynchronize(hipStream_t s) {
 hipError_t __real_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s);
 hipError_t __wrap_hipMallocFromPoolAsync(void** p, size_t bytes, hipMemPool_t pool, hipStream_t s) {
   if (device_of(s) != current) return hipErrorInvalidValue;
-  if (fault_no_memory) return hipErrorOutOfMemory;
+  if (fault_no_memory && bytes >= (size_t)fault_no_memory) return hipErrorOutOfMemory;
   __atomic_fetch_add(&fault_allocs, 1, __ATOMIC_RELAXED);
   return __real_hipMallocFromPoolAsync(p, bytes, pool, s);
 }

@@ -254,10 +254,11 @@ s.close()
 ''')
 
 
-def test_resident_memory_comes_with_the_first_resident_launch(lib):
-    """A handle that is set up and never stepped resident holds what one without a plan holds; when
-    there is no memory for the plan, the per-step kernels make the steps."""
+def test_memory_of_resident_stepping(lib):
+    """Set-up allocates the plan alone; the exchange buffers and the classes come with the first resident
+    launch.  Where there is no memory for any of them, the per-step kernels make the steps."""
     run(lib, r'''
+import time
 case = cases.water_column_block(seed=9, nx=23, ny=14, nz=17, nsteps=12)
 allocs, held = knob("fault_allocs"), []
 for tuning in (None, dict(block_velocity=256)):  # (a named workgroup size: no plan)
@@ -268,25 +269,33 @@ for tuning in (None, dict(block_velocity=256)):  # (a named workgroup size: no p
     held.append((allocs.value - n, s.device_bytes()))
     s.close()
 assert knob("fault_velocity").value == 6 and knob("fault_resident").value == 0
-# the amplitude buffers have room for the classes' sums: 2 x 256 doubles for each
-assert held[0][0] == held[1][0] and 0 <= held[0][1] - held[1][1] <= 2 * 256 * 8 * 256, held
+# the plan: 16 bytes a cell and a tile's node, 8 a halo cell; and room for the classes' sums beside the
+# amplitudes, 2 x 256 doubles each
+assert held[0][0] == held[1][0] + 1 and 0 <= held[0][1] - held[1][1] <= 200 * case.n_cells + 2 * 256 * 8 * 256, held
 s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
 n, b = allocs.value, s.device_bytes()
 s.solve(case.nsteps)
 assert knob("fault_resident").value == 1 and allocs.value - n == 2 and s.device_bytes() > b
 assert same(s.get_state() + (s.traces(),), case)
 s.close()
-for late in (0, 1):  # none for the plan; none for the classes of a new table build
+case.sensors = case.sensors[:0]  # (no trace buffer: nothing else is as large as the plan)
+for what in ("plan", "exchange", "classes"):
+    knob("fault_no_memory").value = 50 * case.n_cells if what == "plan" else 0
     s = rsg.DeviceSolver.from_case(case, rsg.RSG_FP64)
-    if late:
+    if what == "classes":
         s.solve(7)
         s.set_sources([], case.moment[:1])
     v, r = knob("fault_velocity").value, knob("fault_resident").value
-    knob("fault_no_memory").value = 1
+    knob("fault_no_memory").value = knob("fault_no_memory").value or 1
     s.solve(9)
     s.synchronize()
     knob("fault_no_memory").value = 0
     assert knob("fault_velocity").value - v == 9 and knob("fault_resident").value == r
+    if what == "plan":
+        time.sleep(1.1)
+        s.solve(9)
+        s.synchronize()
+        assert knob("fault_resident").value == r + 1
     s.close()
 ''')
 
