@@ -3,6 +3,7 @@
 // pass through here; a test sets the counters through ctypes.
 #include <hip/hip_runtime_api.h>
 
+#include <chrono>
 #include <mutex>
 #include <system_error>
 #include <thread>
@@ -26,10 +27,10 @@ void NAME(__wrap_, START_THREAD)(std::thread* self, void* state, void (*depend)(
   NAME(__real_, START_THREAD)(self, state, depend);
 }
 
-// Resident launches that decide against their steps, when the decisions from now on become known (the
-// host has asked the event that often, or waited for the stream), launches so far, and what the per-step kernels were launched with: the first
+// Resident launches that decide against their steps, how many ms after its launch a decision becomes
+// known (or when the host waits for the stream), whether one is not known yet, launches so far, and what the per-step kernels were launched with: the first
 // channel's amplitude and the trace row's address.
-int fault_refuse = 0, fault_late = 0;
+int fault_refuse = 0, fault_late = 0, fault_undecided = 0;
 int fault_resident = 0, fault_velocity = 0, fault_stress = 0;
 // resident launches that fail, and which of the event records from now on does (1: the next)
 int fault_launch = 0, fault_record = 0;
@@ -54,13 +55,20 @@ int device_of(const void* p) {
   return devices.count(p) ? devices[p] : 0;
 }
 
-// the status word, and what it will hold: late, or at once
+// the status word, what it will hold, and when
 int32_t* late_word = nullptr;
 int32_t late_value = 0;
+std::chrono::steady_clock::time_point late_at;
 void decide(int32_t* status, uint32_t decision) {
   late_word = status + rsg::kResidentDecision;
   late_value = (int32_t)decision;
-  if (fault_late == 0) *late_word = late_value;
+  late_at = std::chrono::steady_clock::now() + std::chrono::milliseconds(fault_late);
+  fault_undecided = fault_late > 0;
+  if (!fault_undecided) *late_word = late_value;
+}
+void decided() {
+  *late_word = late_value;
+  fault_undecided = 0;
 }
 
 template <typename A, typename F>
@@ -95,9 +103,9 @@ extern "C" {
 
 hipError_t __real_hipEventQuery(hipEvent_t e);
 hipError_t __wrap_hipEventQuery(hipEvent_t e) {
-  if (fault_late > 0) {
-    if (--fault_late == 0) *late_word = late_value;
-    return hipErrorNotReady;
+  if (fault_undecided) {
+    if (std::chrono::steady_clock::now() < late_at) return hipErrorNotReady;
+    decided();
   }
   return __real_hipEventQuery(e);
 }
@@ -121,10 +129,7 @@ int fault_waits = 0;
 hipError_t __real_hipStreamSynchronize(hipStream_t s);
 hipError_t __wrap_hipStreamSynchronize(hipStream_t s) {
   __atomic_fetch_add(&fault_waits, 1, __ATOMIC_RELAXED);
-  if (fault_late > 0) {
-    fault_late = 0;
-    *late_word = late_value;
-  }
+  if (fault_undecided) decided();
   return __real_hipStreamSynchronize(s);
 }
 
