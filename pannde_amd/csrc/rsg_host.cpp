@@ -1525,9 +1525,12 @@ int finish_steps(rsg_instance* h);
 int flush_traces(rsg_instance* h) {
   const size_t row = h->sensors.size() * 3;
   if (h->trace_dev_steps == 0 || row == 0) return RSG_OK;
-  if (int rc = finish_steps(h)) return rc;
   const size_t old = h->trace_host.size();
-  h->trace_host.resize(old + (size_t)h->trace_dev_steps * row);
+  h->trace_host.resize(old + (size_t)h->trace_dev_steps * row);  // while the steps run
+  if (int rc = finish_steps(h)) {
+    h->trace_host.resize(old);
+    return rc;
+  }
   if (h->batch_stream) HIP_TRY(hipStreamSynchronize(h->batch_stream));
   HIP_TRY(copy_on(h->trace_host.data() + old, h->trace.p, (size_t)h->trace_dev_steps * row * sizeof(double),
                   hipMemcpyDeviceToHost, h->stream));
