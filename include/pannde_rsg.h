@@ -186,8 +186,8 @@ int rsg_set_state(rsg_handle h, const double* V, const double* S);
 int rsg_get_traces(rsg_handle h, int64_t first_step, int64_t nsteps, double* out);
 
 /* Blocks until every step queued on the handle's stream has finished (rsg_step only
- * enqueues work).  The reference's solve() is synchronous; this is its completion
- * point. */
+ * enqueues work; before a one-launch call it waits up to 200 us for the GPU to begin the
+ * one before).  The reference's solve() is synchronous; this is its completion point. */
 int rsg_synchronize(rsg_handle h);
 
 /* Current simulation time (the value solve() last returned) and steps taken. */
