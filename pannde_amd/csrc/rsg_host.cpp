@@ -264,7 +264,7 @@ std::vector<PinnedChunk> take_chunks(int device, int want, bool ahead) {
   if (ahead && (int)d.idle.size() + kPinnedChunks - d.made < want + kPinnedChunks / 2) return got;
   // the ones idle longest first, and new ones until a transfer leaves as many behind: chunks that the
   // last transfer's threads still hold in their caches are slower for the GPU (a million cells written
-  // and read, three handles in turn: 4.12 ms with two sets of 8 chunks, 4.30 with one)
+  // and read, three handles in turn: 4.15 ms with two sets of 8 chunks, 4.33 with one)
   int fresh = (int)d.idle.size() < 2 * want ? std::min(want, kPinnedChunks - d.made) : 0;
   while ((int)got.size() < want) {
     if (!d.idle.empty() && fresh == 0) {
